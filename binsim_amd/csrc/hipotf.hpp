@@ -274,6 +274,17 @@ struct PairList {            // pattern within one spin: strings u with ann subs
     DevBuf uw;               // int32[2*len]: (index of u, index of w = u^cre^ann)
     bool identity = false;   // (x, x) for every string
     int spin = 0;            // 0 alpha, 1 beta
+    std::vector<int32_t> h;  // host copy of uw
+};
+
+// blocks, bins and pair lists of the rotation runs of one (spin, pair or row, rank)
+// (rot_levels.hpp); built on first use, a few MB
+struct LevelPlan {
+    bool ok = false;
+    int nbins = 0, maxslot = 0, maxlen = 0;
+    DevBuf slots, soff, list;
+    std::vector<int> pat;    // pattern id -> row of ol, -1 if of another rank or spin
+    std::vector<int2> ol;    // [row][bin]: first word in list, words
 };
 
 struct Generator {
@@ -282,6 +293,7 @@ struct Generator {
     int cre[8];              // 1 = creation
     int kind = 0;            // 0 identity, 1 alpha only, 2 beta only, 3 mixed
     int pa = -1, pb = -1;    // pattern ids (into DevPool::lists)
+    bool kap = false;        // constant sign in the alpha-major gauge (rot_levels.hpp)
 };
 
 struct DevPool {
@@ -295,6 +307,9 @@ struct DevPool {
     DevBuf tz;                     // fused adjoint sweep on interleaved rows: (l, r) per element
     DevBuf vqe_res;                // fused VQE objective: per-parameter results + norms (grown, kept)
     DevBuf zeros;                  // batch tran: a zero angle per generator
+    u64 cm[2] = {0, 0}, am[2] = {0, 0};      // per spin: all orbitals created / annihilated in
+    std::unique_ptr<LevelPlan> lv[2][2][5];  // [spin][pair][rank]
+    DevBuf lvdesc, lvpart, lvsums;           // level runs: descriptors, gradient partials, their sums
 };
 
 // forward expm sweep and/or adjoint backgrad sweep over positions idxs[0..n) with fused

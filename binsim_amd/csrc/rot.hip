@@ -21,6 +21,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <map>
 
 namespace hipotf {
 
@@ -32,7 +33,15 @@ struct GenDev {
     int cre[8];
 };
 
-__device__ __forceinline__ int jw_sign(const GenDev &g, u64 a, u64 b) {
+__host__ __device__ __forceinline__ int pop64(u64 v) {
+#ifdef __HIP_DEVICE_COMPILE__
+    return (int)__popcll(v);
+#else
+    return __builtin_popcountll(v);
+#endif
+}
+
+__host__ __device__ __forceinline__ int jw_sign(const GenDev &g, u64 a, u64 b) {
     int par = 0;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -41,10 +50,10 @@ __device__ __forceinline__ int jw_sign(const GenDev &g, u64 a, u64 b) {
         const int q = p >> 1;
         const u64 lowq = (1ull << q) - 1;
         if ((p & 1) == 0) {
-            par += __popcll(a & lowq) + __popcll(b & lowq);
+            par += pop64(a & lowq) + pop64(b & lowq);
             a ^= 1ull << q;
         } else {
-            par += __popcll(a & ((lowq << 1) | 1ull)) + __popcll(b & lowq);
+            par += pop64(a & ((lowq << 1) | 1ull)) + pop64(b & lowq);
             b ^= 1ull << q;
         }
     }
@@ -209,6 +218,8 @@ __global__ __launch_bounds__(256) void k_sum_partials(const double *__restrict__
     if (threadIdx.x == 0) *out = t * scale;
 }
 
+#include "rot_levels.hpp"
+
 // ---------------------------------------------------------------------------------------
 // pool construction
 // ---------------------------------------------------------------------------------------
@@ -232,8 +243,29 @@ static int pattern_id(DevPool &P, const SpinSpace &S, int spin, u64 cre, u64 ann
     }
     L.len = (i64)(uw.size() / 2);
     L.uw.upload(uw);
+    L.h = std::move(uw);
     P.lists.push_back(std::move(L));
     return (int)P.lists.size() - 1;
+}
+
+// the constant part of generator G's sign in the alpha-major gauge: its sign on one pair, less the
+// gauge of the two determinants and the two spins' own factors (0 if the generator has no pair)
+static bool gauge_const(const Generator &G, const DevPool &P, const HostBasis &hb) {
+    const PairList &LA = P.lists[G.pa], &LB = P.lists[G.pb];
+    if (LA.len == 0 || LB.len == 0) return false;
+    GenDev g;
+    g.nops = G.nops;
+    for (int i = 0; i < 8; ++i) g.pos[i] = i < G.nops ? G.pos[i] : 0;
+    auto M = [](u64 a) {
+        u64 m = 0;
+        for (; a; a &= a - 1) m ^= (a & (~a + 1)) - 1;
+        return m;
+    };
+    const u64 a0 = hb.A.strs[LA.h[0]], a1 = hb.A.strs[LA.h[1]], b0 = hb.B.strs[LB.h[0]], b1 = hb.B.strs[LB.h[1]];
+    int par = jw_sign(g, a0, b0) + pop64(b0 & M(a0)) + pop64(b1 & M(a1));
+    if (!LA.identity) par += lv_canon(a0, LA.cre, LA.ann);
+    if (!LB.identity) par += lv_canon(b0, LB.cre, LB.ann);
+    return par & 1;
 }
 
 // structural checks of a generator list (no basis needed): creators first, <= 8 ladder
@@ -282,6 +314,7 @@ DevPool *make_dev_pool(DevBasis *b, i64 nops, const int32_t *offsets, const int3
         for (i64 i = 0; i < S.N; ++i) uw[2 * i] = uw[2 * i + 1] = (int32_t)i;
         L.len = S.N;
         L.uw.upload(uw);
+        L.h = std::move(uw);
         P->lists.push_back(std::move(L));
     }
     for (i64 g = 0; g < nops; ++g) {
@@ -313,6 +346,8 @@ DevPool *make_dev_pool(DevBasis *b, i64 nops, const int32_t *offsets, const int3
         G.kind = ta && tb ? 3 : (ta ? 1 : 2);
         G.pa = pattern_id(*P, hb.A, 0, cre_a, ann_a);
         G.pb = pattern_id(*P, hb.B, 1, cre_b, ann_b);
+        G.kap = gauge_const(G, *P, hb);
+        P->cm[0] |= cre_a, P->am[0] |= ann_a, P->cm[1] |= cre_b, P->am[1] |= ann_b;
         P->gens.push_back(G);
     }
     P->partial.alloc(4096 * sizeof(double));
@@ -463,7 +498,9 @@ struct SegGen {
     double c, s;
 };
 
-enum { SEG_ROW_A = 0, SEG_ROW_B = 1, SEG_PAIR = 2, SEG_SINGLE = 3 };
+// the LV kinds are parts of such segments on excitation levels (rot_levels.hpp); LV0: one
+// alpha-only generator of a pair segment
+enum { SEG_ROW_A = 0, SEG_ROW_B = 1, SEG_PAIR = 2, SEG_SINGLE = 3, SEG_LV_ROW_A, SEG_LV_ROW_B, SEG_LV_PAIR, SEG_LV0 };
 
 // A thread's first pair of a generator, (u, w) and the element string of u, loaded while the
 // previous generator runs (list(): the pair, early in that generator; str(): the string, once the
@@ -841,6 +878,7 @@ struct Segment {
     int nst;    // rows per block staged in LDS whole (the rest updated in place in global memory)
     i64 sp;     // elements of the next row staged too
     int nrow;   // rows per block: 1 (ROW) or 2 (PAIR), times 1 forward / 2 adjoint
+    LevelPlan *lv = nullptr;  // LV kinds other than LV0
 };
 
 static size_t seg_lds_budget() {
@@ -904,8 +942,40 @@ static std::vector<Segment> plan_sweep(DevPool *P, const i64 *idxs, i64 n, int n
                 ++s.count;
         }
         if (s.kind != SEG_SINGLE && s.count > 4096) s.count = 4096;
-        segs.push_back(s);
         i += s.count;
+        if (mode != 0 || s.kind == SEG_SINGLE) {
+            segs.push_back(s);
+            continue;
+        }
+        // runs of one rank of the moved spin that fit the LDS level by level; what does not stays
+        // on the segment's own form
+        const bool pair = s.kind == SEG_PAIR;
+        const int spin = s.kind == SEG_ROW_B ? 0 : 1;
+        auto rank = [&](i64 j) {
+            return __builtin_popcountll(P->lists[spin == 0 ? gen(j).pa : gen(j).pb].cre);
+        };
+        auto plan_of = [&](int k) -> LevelPlan * {
+            LevelPlan *lp = k > 0 ? level_plan(P, spin, pair, k) : nullptr;
+            return lp && (nvec == 1 || lp->maxslot <= lv_cap(true)) ? lp : nullptr;
+        };
+        for (i64 j = s.first, end = s.first + s.count; j < end;) {
+            const int k = rank(j);
+            Segment t = s;
+            t.first = (int)j;
+            t.count = 1;
+            LevelPlan *lp = plan_of(k);
+            if (pair && k == 0) {
+                t.kind = SEG_LV0;
+            } else if (lp) {
+                t.kind = pair ? SEG_LV_PAIR : (spin == 0 ? SEG_LV_ROW_B : SEG_LV_ROW_A);
+                t.lv = lp;
+                while (j + t.count < end && rank(j + t.count) == k) ++t.count;
+            } else {
+                while (j + t.count < end && rank(j + t.count) > 0 && !plan_of(rank(j + t.count))) ++t.count;
+            }
+            segs.push_back(t);
+            j += t.count;
+        }
     }
     return segs;
 }
@@ -966,8 +1036,31 @@ static void sweeps(DevPool *P, i64 n, const i64 *idxs, const double *thetas, con
         HIPOTF_REQUIRE(idxs[i] >= 0 && idxs[i] < (i64)P->gens.size(), "generator index out of range");
     // descriptors of every sweep position (for ROW_B the list is the alpha pattern)
     std::vector<SegGen> host(n);
-    auto fill = [&](const std::vector<Segment> &segs) {
-        for (const Segment &s : segs)
+    std::vector<LvGen> lvh;
+    int lvbins = 0;
+    auto fill_descs = [&](const std::vector<Segment> &segs) {
+        lvbins = 0;
+        for (const Segment &s : segs) lvbins = std::max(lvbins, s.kind == SEG_LV0 ? 1 : (s.lv ? s.lv->nbins : 0));
+        lvh.assign((size_t)lvbins * n, LvGen{});
+        for (const Segment &s : segs) {
+            if (s.lv || s.kind == SEG_LV0)
+                for (int k = 0; k < s.count; ++k) {
+                    const i64 i = s.first + k;
+                    const Generator &G = P->gens[idxs[i]];
+                    const double c = thetas ? std::cos(thetas[i]) : 0.0, sn = thetas ? std::sin(thetas[i]) : 0.0;
+                    const int q = s.lv ? s.lv->pat[s.kind == SEG_LV_ROW_B ? G.pa : G.pb] : 0;
+                    for (int b = 0; b < (s.lv ? s.lv->nbins : 1); ++b) {
+                        LvGen &d = lvh[(size_t)b * n + i];
+                        d.c = c;
+                        d.s = sn;
+                        d.kap = G.kap ? 0x80000000u : 0u;
+                        if (s.lv) {
+                            d.off = s.lv->ol[(size_t)q * s.lv->nbins + b].x;
+                            d.len = s.lv->ol[(size_t)q * s.lv->nbins + b].y;
+                        }
+                    }
+                }
+            else
             for (int k = 0; k < s.count; ++k) {
                 const i64 i = s.first + k;
                 const Generator &G = P->gens[idxs[i]];
@@ -983,19 +1076,118 @@ static void sweeps(DevPool *P, i64 n, const i64 *idxs, const double *thetas, con
                 d.c = thetas ? std::cos(thetas[i]) : 0.0;
                 d.s = thetas ? std::sin(thetas[i]) : 0.0;
             }
+        }
     };
     bool transposed = false;  // grad: the beta-major copies are made once (the vectors do not change)
     auto run = [&](const std::vector<Segment> &segs, bool back, bool il) {
-        fill(segs);
+        fill_descs(segs);
+        bool old_desc = false;
+        for (const Segment &s : segs) old_desc |= s.kind <= SEG_PAIR;
         P->segdesc.ensure((size_t)std::max<i64>(n, 1) * sizeof(SegGen));
-        if (n) HIPOTF_CHECK(hipMemcpyAsync(P->segdesc.p, host.data(), n * sizeof(SegGen), hipMemcpyHostToDevice, st));
-        if (grad && n) {
-            hipLaunchKernelGGL(k_seg_cs, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
-                               P->segdesc.as<SegGen>(), thetas_dev, n);
-            HIPOTF_CHECK(hipGetLastError());
+        if (n && old_desc) {
+            HIPOTF_CHECK(hipMemcpyAsync(P->segdesc.p, host.data(), n * sizeof(SegGen), hipMemcpyHostToDevice, st));
+            if (grad) {
+                hipLaunchKernelGGL(k_seg_cs, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
+                                   P->segdesc.as<SegGen>(), thetas_dev, n);
+                HIPOTF_CHECK(hipGetLastError());
+            }
         }
         const SegGen *dg = P->segdesc.as<SegGen>();
-        const int nvec = back ? 2 : 1;
+        const i64 nlv = (i64)lvh.size();
+        if (nlv) {
+            P->lvdesc.ensure(nlv * sizeof(LvGen));
+            HIPOTF_CHECK(hipMemcpyAsync(P->lvdesc.p, lvh.data(), nlv * sizeof(LvGen), hipMemcpyHostToDevice, st));
+            if (grad) {
+                hipLaunchKernelGGL(k_lv_cs, dim3((unsigned)((nlv + 255) / 256)), dim3(256), 0, st,
+                                   P->lvdesc.as<LvGen>(), thetas_dev, n, nlv);
+                HIPOTF_CHECK(hipGetLastError());
+            }
+        }
+        // gradient sums of the level runs: their partials collect in one buffer (up to 256 MB unless
+        // one run needs more) and are added up together
+        const int nch = (int)((NB + LV0_EL - 1) / LV0_EL);
+        auto lv_rows = [&](const Segment &s) -> i64 {  // partial rows of a level run
+            if (s.kind == SEG_LV0) return P->lists[s.pa].len * nch;
+            const i64 nu = s.kind == SEG_LV_PAIR ? P->lists[s.pa].len : (s.kind == SEG_LV_ROW_A ? NA : NB);
+            return nu * s.lv->nbins;
+        };
+        i64 cap = 0, used = 0;
+        if (back) {
+            i64 tot = 0;
+            for (const Segment &s : segs)
+                if (s.kind > SEG_SINGLE) {
+                    const i64 need = lv_rows(s) * s.count;
+                    cap = std::max(cap, need);
+                    tot += need;
+                }
+            cap = std::max(cap, std::min<i64>(tot, 32ll << 20));
+            if (cap) P->lvpart.ensure(cap * sizeof(double));
+        }
+        LvPend pend{};
+        auto pend_flush = [&]() {
+            if (!pend.n) return;
+            const int tiles = pend.tile0[pend.n];
+            P->lvsums.ensure((size_t)tiles * LV_SLICES * 64 * sizeof(double));
+            hipLaunchKernelGGL(k_lv_sum1, dim3(tiles, LV_SLICES), dim3(256), 0, st, pend, P->lvpart.as<double>(),
+                               P->lvsums.as<double>());
+            hipLaunchKernelGGL(k_lv_sum2, dim3(tiles), dim3(64), 0, st, pend, P->lvsums.as<double>(), dres);
+            HIPOTF_CHECK(hipGetLastError());
+            pend.n = 0;
+            used = 0;
+        };
+        auto pend_add = [&](const Segment &s) -> double * {
+            const i64 rows = lv_rows(s), need = rows * s.count;
+            if (pend.n == LV_PEND || used + need > cap) pend_flush();
+            const int d = pend.n++;
+            pend.at[d] = used;
+            pend.nrow[d] = rows;
+            pend.ng[d] = s.count;
+            pend.first[d] = s.first;
+            if (d == 0) pend.tile0[0] = 0;
+            pend.tile0[d + 1] = pend.tile0[d] + (s.count + 63) / 64;
+            used += need;
+            return P->lvpart.as<double>() + pend.at[d];
+        };
+        // one level run on (l, r), rows nel elements long
+        auto level_run = [&](const Segment &s, double *l, double *r) {
+            LvArgs a{};
+            a.l = l;
+            a.r = r;
+            const bool pr = s.kind == SEG_LV_PAIR, rowB = s.kind == SEG_LV_ROW_B;
+            if (pr) {
+                const PairList &LA = P->lists[s.pa];
+                a.alist = LA.uw.as<int32_t>();
+                a.nunit = LA.len;
+                a.strsA = B->pA->strs.as<u64>();
+                a.acre = LA.cre;
+                a.aann = LA.ann;
+            } else {
+                a.nunit = rowB ? NB : NA;
+            }
+            a.nel = rowB ? NA : NB;
+            a.nbins = s.lv->nbins;
+            a.ng = s.count;
+            a.slots = s.lv->slots.as<uint2>();
+            a.soff = s.lv->soff.as<int>();
+            a.rword = rowB ? B->pB->strs.as<u64>() : B->gaugeM.as<u64>();
+            a.gens = P->lvdesc.as<LvGen>() + s.first;
+            a.gstride = n;
+            a.list = s.lv->list.as<u32>();
+            if (back) a.partial = pend_add(s);
+            const int bd = lv_threads(*s.lv);
+            const size_t smem = (size_t)s.lv->maxslot * (back ? 16 : 8) + (back ? (size_t)LV_RED * (bd / 64) * 8 : 0);
+            const i64 nblk = (a.nunit * a.nbins + 7) / 8 * 8;
+            HIPOTF_REQUIRE(nblk < (1ll << 31), "rotation sweep grid too large");
+            auto go = [&](auto kern) {
+                HIPOTF_CHECK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                 (int)smem));
+                hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(bd), smem, st, a);
+            };
+            if (grad) go(k_lv<2>);
+            else if (back) go(k_lv<1>);
+            else go(k_lv<0>);
+            HIPOTF_CHECK(hipGetLastError());
+        };
         // interleaved pair segments: z = (psi, lam) element by element, made before the first
         // pair segment of a run of them and split back before a row segment or the end
         double2 *z = nullptr;
@@ -1028,7 +1220,35 @@ static void sweeps(DevPool *P, i64 n, const i64 *idxs, const double *thetas, con
                 }
                 continue;
             }
-            if (s.kind == SEG_ROW_A || s.kind == SEG_ROW_B) {
+            if (s.kind == SEG_LV0 || s.kind == SEG_LV_PAIR) {
+                const PairList &LA = P->lists[s.pa];
+                if (LA.len == 0) {
+                    if (back) fill(dres + s.first, s.count, 0.0, st);
+                    continue;
+                }
+                if (s.kind == SEG_LV_PAIR) {
+                    level_run(s, psi, lam);
+                    continue;
+                }
+                HIPOTF_REQUIRE(LA.len * nch < (1ll << 31), "rotation sweep grid too large");
+                double *part = back ? pend_add(s) : nullptr;
+                auto go = [&](auto kern) {
+                    hipLaunchKernelGGL(kern, dim3((unsigned)(LA.len * nch)), dim3(256), 0, st, psi, lam,
+                                       LA.uw.as<int32_t>(), LA.len, NB, nch, B->gaugeM.as<u64>(),
+                                       B->pA->strs.as<u64>(), B->pB->strs.as<u64>(), LA.cre, LA.ann,
+                                       P->lvdesc.as<LvGen>() + s.first, part);
+                };
+                if (grad) go(k_lv0<2>);
+                else if (back) go(k_lv0<1>);
+                else go(k_lv0<0>);
+                HIPOTF_CHECK(hipGetLastError());
+                continue;
+            }
+            if (s.kind == SEG_LV_ROW_A) {
+                level_run(s, psi, lam);
+                continue;
+            }
+            if (s.kind == SEG_ROW_A || s.kind == SEG_ROW_B || s.kind == SEG_LV_ROW_B) {
                 const bool A = s.kind == SEG_ROW_A;
                 const i64 nrows = A ? NA : NB, nel = A ? NB : NA;
                 double *l = psi, *r = lam;
@@ -1044,6 +1264,19 @@ static void sweeps(DevPool *P, i64 n, const i64 *idxs, const double *thetas, con
                     }
                     l = P->tl.as<double>();
                     r = P->tr.as<double>();
+                }
+                auto untranspose = [&]() {
+                    if (A || grad) return;
+                    dim3 g((unsigned)((NA + 31) / 32), (unsigned)((NB + 31) / 32));
+                    hipLaunchKernelGGL(k_transpose<double>, g, dim3(256), 0, st, P->tl.as<double>(), psi, NB, NA);
+                    if (back)
+                        hipLaunchKernelGGL(k_transpose<double>, g, dim3(256), 0, st, P->tr.as<double>(), lam, NB, NA);
+                };
+                if (s.kind == SEG_LV_ROW_B) {
+                    level_run(s, l, r);
+                    untranspose();
+                    HIPOTF_CHECK(hipGetLastError());
+                    continue;
                 }
                 const size_t staged = (size_t)(nel * s.nst + s.sp) * sizeof(double);
                 const size_t smem = staged ? staged : glob_smem;
@@ -1076,12 +1309,7 @@ static void sweeps(DevPool *P, i64 n, const i64 *idxs, const double *thetas, con
                     else go_row(k_seg_row<false, 1>, (double *)nullptr, (double *)nullptr);
                 }
                 HIPOTF_CHECK(hipGetLastError());
-                if (!A && !grad) {
-                    dim3 g((unsigned)((NA + 31) / 32), (unsigned)((NB + 31) / 32));
-                    hipLaunchKernelGGL(k_transpose<double>, g, dim3(256), 0, st, P->tl.as<double>(), psi, NB, NA);
-                    if (back)
-                        hipLaunchKernelGGL(k_transpose<double>, g, dim3(256), 0, st, P->tr.as<double>(), lam, NB, NA);
-                }
+                untranspose();
                 if (back)
                     hipLaunchKernelGGL(k_seg_reduce, dim3(s.count), dim3(256), 0, st, part, nrows, dres + s.first);
                 HIPOTF_CHECK(hipGetLastError());
@@ -1147,6 +1375,7 @@ static void sweeps(DevPool *P, i64 n, const i64 *idxs, const double *thetas, con
             }
         }
         zip(false);
+        if (back) pend_flush();
     };
     if (grad) {
         run(plan_sweep(P, idxs, n, 2), true, false);

@@ -1,0 +1,467 @@
+// Rotation runs on excitation levels (included by rot.hip).
+//
+// In a pool whose generators only move electrons of a spin from the orbitals A to the disjoint
+// orbitals C (a particle-hole pool, such as UCC from a reference determinant), a generator that
+// excites k electrons of that spin takes a string with c = |s & C| to one with c + k and leaves
+// the orbitals outside A and C alone.  A run of consecutive generators of one rank k therefore
+// never couples elements of different blocks:
+//   pair run (one alpha pattern u -> w, beta rank k):  { row u, level c } + { row w, level c + k }
+//   row run (one spin moves, the other is the row):    { levels c, c + k, c + 2k, .. }
+// for fixed occupation outside A and C.  One workgroup owns a few whole blocks (a bin) of one
+// row (pair): their elements are loaded into LDS once, every generator of the run is applied
+// there, and they are stored once.  At 16 orbitals / 8 electrons the largest pair block has
+// 8,036 elements (129 KB of (l, r) values, 64 KB of l alone) where the row pair itself has
+// 25,740 and had to stay in global memory; the row runs of doubles split into halves of 6,470.
+//
+// Bounds.  LDS bandwidth: 32 bytes per coupled pair forward, 64 in the adjoint sweep, against
+// 128 bytes per cycle and CU; then the latency of a generator's phase (LDS read, a dependent
+// chain of four FP64 operations, LDS write, barrier).  The pair lists are compact (one word per
+// pair: two 14-bit slots and a sign, 0.9 MB for the 64 beta singles at 16 orbitals, L2 resident),
+// and the words and the angle of the next generator are loaded while the current one runs.
+//
+// Signs.  The elements are held in the alpha-major gauge x~ = (-1)^popc(b & M(a)) x, where a
+// generator's sign splits into one factor per spin: the moved strings' factor is a bit of the
+// list word, the alpha factor of a pair run is one bit per workgroup, and the rest is a constant
+// bit of the generator.
+#pragma once
+
+constexpr int LV_SLOT_BITS = 14;
+constexpr int LV_NP = 2;    // list words per thread and generator held ahead
+constexpr int LV_RED = 64;  // generators between two flushes of the gradient sums
+
+struct LvGen {              // one generator as one bin sees it
+    double c, s;
+    int32_t off, len;       // its words in the list
+    u32 kap, pad;           // its constant sign (bit 31)
+};
+static_assert(sizeof(LvGen) == 32, "two 16-byte loads");
+
+// sign of the ladder operators ann (ascending), then cre (ascending), on string s of one spin
+__host__ __device__ __forceinline__ int lv_canon(u64 s, u64 cre, u64 ann) {
+    int par = 0;
+    auto pop = [](u64 v) {
+#ifdef __HIP_DEVICE_COMPILE__
+        return (int)__popcll(v);
+#else
+        return __builtin_popcountll(v);
+#endif
+    };
+    for (u64 m = ann; m; m &= m - 1) {
+        const u64 b = m & (~m + 1);
+        par += pop(s & (b - 1));
+        s ^= b;
+    }
+    for (u64 m = cre; m; m &= m - 1) {
+        const u64 b = m & (~m + 1);
+        par += pop(s & (b - 1));
+        s ^= b;
+    }
+    return par & 1;
+}
+
+struct LvArgs {
+    double *l, *r;
+    const int32_t *alist;   // pair run: (u, w) rows; NULL: row run
+    i64 nunit, nel;         // row pairs or rows; elements per row
+    int nbins, ng;
+    const uint2 *slots;     // per slot: element | row (0: u, 1: w) << 31, gauge word of the element
+    const int *soff;        // first slot of each bin, nbins + 1
+    const u64 *rword;       // gauge word of each row
+    const u64 *strsA;       // pair run: strings of the rows, and their pattern
+    u64 acre, aann;
+    const LvGen *gens;      // [nbins][gstride]
+    i64 gstride;
+    const u32 *list;
+    double *partial;        // [nunit * nbins][ng]
+};
+
+// sum over the wave, valid in lane 63 (VALU moves; a shuffle would go through the LDS, which
+// these kernels are bound by)
+__device__ __forceinline__ double wave_sum63(double v) {
+    auto step = [&](auto ctrl, auto rows) {
+        constexpr int CT = decltype(ctrl)::value, RM = decltype(rows)::value;
+        const long long b = __double_as_longlong(v);
+        const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CT, RM, 0xf, false);
+        const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CT, RM, 0xf, false);
+        v += __longlong_as_double(((long long)hi << 32) | (u32)lo);
+    };
+    step(std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xf>{});  // row_shr 1
+    step(std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xf>{});
+    step(std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xf>{});
+    step(std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xf>{});
+    step(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});  // row_bcast 15
+    step(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});  // row_bcast 31
+    return v;
+}
+
+// MODE 0: forward rotations of l; 1: adjoint step on (l, r) with gradient sums, generators in
+// reverse; 2: gradient sums only (nothing is written, so the generators need no barrier)
+template <int MODE>
+__global__ __launch_bounds__(1024) void k_lv(LvArgs a) {
+    using E = typename std::conditional<MODE == 0, double, double2>::type;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    const i64 total = a.nunit * a.nbins, per = (total + 7) / 8;
+    const i64 wk = (i64)(blockIdx.x & 7) * per + (blockIdx.x >> 3);  // contiguous range per XCD
+    if ((i64)(blockIdx.x >> 3) >= per || wk >= total) return;
+    const i64 unit = wk / a.nbins;
+    const int bin = (int)(wk - unit * a.nbins);
+    const int tid = threadIdx.x, bd = blockDim.x, lane = tid & 63, wave = tid >> 6, nw = bd >> 6;
+    const int s0 = a.soff[bin], ns = a.soff[bin + 1] - s0;
+    E *x = reinterpret_cast<E *>(smem_raw);
+    double *red = reinterpret_cast<double *>(x + ns);  // [LV_RED][nw]
+    i64 ru = unit, rw = unit;
+    int neg = 0;
+    if (a.alist) {
+        ru = a.alist[2 * unit];
+        rw = a.alist[2 * unit + 1];
+        neg = lv_canon(a.strsA[ru], a.acre, a.aann);
+    }
+    const u32 wu = (u32)a.rword[ru], ww = (u32)a.rword[rw];
+    const i64 bu = ru * a.nel, bw = rw * a.nel;
+    auto at = [&](uint2 sl) { return ((sl.x >> 31) ? bw : bu) + (i64)(sl.x & 0x7fffffffu); };
+    auto flip = [&](uint2 sl) { return (u32)(__popc(sl.y & ((sl.x >> 31) ? ww : wu)) & 1) << 31; };
+    auto sgn = [](double v, u32 f) { return __longlong_as_double(__double_as_longlong(v) ^ ((long long)f << 32)); };
+    constexpr int LU = 4;  // elements in flight per thread
+    for (int i = tid; i < ns; i += LU * bd) {
+        uint2 sl[LU];
+        double lv[LU], rv[LU];
+#pragma unroll
+        for (int q = 0; q < LU; ++q) sl[q] = a.slots[s0 + min(i + q * bd, ns - 1)];
+#pragma unroll
+        for (int q = 0; q < LU; ++q) {
+            lv[q] = a.l[at(sl[q])];
+            if (MODE) rv[q] = a.r[at(sl[q])];
+        }
+#pragma unroll
+        for (int q = 0; q < LU; ++q)
+            if (i + q * bd < ns) {
+                const u32 f = flip(sl[q]);
+                if constexpr (MODE == 0) x[i + q * bd] = sgn(lv[q], f);
+                else x[i + q * bd] = make_double2(sgn(lv[q], f), sgn(rv[q], f));
+            }
+    }
+    // descriptors and list words by vector loads (their wait counter is not the LDS's)
+    u32 vz;
+    asm("v_mov_b32 %0, 0" : "=v"(vz));
+    const LvGen *G = a.gens + (i64)bin * a.gstride;
+    auto gen_at = [&](int kk) { return MODE == 1 ? a.ng - 1 - min(kk, a.ng - 1) : min(kk, a.ng - 1); };
+    struct D { double c, s; int off, len; u32 kap; };
+    auto ld = [&](int kk) {
+        const LvGen *g = G + (gen_at(kk) + vz);
+        const double2 cs = *reinterpret_cast<const double2 *>(g);
+        const int4 ol = *reinterpret_cast<const int4 *>(&g->off);
+        return D{cs.x, cs.y, ol.x, ol.y, (u32)ol.z};
+    };
+    auto words = [&](const D &d, u32 (&e)[LV_NP]) {  // clamped: unused words are never applied
+#pragma unroll
+        for (int q = 0; q < LV_NP; ++q) e[q] = a.list[d.off + max(0, min(tid + q * bd, d.len - 1))];
+    };
+    const u32 sflip = (u32)neg << 31;
+    D d0 = ld(0), d1 = ld(1);
+    u32 e0[LV_NP], e1[LV_NP];
+    words(d0, e0);
+    __syncthreads();
+    constexpr u32 SM = (1u << LV_SLOT_BITS) - 1;
+    auto flush = [&](int k1, int cnt) {  // gradient sums of the cnt generators before order position k1
+        __syncthreads();
+        if (tid < cnt) {
+            double t = 0.0;
+            for (int w = 0; w < nw; ++w) t += red[tid * nw + w];
+            a.partial[wk * a.ng + gen_at(k1 - cnt + tid)] = t;
+        }
+        __syncthreads();
+    };
+    for (int kk = 0; kk < a.ng; ++kk) {
+        const D d2 = ld(kk + 2);
+        words(d1, e1);
+        double acc = 0.0;
+        const double c = d0.c, s = d0.s;
+        const u32 gf = sflip ^ d0.kap;
+        auto body = [&](u32 e, E &xu, E &xw, bool act) {
+            const u32 sf = (e & 0x80000000u) ^ gf;
+            const double ts = sgn(s, sf);
+            if constexpr (MODE == 0) {
+                const double nu = c * xu - ts * xw, nw_ = ts * xu + c * xw;
+                if (act) {
+                    x[e & SM] = nu;
+                    x[(e >> LV_SLOT_BITS) & SM] = nw_;
+                }
+            } else if constexpr (MODE == 1) {
+                const double tc = sgn(c, sf);
+                const double nlu = c * xu.x + ts * xw.x, nlw = -ts * xu.x + c * xw.x;
+                const double g = nlu * (-s * xu.y + tc * xw.y) + nlw * (-s * xw.y - tc * xu.y);
+                if (act) {
+                    acc += g;
+                    x[e & SM] = make_double2(nlu, c * xu.y + ts * xw.y);
+                    x[(e >> LV_SLOT_BITS) & SM] = make_double2(nlw, -ts * xu.y + c * xw.y);
+                }
+            } else {
+                const double tc = sgn(c, sf);
+                const double g = xu.x * (-s * xu.y + tc * xw.y) + xw.x * (-s * xw.y - tc * xu.y);
+                if (act) acc += g;
+            }
+        };
+        E xu[LV_NP], xw[LV_NP];
+#pragma unroll
+        for (int q = 0; q < LV_NP; ++q) {
+            xu[q] = x[e0[q] & SM];
+            xw[q] = x[(e0[q] >> LV_SLOT_BITS) & SM];
+        }
+#pragma unroll
+        for (int q = 0; q < LV_NP; ++q) body(e0[q], xu[q], xw[q], tid + q * bd < d0.len);
+        for (int j = tid + LV_NP * bd; j < d0.len; j += bd) {
+            const u32 e = a.list[d0.off + j];
+            E yu = x[e & SM], yw = x[(e >> LV_SLOT_BITS) & SM];
+            body(e, yu, yw, true);
+        }
+        if constexpr (MODE != 0) {
+            const double t = wave_sum63(acc);
+            if (lane == 63) red[(kk % LV_RED) * nw + wave] = t;
+        }
+        if constexpr (MODE != 2) __syncthreads();
+        if constexpr (MODE != 0)
+            if (kk % LV_RED == LV_RED - 1) flush(kk + 1, LV_RED);
+        d0 = d1;
+        d1 = d2;
+#pragma unroll
+        for (int q = 0; q < LV_NP; ++q) e0[q] = e1[q];
+    }
+    if constexpr (MODE != 0)
+        if (a.ng % LV_RED) flush(a.ng, a.ng % LV_RED);
+    if constexpr (MODE != 2) {
+        for (int i = tid; i < ns; i += bd) {
+            const uint2 sl = a.slots[s0 + i];
+            const u32 f = flip(sl);
+            if constexpr (MODE == 0) {
+                a.l[at(sl)] = sgn(x[i], f);
+            } else {
+                a.l[at(sl)] = sgn(x[i].x, f);
+                a.r[at(sl)] = sgn(x[i].y, f);
+            }
+        }
+    }
+}
+
+// A generator that moves no beta electron of a pair run (an alpha single): rows u and w of each
+// pair rotated element by element, LV0_EL elements per workgroup.  HBM bound (32 bytes per
+// element forward, 64 in the adjoint sweep).
+constexpr int LV0_EL = 2048;
+template <int MODE>
+__global__ __launch_bounds__(256) void k_lv0(double *__restrict__ l, double *__restrict__ r,
+                                             const int32_t *__restrict__ alist, i64 npairs, i64 nel, int nch,
+                                             const u64 *__restrict__ rword, const u64 *__restrict__ strsA,
+                                             const u64 *__restrict__ strsB, u64 acre, u64 aann,
+                                             const LvGen *__restrict__ gen, double *__restrict__ partial) {
+    const i64 wk = blockIdx.x, p = wk / nch;
+    const i64 e0 = (wk - p * nch) * LV0_EL, e1 = min(nel, e0 + LV0_EL);
+    const i64 ua = alist[2 * p], wa = alist[2 * p + 1];
+    const u64 M = rword[ua] ^ rword[wa];
+    const int neg = lv_canon(strsA[ua], acre, aann) ^ (int)(gen->kap >> 31);
+    const double c = gen->c, s = gen->s;
+    double acc = 0.0;
+    constexpr int U = 4;
+    for (i64 e = e0 + threadIdx.x; e < e1; e += U * 256) {
+        u64 b[U];
+        double lu[U], lw[U], ru[U], rw[U];
+#pragma unroll
+        for (int q = 0; q < U; ++q) {
+            const i64 i = min(e + q * 256, e1 - 1);
+            b[q] = strsB[i];
+            lu[q] = l[ua * nel + i];
+            lw[q] = l[wa * nel + i];
+            if (MODE) ru[q] = r[ua * nel + i], rw[q] = r[wa * nel + i];
+        }
+#pragma unroll
+        for (int q = 0; q < U; ++q) {
+            const i64 i = e + q * 256;
+            if (i >= e1) continue;
+            const bool sg = ((__popcll(b[q] & M) & 1) ^ neg) != 0;
+            const double ts = sg ? -s : s, tc = sg ? -c : c;
+            if (MODE == 0) {
+                l[ua * nel + i] = c * lu[q] - ts * lw[q];
+                l[wa * nel + i] = ts * lu[q] + c * lw[q];
+            } else if (MODE == 1) {
+                const double nlu = c * lu[q] + ts * lw[q], nlw = -ts * lu[q] + c * lw[q];
+                acc += nlu * (-s * ru[q] + tc * rw[q]) + nlw * (-s * rw[q] - tc * ru[q]);
+                l[ua * nel + i] = nlu;
+                l[wa * nel + i] = nlw;
+                r[ua * nel + i] = c * ru[q] + ts * rw[q];
+                r[wa * nel + i] = -ts * ru[q] + c * rw[q];
+            } else {
+                acc += lu[q] * (-s * ru[q] + tc * rw[q]) + lw[q] * (-s * rw[q] - tc * ru[q]);
+            }
+        }
+    }
+    if (MODE) {
+        const double t = block_sum(acc);
+        if (threadIdx.x == 0) partial[wk] = t;
+    }
+}
+
+// Column sums of pending [nrow][ng] partial blocks: out[k] = sum over rows, in fixed order.
+// Stage 1: LV_SLICES row slices per 64 columns; stage 2 adds the slices.
+constexpr int LV_PEND = 48, LV_SLICES = 16;
+struct LvPend {
+    i64 at[LV_PEND];        // first value in the partial buffer
+    i64 nrow[LV_PEND];
+    int ng[LV_PEND];
+    int first[LV_PEND];     // result position
+    int tile0[LV_PEND + 1]; // first 64-column tile
+    int n;
+};
+__device__ __forceinline__ int lv_pend_of(const LvPend &p, int tile) {
+    int d = 0;
+    while (d + 1 < p.n && p.tile0[d + 1] <= tile) ++d;
+    return d;
+}
+__global__ __launch_bounds__(256) void k_lv_sum1(LvPend p, const double *__restrict__ partial,
+                                                 double *__restrict__ sums) {
+    __shared__ double sm[256];
+    const int tile = blockIdx.x, sl = blockIdx.y, d = lv_pend_of(p, tile);
+    const int ng = p.ng[d], k0 = (tile - p.tile0[d]) * 64, nc = min(64, ng - k0);
+    int w = 1;  // columns handled side by side: nc rounded up to a power of two
+    while (w < nc) w *= 2;
+    const int col = threadIdx.x & (w - 1), rl = threadIdx.x / w, nr = 256 / w;
+    const i64 r0 = p.nrow[d] * sl / LV_SLICES, r1 = p.nrow[d] * (sl + 1) / LV_SLICES;
+    double t = 0.0;
+    if (col < nc)
+        for (i64 i = r0 + rl; i < r1; i += nr) t += partial[p.at[d] + i * ng + k0 + col];
+    sm[threadIdx.x] = t;
+    __syncthreads();
+    if (rl == 0 && col < nc) {
+        for (int q = 1; q < nr; ++q) t += sm[q * w + col];
+        sums[((i64)tile * LV_SLICES + sl) * 64 + col] = t;
+    }
+}
+__global__ __launch_bounds__(64) void k_lv_sum2(LvPend p, const double *__restrict__ sums,
+                                                double *__restrict__ dres) {
+    const int tile = blockIdx.x, d = lv_pend_of(p, tile), k = (tile - p.tile0[d]) * 64 + (int)threadIdx.x;
+    if (k >= p.ng[d]) return;
+    double t = 0.0;
+    for (int s = 0; s < LV_SLICES; ++s) t += sums[((i64)tile * LV_SLICES + s) * 64 + threadIdx.x];
+    dres[p.first[d] + k] = t;
+}
+
+// c, s of the level descriptors from the device angles (gradient-only pass): entry i of bin b is
+// position i
+__global__ __launch_bounds__(256) void k_lv_cs(LvGen *__restrict__ g, const double *__restrict__ th, i64 n,
+                                               i64 nent) {
+    const i64 i = (i64)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= nent) return;
+    const double t = th[i % n];
+    g[i].c = cos(t);
+    g[i].s = sin(t);
+}
+
+// ---- plans --------------------------------------------------------------------------------
+static size_t seg_lds_budget();
+// largest bin: (l, r) values with the gradient sums of 16 waves beside them, or l alone
+static i64 lv_cap(bool back) {
+    const i64 b = (i64)seg_lds_budget() - (back ? LV_RED * 16 * 8 : 0);
+    return std::min<i64>(b / (back ? 16 : 8), 1 << LV_SLOT_BITS);
+}
+
+// The blocks, bins and pair lists of (spin, pair or row run, rank kb); NULL if the pool is not
+// particle-hole in that spin or a block does not fit the LDS even for one vector
+static LevelPlan *level_plan(DevPool *P, int spin, bool pair, int kb) {
+    if (kb < 1 || kb > 4 || (P->cm[spin] & P->am[spin]) != 0) return nullptr;
+    auto &slot = P->lv[spin][pair ? 1 : 0][kb];
+    if (slot) return slot->ok ? slot.get() : nullptr;
+    slot = std::make_unique<LevelPlan>();
+    LevelPlan &L = *slot;
+    const HostBasis &hb = P->basis->host;
+    if (hb.norb > 32) return nullptr;
+    const SpinSpace &S = spin == 0 ? hb.A : hb.B;
+    const u64 C = P->cm[spin], out = ~(C | P->am[spin]);
+    // blocks: occupation outside A and C, and the level (pair) or the level modulo kb (row)
+    std::map<std::pair<u64, int>, std::vector<u32>> blocks;  // slots: element | row << 31
+    for (i64 i = 0; i < S.N; ++i) {
+        const u64 s = S.strs[i];
+        const int c = __builtin_popcountll(s & C);
+        if (pair) {
+            blocks[{s & out, c}].push_back((u32)i);
+            if (c >= kb) blocks[{s & out, c - kb}].push_back((u32)i | 0x80000000u);
+        } else {
+            blocks[{s & out, c % kb}].push_back((u32)i);
+        }
+    }
+    std::vector<std::vector<u32>> bl;
+    for (auto &kv : blocks) {
+        auto &v = kv.second;
+        bool two = false;  // both sides of a pair, or more than one level
+        const int c0 = __builtin_popcountll(S.strs[v[0] & 0x7fffffffu] & C);
+        for (u32 e : v) two |= pair ? (e >> 31) != (v[0] >> 31) : __builtin_popcountll(S.strs[e] & C) != c0;
+        if (two) {
+            if (pair) std::stable_sort(v.begin(), v.end(), [](u32 a, u32 b) { return (a >> 31) < (b >> 31); });
+            bl.push_back(std::move(v));
+        }
+    }
+    std::stable_sort(bl.begin(), bl.end(), [](const auto &a, const auto &b) { return a.size() > b.size(); });
+    if (bl.empty() || (i64)bl[0].size() > lv_cap(false)) return nullptr;
+    // bins: largest blocks first, smaller ones added while a bin stays within 5/4 of the largest
+    // block (a bin of a few elements takes as long per generator as a full one) and the LDS
+    const i64 big = (i64)bl[0].size(), capb = lv_cap(big <= lv_cap(true));
+    const i64 cap = std::min(capb, big + big / 4);
+    std::vector<std::vector<u32>> bins;
+    for (auto &v : bl) {
+        size_t b = 0;
+        while (b < bins.size() && (i64)(bins[b].size() + v.size()) > cap) ++b;
+        if (b == bins.size()) bins.emplace_back();
+        bins[b].insert(bins[b].end(), v.begin(), v.end());
+    }
+    L.nbins = (int)bins.size();
+    // slot of an element: [row side][element]
+    std::vector<int> bin_of[2], loc[2];
+    for (int q = 0; q < 2; ++q) bin_of[q].assign(S.N, -1), loc[q].assign(S.N, 0);
+    std::vector<uint2> slots;
+    std::vector<int> soff{0};
+    for (int b = 0; b < L.nbins; ++b) {
+        for (size_t i = 0; i < bins[b].size(); ++i) {
+            const u32 e = bins[b][i], el = e & 0x7fffffffu;
+            for (int q = 0; q < 2; ++q)
+                if (!pair || q == (int)(e >> 31)) bin_of[q][el] = b, loc[q][el] = (int)i;
+            u64 word = S.strs[el];
+            if (spin == 0) {
+                word = 0;
+                for (u64 m = S.strs[el]; m; m &= m - 1) word ^= (m & (~m + 1)) - 1;
+            }
+            slots.push_back(make_uint2(e, (u32)word));
+        }
+        soff.push_back((int)slots.size());
+        L.maxslot = std::max(L.maxslot, (int)bins[b].size());
+    }
+    // pair lists of every pattern of this rank, by bin
+    std::vector<u32> list;
+    L.pat.assign(P->lists.size(), -1);
+    for (size_t q = 2; q < P->lists.size(); ++q) {
+        const PairList &pl = P->lists[q];
+        if (pl.spin != spin || __builtin_popcountll(pl.cre) != kb) continue;
+        L.pat[q] = (int)(L.ol.size() / L.nbins);
+        std::vector<std::vector<u32>> w(L.nbins);
+        for (i64 j = 0; j < pl.len; ++j) {
+            const int u = pl.h[2 * j], v = pl.h[2 * j + 1];
+            const int b = bin_of[0][u];
+            HIPOTF_REQUIRE(b >= 0 && b == bin_of[1][v], "internal: a pair leaves its level block");
+            w[b].push_back((u32)loc[0][u] | ((u32)loc[1][v] << LV_SLOT_BITS) |
+                           ((u32)lv_canon(S.strs[u], pl.cre, pl.ann) << 31));
+        }
+        for (int b = 0; b < L.nbins; ++b) {
+            L.ol.push_back(make_int2((int)list.size(), (int)w[b].size()));
+            L.maxlen = std::max(L.maxlen, (int)w[b].size());
+            list.insert(list.end(), w[b].begin(), w[b].end());
+        }
+    }
+    list.push_back(0);  // (an empty list at the end is still read at its first word)
+    HIPOTF_REQUIRE(list.size() < (1u << 31), "internal: level lists too long");
+    L.slots.upload(slots);
+    L.soff.upload(soff);
+    L.list.upload(list);
+    L.ok = true;
+    return &L;
+}
+
+// threads of a run's workgroups: LV_NP list words per thread cover the longest list
+static int lv_threads(const LevelPlan &L) {
+    const int t = (L.maxlen + LV_NP - 1) / LV_NP;
+    return std::min(1024, std::max(64, (t + 63) / 64 * 64));
+}
