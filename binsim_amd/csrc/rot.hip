@@ -956,7 +956,7 @@ static std::vector<Segment> plan_sweep(DevPool *P, const i64 *idxs, i64 n, int n
         };
         auto plan_of = [&](int k) -> LevelPlan * {
             LevelPlan *lp = k > 0 ? level_plan(P, spin, pair, k) : nullptr;
-            return lp && (nvec == 1 || lp->maxslot <= lv_cap(true)) ? lp : nullptr;
+            return lp && (nvec == 1 || (lp->maxslot <= lv_cap(true) && lp->maxlen <= 2048)) ? lp : nullptr;
         };
         for (i64 j = s.first, end = s.first + s.count; j < end;) {
             const int k = rank(j);
@@ -1174,18 +1174,26 @@ static void sweeps(DevPool *P, i64 n, const i64 *idxs, const double *thetas, con
             a.gstride = n;
             a.list = s.lv->list.as<u32>();
             if (back) a.partial = pend_add(s);
-            const int bd = lv_threads(*s.lv);
-            const size_t smem = (size_t)s.lv->maxslot * (back ? 16 : 8) + (back ? (size_t)LV_RED * (bd / 64) * 8 : 0);
             const i64 nblk = (a.nunit * a.nbins + 7) / 8 * 8;
+            const int np = lv_words(*s.lv, back, nblk), bd = lv_threads(*s.lv, np);
+            const size_t smem = lv_lds(*s.lv, back, bd);
             HIPOTF_REQUIRE(nblk < (1ll << 31), "rotation sweep grid too large");
             auto go = [&](auto kern) {
                 HIPOTF_CHECK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                                  (int)smem));
                 hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(bd), smem, st, a);
             };
-            if (grad) go(k_lv<2>);
-            else if (back) go(k_lv<1>);
-            else go(k_lv<0>);
+            if (np == 1) {
+                if (grad) go(k_lv<2, 1>);
+                else if (back) go(k_lv<1, 1>);
+                else go(k_lv<0, 1>);
+            } else if (np == 2) {
+                if (grad) go(k_lv<2, 2>);
+                else if (back) go(k_lv<1, 2>);
+                else go(k_lv<0, 2>);
+            } else {
+                go(k_lv<0, 4>);  // (plan_of admits lists this long forward only)
+            }
             HIPOTF_CHECK(hipGetLastError());
         };
         // interleaved pair segments: z = (psi, lam) element by element, made before the first

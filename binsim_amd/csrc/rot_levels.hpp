@@ -17,7 +17,12 @@
 // 128 bytes per cycle and CU; then the latency of a generator's phase (LDS read, a dependent
 // chain of four FP64 operations, LDS write, barrier).  The pair lists are compact (one word per
 // pair: two 14-bit slots and a sign, 0.9 MB for the 64 beta singles at 16 orbitals, L2 resident),
-// and the words and the angle of the next generator are loaded while the current one runs.
+// and the words and angles of later generators are loaded while the current one runs.
+// Measured at 16 orbitals (energy + gradient): pair runs 504 -> 143 ms adjoint and 212 -> 66 ms
+// forward against row pairs in global memory, rows of doubles 151 -> 60 and 99 -> 21 ms; the LDS
+// is busy half of an adjoint pair run.  Not kept: list words ordered so that no two of 16 (32)
+// threads share a bank (an edge colouring: -1.5%, 0.1 s more in the first pass), l and r in
+// separate arrays (same).
 //
 // Signs.  The elements are held in the alpha-major gauge x~ = (-1)^popc(b & M(a)) x, where a
 // generator's sign splits into one factor per spin: the moved strings' factor is a bit of the
@@ -26,12 +31,13 @@
 #pragma once
 
 constexpr int LV_SLOT_BITS = 14;
-constexpr int LV_NP = 2;    // list words per thread and generator held ahead
+constexpr int LV_PAD = 4096; // words after the last list that idle threads may read
 constexpr int LV_RED = 64;  // generators between two flushes of the gradient sums
 
 struct LvGen {              // one generator as one bin sees it
     double c, s;
-    int32_t off, len;       // its words in the list
+    u32 off;                // its words in the list: first byte, count
+    int32_t len;
     u32 kap, pad;           // its constant sign (bit 31)
 };
 static_assert(sizeof(LvGen) == 32, "two 16-byte loads");
@@ -75,28 +81,37 @@ struct LvArgs {
     double *partial;        // [nunit * nbins][ng]
 };
 
-// sum over the wave, valid in lane 63 (VALU moves; a shuffle would go through the LDS, which
-// these kernels are bound by)
-__device__ __forceinline__ double wave_sum63(double v) {
-    auto step = [&](auto ctrl, auto rows) {
-        constexpr int CT = decltype(ctrl)::value, RM = decltype(rows)::value;
+// Wave sums of four values at once: lanes 12..15 end with the sums of a[0..3].  The values of two,
+// then four lanes are dealt to the lanes of a quad while they are added, so the four sums share
+// the later steps (8 VALU operations per value; one at a time takes 18).
+__device__ __forceinline__ double wave_sum4(const double (&a)[4]) {
+    const int lane = threadIdx.x & 63;
+    auto dpp = [](double v, auto ctrl) {
+        constexpr int CT = decltype(ctrl)::value;
         const long long b = __double_as_longlong(v);
-        const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CT, RM, 0xf, false);
-        const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CT, RM, 0xf, false);
-        v += __longlong_as_double(((long long)hi << 32) | (u32)lo);
+        const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CT, 0xf, 0xf, false);
+        const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CT, 0xf, 0xf, false);
+        return __longlong_as_double(((long long)hi << 32) | (u32)lo);
     };
-    step(std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xf>{});  // row_shr 1
-    step(std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xf>{});
-    step(std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xf>{});
-    step(std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xf>{});
-    step(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});  // row_bcast 15
-    step(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});  // row_bcast 31
-    return v;
+    using X1 = std::integral_constant<int, 0xb1>;   // quad_perm 1,0,3,2
+    using X2 = std::integral_constant<int, 0x4e>;   // quad_perm 2,3,0,1
+    using S4 = std::integral_constant<int, 0x114>;  // row_shr 4
+    using S8 = std::integral_constant<int, 0x118>;  // row_shr 8
+    const bool o1 = lane & 1, o2 = lane & 2;
+    const double u = (o1 ? a[1] : a[0]) + dpp(o1 ? a[0] : a[1], X1{});
+    const double v = (o1 ? a[3] : a[2]) + dpp(o1 ? a[2] : a[3], X1{});
+    double w = (o2 ? v : u) + dpp(o2 ? u : v, X2{});
+    w += dpp(w, S4{});
+    w += dpp(w, S8{});  // lanes 12..15 of each row of 16: the row's sums
+    w += __shfl_xor(w, 16, 64);
+    w += __shfl_xor(w, 32, 64);
+    return w;
 }
 
 // MODE 0: forward rotations of l; 1: adjoint step on (l, r) with gradient sums, generators in
-// reverse; 2: gradient sums only (nothing is written, so the generators need no barrier)
-template <int MODE>
+// reverse; 2: gradient sums only (nothing is written, so the generators need no barrier).  NP * bd
+// threads' words cover the longest list.
+template <int MODE, int NP>
 __global__ __launch_bounds__(1024) void k_lv(LvArgs a) {
     using E = typename std::conditional<MODE == 0, double, double2>::type;
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -105,10 +120,14 @@ __global__ __launch_bounds__(1024) void k_lv(LvArgs a) {
     if ((i64)(blockIdx.x >> 3) >= per || wk >= total) return;
     const i64 unit = wk / a.nbins;
     const int bin = (int)(wk - unit * a.nbins);
-    const int tid = threadIdx.x, bd = blockDim.x, lane = tid & 63, wave = tid >> 6, nw = bd >> 6;
+    const int tid = threadIdx.x, bd = blockDim.x, lane = tid & 63, nw = bd >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int s0 = a.soff[bin], ns = a.soff[bin + 1] - s0;
     E *x = reinterpret_cast<E *>(smem_raw);
-    double *red = reinterpret_cast<double *>(x + ns);  // [LV_RED][nw]
+    // x: the bin's elements, then a zero per lane that idle threads rotate (it stays zero), then the
+    // gradient sums [LV_RED][nw]
+    double *red = reinterpret_cast<double *>(x + ns + 64);
+    if (tid < 64) x[ns + tid] = E{};
     i64 ru = unit, rw = unit;
     int neg = 0;
     if (a.alist) {
@@ -140,28 +159,40 @@ __global__ __launch_bounds__(1024) void k_lv(LvArgs a) {
                 else x[i + q * bd] = make_double2(sgn(lv[q], f), sgn(rv[q], f));
             }
     }
-    // descriptors and list words by vector loads (their wait counter is not the LDS's)
+    // Descriptors and list words by vector loads (their wait counter is not the LDS's), four and two
+    // generators ahead in register rings of four: the loads are waited for in the order they were
+    // issued, so a descriptor has to be older than the words in flight, and the generator loop is
+    // unrolled by four because moving a register waits for its load.
     u32 vz;
     asm("v_mov_b32 %0, 0" : "=v"(vz));
     const LvGen *G = a.gens + (i64)bin * a.gstride;
     auto gen_at = [&](int kk) { return MODE == 1 ? a.ng - 1 - min(kk, a.ng - 1) : min(kk, a.ng - 1); };
-    struct D { double c, s; int off, len; u32 kap; };
-    auto ld = [&](int kk) {
-        const LvGen *g = G + (gen_at(kk) + vz);
+    struct D { double c, s; u32 off; int len; u32 kap; };
+    auto ld = [&](D &d, int kk) {
+        const char *g = reinterpret_cast<const char *>(G) + ((u32)gen_at(kk) * (u32)sizeof(LvGen) + vz);
         const double2 cs = *reinterpret_cast<const double2 *>(g);
-        const int4 ol = *reinterpret_cast<const int4 *>(&g->off);
-        return D{cs.x, cs.y, ol.x, ol.y, (u32)ol.z};
+        const int4 ol = *reinterpret_cast<const int4 *>(g + 16);
+        d.c = cs.x, d.s = cs.y, d.off = (u32)ol.x, d.len = ol.y, d.kap = (u32)ol.z;
     };
-    auto words = [&](const D &d, u32 (&e)[LV_NP]) {  // clamped: unused words are never applied
+    // (threads past the end of a list read words of later ones, or the padding: slots of this plan
+    // all the same, which they do not use)
+    const u32 tid4 = (u32)tid * 4, bd4 = (u32)bd * 4;
+    auto word = [&](u32 at) { return *reinterpret_cast<const u32 *>(reinterpret_cast<const char *>(a.list) + at); };
+    auto words = [&](const D &d, u32 (&e)[NP]) {
 #pragma unroll
-        for (int q = 0; q < LV_NP; ++q) e[q] = a.list[d.off + max(0, min(tid + q * bd, d.len - 1))];
+        for (int q = 0; q < NP; ++q) e[q] = word(d.off + tid4 + q * bd4);
     };
     const u32 sflip = (u32)neg << 31;
-    D d0 = ld(0), d1 = ld(1);
-    u32 e0[LV_NP], e1[LV_NP];
-    words(d0, e0);
+    D d[4];
+    u32 e[4][NP];
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) ld(d[q], q);
+    words(d[0], e[0]);
+    words(d[1], e[1]);
     __syncthreads();
     constexpr u32 SM = (1u << LV_SLOT_BITS) - 1;
+    const u32 idle = (u32)(ns + lane);  // (a wave's idle threads rotate its own zeros)
     auto flush = [&](int k1, int cnt) {  // gradient sums of the cnt generators before order position k1
         __syncthreads();
         if (tid < cnt) {
@@ -171,72 +202,84 @@ __global__ __launch_bounds__(1024) void k_lv(LvArgs a) {
         }
         __syncthreads();
     };
-    for (int kk = 0; kk < a.ng; ++kk) {
-        const D d2 = ld(kk + 2);
-        words(d1, e1);
-        double acc = 0.0;
-        const double c = d0.c, s = d0.s;
-        const u32 gf = sflip ^ d0.kap;
-        auto body = [&](u32 e, E &xu, E &xw, bool act) {
-            const u32 sf = (e & 0x80000000u) ^ gf;
-            const double ts = sgn(s, sf);
-            if constexpr (MODE == 0) {
-                const double nu = c * xu - ts * xw, nw_ = ts * xu + c * xw;
-                if (act) {
-                    x[e & SM] = nu;
-                    x[(e >> LV_SLOT_BITS) & SM] = nw_;
+    auto reduce4 = [&](int k0) {  // the sums of generators k0 .. k0 + 3
+        const double t = wave_sum4(acc);
+        if ((lane & 60) == 12) red[(k0 % LV_RED + (lane & 3)) * nw + wave] = t;
+    };
+    auto step = [&](auto qc, int kk) {
+        constexpr int Q = decltype(qc)::value;
+        words(d[(Q + 2) & 3], e[(Q + 2) & 3]);
+        const double c = d[Q].c, s = d[Q].s;
+        const u32 gf = sflip ^ d[Q].kap;
+        const int len = kk < a.ng ? d[Q].len : 0;
+        if constexpr (MODE != 0 && Q == 0) {
+            if (kk) {  // the previous four generators' sums
+                reduce4(kk - 4);
+                if (kk % LV_RED == 0) flush(kk, LV_RED);
+            }
+        }
+        // the wave's first N words per thread (waves past the end of the list skip them)
+        double sa = 0.0, sb = 0.0;
+        auto apply = [&](auto nc) {
+            constexpr int N = decltype(nc)::value;
+            E xu[N], xw[N];
+            u32 pu[N], pw[N];
+#pragma unroll
+            for (int q = 0; q < N; ++q) {
+                const bool act = tid + q * bd < len;
+                pu[q] = act ? e[Q][q] & SM : idle;
+                pw[q] = act ? (e[Q][q] >> LV_SLOT_BITS) & SM : idle;
+                xu[q] = x[pu[q]];
+                xw[q] = x[pw[q]];
+            }
+#pragma unroll
+            for (int q = 0; q < N; ++q) {
+                const u32 sf = (e[Q][q] & 0x80000000u) ^ gf;
+                const double ts = sgn(s, sf);
+                if constexpr (MODE == 0) {
+                    x[pu[q]] = c * xu[q] - ts * xw[q];
+                    x[pw[q]] = ts * xu[q] + c * xw[q];
+                } else if constexpr (MODE == 1) {
+                    const double nlu = c * xu[q].x + ts * xw[q].x, nru = c * xu[q].y + ts * xw[q].y;
+                    const double nlw = c * xw[q].x - ts * xu[q].x, nrw = c * xw[q].y - ts * xu[q].y;
+                    // d/dtheta of the rotated r is t (r_w, -r_u) of the new values
+                    sa += sgn(nlu * nrw - nlw * nru, sf);
+                    x[pu[q]] = make_double2(nlu, nru);
+                    x[pw[q]] = make_double2(nlw, nrw);
+                } else {
+                    sa += xu[q].x * xu[q].y + xw[q].x * xw[q].y;
+                    sb += sgn(xu[q].x * xw[q].y - xw[q].x * xu[q].y, sf);
                 }
-            } else if constexpr (MODE == 1) {
-                const double tc = sgn(c, sf);
-                const double nlu = c * xu.x + ts * xw.x, nlw = -ts * xu.x + c * xw.x;
-                const double g = nlu * (-s * xu.y + tc * xw.y) + nlw * (-s * xw.y - tc * xu.y);
-                if (act) {
-                    acc += g;
-                    x[e & SM] = make_double2(nlu, c * xu.y + ts * xw.y);
-                    x[(e >> LV_SLOT_BITS) & SM] = make_double2(nlw, -ts * xu.y + c * xw.y);
-                }
-            } else {
-                const double tc = sgn(c, sf);
-                const double g = xu.x * (-s * xu.y + tc * xw.y) + xw.x * (-s * xw.y - tc * xu.y);
-                if (act) acc += g;
             }
         };
-        E xu[LV_NP], xw[LV_NP];
-#pragma unroll
-        for (int q = 0; q < LV_NP; ++q) {
-            xu[q] = x[e0[q] & SM];
-            xw[q] = x[(e0[q] >> LV_SLOT_BITS) & SM];
-        }
-#pragma unroll
-        for (int q = 0; q < LV_NP; ++q) body(e0[q], xu[q], xw[q], tid + q * bd < d0.len);
-        for (int j = tid + LV_NP * bd; j < d0.len; j += bd) {
-            const u32 e = a.list[d0.off + j];
-            E yu = x[e & SM], yw = x[(e >> LV_SLOT_BITS) & SM];
-            body(e, yu, yw, true);
-        }
-        if constexpr (MODE != 0) {
-            const double t = wave_sum63(acc);
-            if (lane == 63) red[(kk % LV_RED) * nw + wave] = t;
-        }
+        const int left = __builtin_amdgcn_readfirstlane(len - wave * 64);
+        if (left > (NP > 1 ? bd : 0)) apply(std::integral_constant<int, NP>{});
+        else if (left > 0) apply(std::integral_constant<int, 1>{});
+        acc[Q] = MODE == 2 ? c * sb - s * sa : sa;
+        ld(d[Q], kk + 4);
         if constexpr (MODE != 2) __syncthreads();
-        if constexpr (MODE != 0)
-            if (kk % LV_RED == LV_RED - 1) flush(kk + 1, LV_RED);
-        d0 = d1;
-        d1 = d2;
-#pragma unroll
-        for (int q = 0; q < LV_NP; ++q) e0[q] = e1[q];
+    };
+    for (int kk = 0; kk < a.ng; kk += 4) {  // (steps past the last generator have no pairs)
+        step(std::integral_constant<int, 0>{}, kk);
+        step(std::integral_constant<int, 1>{}, kk + 1);
+        step(std::integral_constant<int, 2>{}, kk + 2);
+        step(std::integral_constant<int, 3>{}, kk + 3);
     }
-    if constexpr (MODE != 0)
-        if (a.ng % LV_RED) flush(a.ng, a.ng % LV_RED);
+    if constexpr (MODE != 0) {
+        const int k0 = (a.ng - 1) & ~3;
+        reduce4(k0);
+        flush(a.ng, a.ng - k0 / LV_RED * LV_RED);
+    }
     if constexpr (MODE != 2) {
         for (int i = tid; i < ns; i += bd) {
             const uint2 sl = a.slots[s0 + i];
             const u32 f = flip(sl);
+            const E v = x[i];
             if constexpr (MODE == 0) {
-                a.l[at(sl)] = sgn(x[i], f);
+                a.l[at(sl)] = sgn(v, f);
             } else {
-                a.l[at(sl)] = sgn(x[i].x, f);
-                a.r[at(sl)] = sgn(x[i].y, f);
+                a.l[at(sl)] = sgn(v.x, f);
+                a.r[at(sl)] = sgn(v.y, f);
             }
         }
     }
@@ -358,7 +401,10 @@ static size_t seg_lds_budget();
 // largest bin: (l, r) values with the gradient sums of 16 waves beside them, or l alone
 static i64 lv_cap(bool back) {
     const i64 b = (i64)seg_lds_budget() - (back ? LV_RED * 16 * 8 : 0);
-    return std::min<i64>(b / (back ? 16 : 8), 1 << LV_SLOT_BITS);
+    return std::min<i64>(b / (back ? 16 : 8), 1 << LV_SLOT_BITS) - 64;
+}
+static size_t lv_lds(const LevelPlan &L, bool back, int bd) {
+    return ((size_t)L.maxslot + 64) * (back ? 16 : 8) + (back ? (size_t)LV_RED * (bd / 64) * 8 : 0);
 }
 
 // The blocks, bins and pair lists of (spin, pair or row run, rank kb); NULL if the pool is not
@@ -446,13 +492,14 @@ static LevelPlan *level_plan(DevPool *P, int spin, bool pair, int kb) {
                            ((u32)lv_canon(S.strs[u], pl.cre, pl.ann) << 31));
         }
         for (int b = 0; b < L.nbins; ++b) {
-            L.ol.push_back(make_int2((int)list.size(), (int)w[b].size()));
+            L.ol.push_back(make_int2((int)list.size() * 4, (int)w[b].size()));
             L.maxlen = std::max(L.maxlen, (int)w[b].size());
             list.insert(list.end(), w[b].begin(), w[b].end());
         }
     }
-    list.push_back(0);  // (an empty list at the end is still read at its first word)
-    HIPOTF_REQUIRE(list.size() < (1u << 31), "internal: level lists too long");
+    if (L.maxlen > 4 * 1024) return nullptr;
+    list.resize(list.size() + LV_PAD, 0u);
+    HIPOTF_REQUIRE(list.size() < (1u << 29), "internal: level lists too long");
     L.slots.upload(slots);
     L.soff.upload(soff);
     L.list.upload(list);
@@ -460,8 +507,20 @@ static LevelPlan *level_plan(DevPool *P, int spin, bool pair, int kb) {
     return &L;
 }
 
-// threads of a run's workgroups: LV_NP list words per thread cover the longest list
-static int lv_threads(const LevelPlan &L) {
-    const int t = (L.maxlen + LV_NP - 1) / LV_NP;
-    return std::min(1024, std::max(64, (t + 63) / 64 * 64));
+// Threads of a run's workgroups, and list words per thread (1, 2 or 4) to cover the longest list.
+// Two words per thread share the descriptor work, but where few waves are in flight on a CU (a
+// bin that fills the LDS, or a small grid) a generator's phase is latency and one word on twice the
+// waves is faster (12 orbitals: adjoint runs 31 -> 24 us, forward 24 -> 18; 14 orbitals, nine bins
+// per CU: forward 12.2 ms per sweep with two words, 13.5 with one).  More than four waves
+// come in whole rounds of the CU's four SIMDs.
+static int lv_threads(const LevelPlan &L, int np) {
+    const int t = (L.maxlen + np - 1) / np, m = t > 256 ? 256 : 64;
+    return std::max(64, (t + m - 1) / m * m);
+}
+static int lv_words(const LevelPlan &L, bool back, i64 nblk) {
+    if (L.maxlen > 2048) return 4;
+    if (L.maxlen > 1024) return 2;
+    const int bd = lv_threads(L, 2);
+    const i64 perCU = std::min<i64>((i64)(seg_lds_budget() / lv_lds(L, back, bd)), (nblk + 255) / 256);
+    return perCU * (bd / 64) >= 16 ? 2 : 1;
 }
