@@ -1,4 +1,4 @@
-// Alpha-beta part of the sigma build on the matrix cores (included by sigma.hip), n <= 16.
+// Alpha-beta part of the sigma build on the matrix cores (included by sigma.hip), n <= 18.
 //
 // For a destination alpha row Ia, with c running over its alpha connections -- the nsxA single
 // excitations Ja_c = Ia - p_c + q_c with sign s_c, then Ia itself with the diagonal integral
@@ -13,47 +13,39 @@
 // Jb as it is (sgn = +1).  Y is a dense product of the n(n+1)/2 x nca matrix W with the
 // nca x NB matrix of source rows, so it runs as 16x16x4 MFMA tiles (FP64 or FP32 units) with
 // no gathers: the rows that do not apply to a Jb are computed and dropped (47% of them at 16
-// orbitals / 8 electrons).  Each applying element of Y is then added into an FP64 LDS copy of
-// the destination row (ds_add_f64), with the target rank read from two colex tables (low and
-// high byte of the 16-bit string).  Same sums as the source-lane kernel (ab_src.hpp), in
-// another order.
+// orbitals / 8 electrons).  Each element of Y is then added into an FP64 LDS copy of the
+// destination row (ds_add_f64).  Same sums as the source-lane kernel (ab_src.hpp), in another
+// order.
+//
+// Scatter.  Where an element of Y goes depends on (row, Jb) only, not on Ia, so targets come
+// from a table built once per basis (k_ab_targets): one 16-bit word per element, bit 15 the
+// sign, bits 0..14 the place among the destination elements, an element that does not apply
+// pointing at a spare place of its lane.  The words are in MFMA-result order: a lane reads the
+// four of a row tile as one 8-byte load (3.7 MB in all at 16 orbitals, served by the L2).  On
+// gfx950 FP64 MFMAs and VALU operations of a SIMD do not overlap, so the VALU work per element
+// is what the kernel pays on top of its products: 4 operations here, 22 when the validity, the
+// colex rank and the sign were computed in place.  Measured, FP64, 16 orbitals / 8 + 8
+// electrons: 33.1 -> 28.4 ms per launch (two launches; 20.7 ms of MFMA issue each); FP32, 14 orbitals, per
+// vector: 2.85 -> 1.57 ms with the row tiles and k-steps of 14 orbitals (7 x 13) instead of 16 (9 x 17).
 //
 // Workgroup = destination alpha row (XCD-interleaved like the other alpha-beta kernels),
 // NWV waves; beta strings in tiles of 16 (the MFMA's N), tiles dealt to the waves round robin.
-// W sits in LDS in MFMA-operand order for KSP k-steps (4 connections each) at a time: the A
-// operand of tile (k-step s, row tile m) for lane l is entry (s * MT + m) * 64 + l, a
-// conflict-free 8- or 4-byte read.
+// W sits in LDS in MFMA-operand order: the A operand of tile (k-step s, row tile m) for lane l
+// is entry (s * MT + m) * 64 + l, a conflict-free 8- or 4-byte read.
 //
-// Two forms.  Whole row (FP32): the LDS holds all NB destination elements and W (39 KB at 16
-// orbitals), one launch.  Class split (FP64, CLS): the 78 KB of FP64 W do not fit beside a
-// whole 103 KB FP64 row, so the destinations are split by the top orbital tb = n - 1 into
-// class N (tb empty: ranks [0, NN) in colex order) and class T (the rest), one launch per
-// class with only that class in LDS.  A target stays in the class of its source unless the
-// pair moves an electron onto or off tb, so the launch for class K computes the 8 row tiles of
-// the pairs without tb (and r = t = tb) on the class-K sources, and the one tile of pairs
-// (r, tb) on the sources of the other class: every element of Y is computed once over both
-// launches.
+// Two forms.  Whole row (MC = 0): the LDS holds all NB destination elements and W, one launch.
+// Class split (MC > 0), where they do not fit together (FP64 from 16 orbitals / 7 electrons):
+// the destinations are split by the top orbital tb = n - 1 into class N (tb empty: ranks [0, NN)
+// in colex order) and class T (the rest), one launch per class with only that class in LDS.  A
+// target stays in the class of its source unless the pair moves an electron onto or off tb, so
+// the launch for class K computes the MO row tiles of the pairs without tb (and all r = t) on the
+// class-K sources, and the MC tiles of pairs (r, tb) on the sources of the other class: every
+// element of Y is computed once over both launches.
 //
 // Operand layout of v_mfma_{f64,f32}_16x16x4 on gfx950 (measured): lane l holds A[l % 16][l / 16]
 // and B[l / 16][l % 16]; result element v of lane l is D[4 (l / 16) + v][l % 16] for f32 and
 // D[4 v + l / 16][l % 16] for f64.
 #pragma once
-
-// colex rank tables: low byte (256), (low-byte count, high byte) (9 x 256)
-constexpr int AB_MMA_RANKS = 256 + 9 * 256;
-
-// waves per workgroup (one workgroup per CU: the LDS holds the FP64 destination elements): 16
-// for both forms (128 / 116 VGPRs).  Measured at 16 orbitals: FP64 with 8 waves (row masks in
-// registers, B one tile ahead: 256 VGPRs) 1.4% slower, 12 waves 0.5% slower; FP32 with 12
-// waves 2% slower, 8 waves 6% slower.
-constexpr int AB_MMA_NWV64 = 16, AB_MMA_NWV32 = 16;
-
-__device__ __forceinline__ u32 ab_mma_binom(int a, int b) {
-    if (b < 0 || b > a) return 0u;
-    u32 c = 1;
-    for (int i = 0; i < b; ++i) c = c * (u32)(a - i) / (u32)(i + 1);
-    return c;
-}
 
 template <typename T>
 struct AbMmaOps;
@@ -74,88 +66,108 @@ struct AbMmaOps<float> {
     static constexpr __device__ int row(int g, int v) { return 4 * g + v; }
 };
 
-// LDS bytes of k_ab_mma with NS destination elements in LDS
-template <typename T, int MT, int KSP, int NWV>
-constexpr size_t ab_mma_lds(i64 NS) {
-    return (size_t)NS * sizeof(double) + (size_t)KSP * MT * 64 * sizeof(T) + MT * 16 * 4 +
-           AB_MMA_RANKS * 2 + AB_SRC_CONN * 4 + NWV * 64 * sizeof(double);
-}
-
-// Orbital pair (r <= t) of W row i, or r = t = -1 for a row that never applies.
-//   whole row: tile 0 the rows r = t, tiles 1-2 the pairs inside the low byte (r < t < 8),
-//     tiles 3-4 inside the high byte (8 <= r < t), tiles 5-8 across (r < 8 <= t, row
-//     80 + 8 r + t - 8);
-//   class split (tb = n - 1): tile 0 the rows r = t, tiles 1-2 the low-byte pairs with t < tb,
-//     tiles 3-7 the pairs inside orbitals 8..14, then those across (r < 8 <= t <= 14), each
-//     kept when t < tb, tile 8 the pairs (r, tb), r < tb.
-// The tile of a row fixes how its target rank is formed: with one table read when the pair
-// lies inside the low byte (tiles 1-2) or (whole row) inside the high byte (tiles 3-4).
-template <bool CLS>
-__device__ inline void ab_mma_pair(int i, int n, int &r, int &t) {
-    // e-th pair a < b of the w orbitals from `base`, e < w (w - 1) / 2
-    auto in_run = [](int e, int base, int w, int &a, int &b) {
-        int p = 0;
-        while (e >= w - 1 - p) {
-            e -= w - 1 - p;
-            ++p;
-        }
-        a = base + p;
-        b = a + 1 + e;
-    };
-    const int tb = n - 1;
+// Orbital pair (r <= t) of W row i, or r = t = -1 for a padding row.  Rows r = t sit at result
+// element v of lane group 0, four to a tile (the four groups of an instruction then never add to
+// one place), the pairs r < t fill the other places in order.  Class split (mc > 0): rows below
+// 16 mo as described for orbitals below tb = n - 1 (and r = t = tb), then the pairs (r, tb).
+template <typename T>
+__host__ __device__ inline void ab_mma_pair(int i, int n, int mo, int mc, int &r, int &t) {
     r = t = -1;
-    if (i < 16) {
-        r = t = i;
-    } else if (i < 48) {
-        if (i - 16 < 28) in_run(i - 16, 0, 8, r, t);
-    } else if (!CLS) {
-        if (i < 80) {
-            if (i - 48 < 28) in_run(i - 48, 8, 8, r, t);
-        } else {
-            r = (i - 80) >> 3;
-            t = 8 + ((i - 80) & 7);
+    if (i >= 16 * mo) {
+        if (i - 16 * mo < n - 1) {
+            r = i - 16 * mo;
+            t = n - 1;
         }
-    } else if (i < 128) {
-        const int e = i - 48;
-        if (e < 21) {
-            in_run(e, 8, 7, r, t);
-        } else if (e < 77) {
-            r = (e - 21) / 7;
-            t = 8 + (e - 21) % 7;
-        }
-    } else {
-        r = i - 128;
-        t = tb;
+        return;
     }
-    bool ok = r >= 0 && t < n;
-    if (CLS && ok && i >= 16) ok = i < 128 ? t < tb : r < tb;
-    if (!ok) r = t = -1;
+    const int tile = i >> 4, q = i & 15, left = n - 4 * tile;  // r = t rows of this tile: min(4, left)
+    const bool f64 = sizeof(T) == 8;
+    const int v = f64 ? q >> 2 : q;                              // place among group 0's elements
+    if ((f64 ? (q & 3) == 0 : q < 4) && v < left) {
+        r = t = 4 * tile + v;
+        return;
+    }
+    int before = f64 ? (q + 3) >> 2 : (q < 4 ? q : 4);  // r = t places before q
+    if (before > left) before = left > 0 ? left : 0;
+    int e = i - ((4 * tile < n ? 4 * tile : n) + before);
+    const int w = mc ? n - 1 : n;
+    for (int a = 0; a < w - 1; ++a) {
+        if (e < w - 1 - a) {
+            r = a;
+            t = a + 1 + e;
+            return;
+        }
+        e -= w - 1 - a;
+    }
 }
 
-// nks = k-steps of all connections, ceil((nsxA + 1) / 4); dw rows are nwd entries wide.
-// CLS: destination class cls (0: ranks [0, NN), 1: [NN, NB)); otherwise the whole row.
-template <typename T, int MT, int KSP, int NWV, bool CLS>
-__global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(NWV / 4, NWV / 4)))
+__device__ __forceinline__ u32 ab_colex_rank(u64 s) {
+    u32 rank = 0, j = 0;
+    for (; s; s &= s - 1) {
+        const u32 p = (u32)__builtin_ctzll(s);
+        ++j;
+        u32 c = j <= p ? 1u : 0u;  // C(p, j)
+        for (u32 i = 0; i < j && c; ++i) c = c * (p - i) / (i + 1);
+        rank += c;
+    }
+    return rank;
+}
+
+// target words of row tile m of column tile ct, one uint2 (result elements 0..3) per lane; column
+// tiles of class N, then of class T (NN = NB and one class without a split)
+template <typename T>
+__global__ __launch_bounds__(64) void k_ab_targets(const u64 *__restrict__ strsB, int n, int NB, int NN, int mo,
+                                                   int mc, uint2 *__restrict__ tab) {
+    const int ct = blockIdx.x, m = blockIdx.y, lane = threadIdx.x, g = lane >> 4, col = lane & 15;
+    const int nctN = (NN + 15) >> 4, cls = ct >= nctN;
+    const int b0 = cls ? NN : 0, nb = cls ? NB - NN : NN, Jl = (ct - (cls ? nctN : 0)) * 16 + col;
+    const int tc = m < mo ? cls : 1 - cls;                            // class of the targets
+    const int t0 = tc ? NN : 0, nt = mc ? (tc ? NB - NN : NN) : NB;   // its first rank and size
+    u32 w[4];
+    for (int v = 0; v < 4; ++v) {
+        int r, t;
+        ab_mma_pair<T>(m * 16 + AbMmaOps<T>::row(g, v), n, mo, mc, r, t);
+        w[v] = (u32)(nt + lane);
+        if (r >= 0 && Jl < nb) {
+            const u64 s = strsB[b0 + Jl], ob = (1ull << r) | (1ull << t);
+            if (r == t) {
+                if (s & ob) w[v] = (u32)(b0 + Jl - t0);
+            } else if (__popcll(s & ob) == 1) {
+                const u64 between = ((1ull << t) - 1) & ~((2ull << r) - 1);
+                w[v] = (ab_colex_rank(s ^ ob) - (u32)t0) | ((u32)(__popcll(s & between) & 1) << 15);
+            }
+        }
+    }
+    tab[((i64)ct * (mo + mc) + m) * 64 + lane] = make_uint2(w[0] | w[1] << 16, w[2] | w[3] << 16);
+}
+
+// LDS bytes of k_ab_mma with NS destination elements in LDS
+template <typename T, int MT, int KS>
+constexpr size_t ab_mma_lds(i64 NS) {
+    return (size_t)(NS + 64) * sizeof(double) + (size_t)KS * MT * 64 * sizeof(T) + (AB_SRC_CONN + 4 * 20) * 4 + MT * 16 * 4;
+}
+
+// KS: k-steps of 4 connections (4 KS >= nsxA + 1); dw rows are nwd entries wide.  MC > 0:
+// destination class cls (0: ranks [0, NN), 1: [NN, NB)); otherwise the whole row (NN = NB).
+template <typename T, int MO, int MC, int KS, int NWV, int WPE>
+__global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
 void k_ab_mma(const T *__restrict__ xt, T *__restrict__ s1, int nvst, int v0, const u32 *__restrict__ sxA,
-              const u64 *__restrict__ strsB, const T *__restrict__ eri, const T *__restrict__ dw, int nwd, int n,
-              i64 NA, int NB, int nsxA, int nks, int cls, int NN) {
+              const uint2 *__restrict__ tab, const T *__restrict__ eri, const T *__restrict__ dw, int nwd, int n,
+              i64 NA, int NB, int nsxA, int cls, int NN) {
     using Ops = AbMmaOps<T>;
     using V4 = typename Ops::V4;
-    constexpr int BD = NWV * 64;
-    static_assert(MT == 9, "row layout: 9 tiles of 16");
-    // own columns and destinations [o0, o0 + NK); other columns [c0, c0 + NC) (CLS only)
-    const int o0 = CLS && cls ? NN : 0, NK = CLS ? (cls ? NB - NN : NN) : NB;
-    const int c0 = CLS && !cls ? NN : 0, NC = CLS ? NB - NK : 0;
+    constexpr int BD = NWV * 64, MT = MO + MC, KR = 20;
+    static_assert(KS <= KR, "source row table");
+    // own columns and destinations [o0, o0 + NK); other columns [c0, c0 + NC) (MC > 0 only)
+    const int o0 = MC && cls ? NN : 0, NK = MC ? (cls ? NB - NN : NN) : NB;
+    const int c0 = MC && !cls ? NN : 0, NC = MC ? NB - NK : 0;
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    double *S = reinterpret_cast<double *>(smem_raw);                       // destinations
-    T *Wl = reinterpret_cast<T *>(smem_raw + (size_t)NK * sizeof(double));  // KSP x MT x 64
-    u32 *rinfo = reinterpret_cast<u32 *>(Wl + KSP * MT * 64);               // per W row
-    unsigned short *rk = reinterpret_cast<unsigned short *>(rinfo + MT * 16);
-    u32 *conn = reinterpret_cast<u32 *>(rk + AB_MMA_RANKS);
+    double *S = reinterpret_cast<double *>(smem_raw);                              // NK destinations, 64 spare
+    T *Wl = reinterpret_cast<T *>(smem_raw + (size_t)(NK + 64) * sizeof(double));  // KS x MT x 64
+    u32 *jrow = reinterpret_cast<u32 *>(Wl + KS * MT * 64);                        // source rows [g][KR]
+    u32 *conn = jrow + 4 * KR;
+    u32 *rowrt = conn + AB_SRC_CONN;                                               // r * n + t of a W row
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    // per-thread slot that takes the adds of the elements that do not apply (every element is
-    // added, unconditionally: no branches in the scatter; 1% faster than masked adds)
-    const u32 dmy = (u32)(reinterpret_cast<double *>(conn + AB_SRC_CONN) - S) + (u32)tid;
     const int g = lane >> 4, col = lane & 15;
     const i64 per = (NA + 7) / 8;
     const i64 Ia = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
@@ -163,182 +175,84 @@ void k_ab_mma(const T *__restrict__ xt, T *__restrict__ s1, int nvst, int v0, co
     const int n2 = n * n;
 
     for (int t = tid; t < nsxA; t += BD) conn[t] = sxA[(i64)t * NA + Ia];
-    // a row's entry: its orbital mask (low half) and the mask of the orbitals strictly between
-    // r and t (high half); 0 for a row that never applies
     for (int i = tid; i < MT * 16; i += BD) {
         int r, t;
-        ab_mma_pair<CLS>(i, n, r, t);
-        u32 v = 0;
-        if (r >= 0) v = r == t ? 1u << r : (1u << r) | (1u << t) | ((((1u << t) - (2u << r)) & 0xffffu) << 16);
-        rinfo[i] = v;
+        ab_mma_pair<T>(i, n, MO, MC, r, t);
+        rowrt[i] = r >= 0 ? (u32)(r * n + t) : ~0u;
     }
-    // colex ranks rank(s) = rk[s & 255] + rk[256 + 256 * popc(s & 255) + (s >> 8)], from the
-    // binomials C(a, b), a < 16, b <= 16, staged at the start of the (not yet used)
-    // destination and W area
-    u32 *bn = reinterpret_cast<u32 *>(S);
-    for (int e = tid; e < 16 * 17; e += BD) bn[e] = ab_mma_binom(e / 17, e % 17);
-    __syncthreads();
-    for (int e = tid; e < AB_MMA_RANKS; e += BD) {
-        const int hi = e >= 256;
-        const int k0 = hi ? (e - 256) >> 8 : 0, bits = hi ? (e - 256) & 255 : e, base = hi ? 8 : 0;
-        u32 v = 0;
-        int j = k0;
-        for (int q = 0; q < 8; ++q)
-            if ((bits >> q) & 1) {
-                v += j + 1 <= 16 ? bn[(base + q) * 17 + j + 1] : 0u;
-                ++j;
-            }
-        rk[e] = (unsigned short)v;
-    }
-    __syncthreads();
     for (int t = tid; t < NK; t += BD) S[t] = 0.0;
     __syncthreads();
-
-    // this lane's W row of result element v in row tile m
-    auto row_info = [&](int m, int v) -> u32 { return rinfo[m * 16 + Ops::row(g, v)]; };
-    const int npass = (nks + KSP - 1) / KSP;
-    for (int pass = 0; pass < npass; ++pass) {
-        const int s0 = pass * KSP;
-        // W of k-steps s0 .. s0 + KSP - 1 in operand order (zero past the last connection)
-        for (int e = tid; e < KSP * MT * 64; e += BD) {
-            const int l = e & 63, m = (e >> 6) % MT, s = (e >> 6) / MT;
-            const int i = m * 16 + (l & 15), c = 4 * (s0 + s) + (l >> 4);
-            T v = T(0);
-            const u32 om = rinfo[i] & 0xffffu;
-            if (om != 0u && c <= nsxA) {
-                const int r = __builtin_ctz(om), t = 31 - __builtin_clz(om);
-                if (c < nsxA) {
-                    const u32 d = conn[c];
-                    v = eri[(i64)(sx_r(d) * n + sx_s(d)) * n2 + r * n + t];
-                    if (sx_neg(d)) v = -v;
-                } else {
-                    v = dw[Ia * nwd + r * n + t];
-                }
+    // source rows of connection 4 s + g (past the last connection row Ia, against zero W)
+    for (int e = tid; e < 4 * KS; e += BD) jrow[(e & 3) * KR + (e >> 2)] = (e < nsxA ? sx_J(conn[e]) : (u32)Ia) * (u32)NB;
+    // W in operand order (zero past the last connection and in padding rows)
+    for (int e = tid; e < KS * MT * 64; e += BD) {
+        const int l = e & 63, m = (e >> 6) % MT, s = (e >> 6) / MT;
+        const int c = 4 * s + (l >> 4);
+        const u32 rt = rowrt[m * 16 + (l & 15)];
+        T v = T(0);
+        if (rt != ~0u && c <= nsxA) {
+            if (c < nsxA) {
+                const u32 d = conn[c];
+                v = eri[(i64)(sx_r(d) * n + sx_s(d)) * n2 + rt];
+                if (sx_neg(d)) v = -v;
+            } else {
+                v = dw[Ia * nwd + rt];
             }
-            Wl[e] = v;
         }
-        // this lane's source rows: connection 4 (s0 + s) + g (rows past the last connection
-        // read row Ia against zero W)
-        u32 jo[KSP];
-#pragma unroll
-        for (int s = 0; s < KSP; ++s) {
-            const int c = 4 * (s0 + s) + g;
-            const u32 Ja = c < nsxA ? sx_J(conn[c]) : (u32)Ia;
-            jo[s] = Ja * (u32)NB;
-        }
-        __syncthreads();
-
-        // the column tiles of [b0, b0 + nb) on the row tiles [M0, M0 + NM)
-        auto run = [&](auto m0_c, auto nm_c, int b0, int nb) {
-            constexpr int M0 = decltype(m0_c)::value, NM = decltype(nm_c)::value;
-            const int ntiles = (nb + 15) >> 4;
-            if (ntiles == 0) return;
-            // B operands and string of a tile, loaded unconditionally with clamped indices (a
-            // load on one path only would make the compiler drain every outstanding load)
-            auto load_tile = [&](T (&b)[KSP], u32 &jb, int nt) {
-                const int ntc = nt < ntiles ? nt : ntiles - 1;
-                const int Jl = ntc * 16 + col;
-                const int Jb = b0 + (Jl < nb ? Jl : nb - 1);
-#pragma unroll
-                for (int s = 0; s < KSP; ++s) b[s] = xt[(size_t)((jo[s] + (u32)Jb) * (u32)nvst + (u32)v0)];
-                jb = (u32)strsB[Jb];
-            };
-            // FP32: B operands loaded one tile ahead; FP64 (more registers per operand) loads
-            // them at the tile, the other waves covering the latency
-            constexpr bool PF = sizeof(T) == 4;
-            T bq[PF ? KSP : 1];
-            u32 jbq = 0;
-            if constexpr (PF) load_tile(bq, jbq, wave);
-            for (int nt = wave; nt < ntiles; nt += NWV) {
-                T b[KSP];
-                u32 jb;
-                if constexpr (PF) {
-#pragma unroll
-                    for (int s = 0; s < KSP; ++s) b[s] = bq[s % (PF ? KSP : 1)];
-                    jb = jbq;
-                    load_tile(bq, jbq, nt + NWV);
-                } else {
-                    load_tile(b, jb, nt);
-                }
-                V4 acc[NM];
-#pragma unroll
-                for (int m = 0; m < NM; ++m) acc[m] = V4{T(0), T(0), T(0), T(0)};
-                // A operands of the next k-step are read while this one's MFMAs run
-                T a0[NM], a1[NM];
-#pragma unroll
-                for (int m = 0; m < NM; ++m) a0[m] = Wl[(M0 + m) * 64 + lane];
-#pragma unroll
-                for (int s = 0; s < KSP; ++s) {
-                    T(&ac)[NM] = (s & 1) ? a1 : a0;
-                    T(&an)[NM] = (s & 1) ? a0 : a1;
-                    if (s + 1 < KSP) {
-#pragma unroll
-                        for (int m = 0; m < NM; ++m) an[m] = Wl[((s + 1) * MT + M0 + m) * 64 + lane];
-                    }
-#pragma unroll
-                    for (int m = 0; m < NM; ++m) acc[m] = Ops::mma(ac[m], b[s], acc[m]);
-                }
-                // scatter.  Colex rank of a target Ib = Jb ^ om: rank = rk[lo(Ib)] + rk[256 +
-                // 256 popc(lo(Ib)) + hi(Ib)]; a pair inside one byte leaves the other byte's
-                // term as it is for Jb.  Two row tiles at a time, every target rank is read
-                // first, then the adds -- an element that does not apply goes to the thread's
-                // spare slot; the sign goes into the value.
-                const int Jl = nt * 16 + col;
-                const bool live = Jl < nb;
-                const u32 jlo = jb & 255u, jbase = 256u + ((u32)__popc(jlo) << 8);
-                const u32 RL = rk[jlo], RH = rk[jbase + (jb >> 8)];
-                if constexpr (M0 == 0) {
-                    double dsum = 0.0;
-#pragma unroll
-                    for (int v = 0; v < 4; ++v)
-                        if (jb & row_info(0, v)) dsum += (double)acc[0][v];
-                    if (live) atomicAdd(&S[b0 + Jl - o0], dsum);
-                }
-                constexpr int F = M0 == 0 ? 1 : 0;  // first off-diagonal tile (local index)
-#pragma unroll
-                for (int q0 = F; q0 < NM; q0 += 2) {
-                    u32 tg[2][4];
-#pragma unroll
-                    for (int qq = 0; qq < 2; ++qq)
-#pragma unroll
-                        for (int v = 0; v < 4; ++v) {
-                            if (q0 + qq >= NM) continue;
-                            const int m = M0 + q0 + qq;  // row tile
-                            const u32 ri = row_info(m, v), om = ri & 0xffffu, x = jb & om;
-                            const u32 ib = jb ^ om;
-                            u32 rank;
-                            if (m <= 2) {
-                                rank = (u32)rk[ib & 255u] + RH;
-                            } else if (!CLS && m <= 4) {
-                                rank = RL + (u32)rk[jbase + (ib >> 8)];
-                            } else {
-                                const u32 l2 = ib & 255u;
-                                rank = (u32)rk[l2] + (u32)rk[256u + ((u32)__popc(l2) << 8) + (ib >> 8)];
-                            }
-                            acc[q0 + qq][v] =
-                                flip_sign(acc[q0 + qq][v], (u32)(__popc(jb & (ri >> 16)) & 1) << 31);
-                            tg[qq][v] = (live && __popc(x) == 1) ? rank - (u32)o0 : dmy;
-                        }
-#pragma unroll
-                    for (int qq = 0; qq < 2; ++qq)
-#pragma unroll
-                        for (int v = 0; v < 4; ++v)
-                            if (q0 + qq < NM) atomicAdd(&S[tg[qq][v]], (double)acc[q0 + qq][v]);
-                }
-            }
-        };
-        using I0 = std::integral_constant<int, 0>;
-        using I1 = std::integral_constant<int, 1>;
-        using I8 = std::integral_constant<int, 8>;
-        using I9 = std::integral_constant<int, 9>;
-        if constexpr (CLS) {
-            run(I0{}, I8{}, o0, NK);
-            run(I8{}, I1{}, c0, NC);
-        } else {
-            run(I0{}, I9{}, 0, NB);
-        }
-        __syncthreads();  // W is refilled by the next pass
+        Wl[e] = v;
     }
+    __syncthreads();
+
+    // the column tiles of [b0, b0 + nb), the first one at column tile ct0 of the target table, on the
+    // row tiles [M0, M0 + NM)
+    auto run = [&](auto m0_c, auto nm_c, int ct0, int b0, int nb) {
+        constexpr int M0 = decltype(m0_c)::value, NM = decltype(nm_c)::value;
+        const int ntiles = (nb + 15) >> 4;
+        for (int nt = wave; nt < ntiles; nt += NWV) {
+            const int Jl = nt * 16 + col;
+            const u32 Jb = (u32)(b0 + (Jl < nb ? Jl : nb - 1));
+            // B operands, all in flight at once; the other waves of the SIMD cover the latency
+            T b[KS];
+#pragma unroll
+            for (int s = 0; s < KS; ++s) b[s] = xt[(size_t)((jrow[g * KR + s] + Jb) * (u32)nvst + (u32)v0)];
+            uint2 tg[NM];
+            const uint2 *tp = tab + ((i64)(ct0 + nt) * MT + M0) * 64 + lane;
+            V4 acc[NM];
+#pragma unroll
+            for (int m = 0; m < NM; ++m) acc[m] = V4{T(0), T(0), T(0), T(0)};
+            // A operands PD products ahead (an LDS read takes about two FP64 MFMAs)
+            constexpr int PD = 6;
+            T a[PD];
+            auto A = [&](int i) { return Wl[((i / NM) * MT + M0 + i % NM) * 64 + lane]; };
+#pragma unroll
+            for (int i = 0; i < PD; ++i) a[i] = A(i < KS * NM ? i : 0);
+#pragma unroll
+            for (int i = 0; i < KS * NM; ++i) {
+                if (i == (KS > 6 ? KS - 6 : 0) * NM) {
+                    // target words, into the registers the first operands have left
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int m = 0; m < NM; ++m) tg[m] = tp[m * 64];
+                }
+                acc[i % NM] = Ops::mma(a[i % PD], b[i / NM], acc[i % NM]);
+                if (i + PD < KS * NM) a[i % PD] = A(i + PD);
+            }
+#pragma unroll
+            for (int m = 0; m < NM; ++m)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const u32 w = v < 2 ? tg[m].x : tg[m].y;
+                    const u32 at = v & 1 ? (w >> 16) & 0x7fffu : w & 0x7fffu;
+                    const u32 sg = (v & 1 ? w : w << 16) & 0x80000000u;
+                    atomicAdd(&S[at], flip_sign((double)acc[m][v], sg));
+                }
+        }
+    };
+    const int nctN = (NN + 15) >> 4;
+    run(std::integral_constant<int, 0>{}, std::integral_constant<int, MO>{}, MC && cls ? nctN : 0, o0, NK);
+    if constexpr (MC > 0)
+        run(std::integral_constant<int, MO>{}, std::integral_constant<int, MC>{}, cls ? 0 : nctN, c0, NC);
+    __syncthreads();
     for (int t = tid; t < NK; t += BD) {
         T &o = s1[(size_t)((Ia * NB + o0 + t) * nvst + v0)];
         o = (T)((double)o + S[t]);

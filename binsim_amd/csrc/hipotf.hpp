@@ -144,6 +144,7 @@ struct DevBasis {
     // scratch shared by sigma calls on this basis
     DevBuf xt, xtT, s1, s2T;
     DevBuf red;               // reduction partials
+    DevBuf abt64, abt32;      // target words of the matrix-core alpha-beta kernel (first use)
 };
 
 DevBasis *make_dev_basis(const HostBasis &hb);

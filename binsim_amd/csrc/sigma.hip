@@ -598,7 +598,9 @@ constexpr int ab_eptmax() { return (sizeof(T) == 8 && NVS >= 4) ? 4 : 8; }
 // launch, n <= 16) first.  The matrix-core kernel's default range is where it was measured
 // faster: at 12 orbitals its FP64 sigma is 8% slower (0.66 vs 0.61 ms), at 14 and 16 it is 1.4
 // and 1.6 times faster.
-static bool ab_mma_first(int pref, int n) { return pref == 5 || (pref == 0 && n >= 14 && n <= 16); }
+static bool ab_mma_first(int pref, int prec, int n) {
+    return pref == 5 || (pref == 0 && (prec == 0 || (n >= 14 && n <= 16)));
+}
 static int ab_kernel_pref(int prec) {
     const int p = tuning(prec).ab_kernel;
     return p >= 0 && p <= 5 ? p : 0;
@@ -777,10 +779,25 @@ static bool try_ab_src_r(DevHam *H, const T *xt, T *s1, int nvst, int v0, const 
     }
 }
 
-// the matrix-core kernel (ab_mma.hpp) for vector v0: up to 16 orbitals (16-bit strings), W and
-// the FP64 destination elements in LDS -- FP32 the whole row, FP64 one class of destinations
-// per launch (split by the top orbital); not in the deterministic mode (its LDS adds come from
-// all waves at once)
+// target table of the matrix-core kernel for one precision and form (mo, mc row tiles), built on
+// first use; the form is a function of the basis and the precision
+template <typename T>
+static const uint2 *ab_target_table(DevBasis *B, int n, int NN, int mo, int mc, hipStream_t st) {
+    DevBuf &b = sizeof(T) == 8 ? B->abt64 : B->abt32;
+    if (!b.p) {
+        const int NB = (int)B->pB->N, ct = (NN + 15) / 16 + (NB - NN + 15) / 16;
+        b.alloc((size_t)ct * (mo + mc) * 64 * sizeof(uint2));
+        hipLaunchKernelGGL(k_ab_targets<T>, dim3(ct, mo + mc), dim3(64), 0, st, B->pB->strs.as<u64>(), n, NB, NN, mo,
+                           mc, b.as<uint2>());
+        HIPOTF_CHECK(hipGetLastError());
+    }
+    return b.as<uint2>();
+}
+
+// the matrix-core kernel (ab_mma.hpp) for vector v0: W and the FP64 destination elements in LDS,
+// the whole row where both fit, else (FP64, 16 to 18 orbitals) one class of destinations per
+// launch, split by the top orbital; not in the deterministic mode (its LDS adds come from all
+// waves at once)
 template <typename T>
 static bool try_ab_mma(DevHam *H, const T *xt, T *s1, int nvst, int v0, const T *eri, hipStream_t st) {
     constexpr int prec = sizeof(T) == 4;
@@ -788,34 +805,53 @@ static bool try_ab_mma(DevHam *H, const T *xt, T *s1, int nvst, int v0, const T 
     DevBasis *B = H->basis;
     const DevSpin &A = *B->pA, &Bs = *B->pB;
     const int n = H->n;
-    constexpr bool CLS = sizeof(T) == 8;
-    constexpr int MT = 9, KSP = 17, NWV = CLS ? AB_MMA_NWV64 : AB_MMA_NWV32;
-    if (n > 16 || n < 1 || A.nsx + 1 > 4 * KSP || A.nsx + 1 > AB_SRC_CONN || Bs.N < 1) return false;
+    if (n > 18 || n < 1 || A.nsx + 1 > AB_SRC_CONN || Bs.N < 1 || Bs.N > 32000) return false;
     const i64 NB = Bs.N;
     if ((u64)A.N * (u64)NB * (u64)nvst >= (1ull << 32)) return false;  // 32-bit element offsets
     // class N: the beta strings without orbital n - 1, the first C(n - 1, k) in colex order
-    i64 NN = NB;
-    if (CLS) {
-        NN = 1;
-        for (int i = 0; i < Bs.k; ++i) NN = NN * (n - 1 - i) / (i + 1);
-        if (Bs.k > n - 1) NN = 0;
-    }
-    const size_t smem = ab_mma_lds<T, MT, KSP, NWV>(CLS ? std::max(NN, NB - NN) : NB);
-    if (smem > std::min<size_t>(lds_budget(), 160 * 1024)) return false;
+    i64 NN = 1;
+    for (int i = 0; i < Bs.k; ++i) NN = NN * (n - 1 - i) / (i + 1);
+    if (Bs.k > n - 1) NN = 0;
     const i64 nblocks = (A.N + 7) / 8 * 8;
     HIPOTF_REQUIRE(nblocks < (1ll << 31), "alpha-beta grid too large");
-    const T *dw = diag_w_table<T>(H, st);
-    const int nks = (A.nsx + 1 + 3) / 4;
-    auto kern = k_ab_mma<T, MT, KSP, NWV, CLS>;
-    HIPOTF_CHECK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
-    for (int cls = 0; cls < (CLS ? 2 : 1); ++cls) {
-        if (CLS && (cls ? NB - NN : NN) == 0) continue;
-        hipLaunchKernelGGL(kern, dim3((unsigned)nblocks), dim3(NWV * 64), smem, st, xt, s1, nvst, v0, A.sx.as<u32>(),
-                           Bs.strs.as<u64>(), eri, dw, ab_src_nw(n), n, A.N, (int)NB, A.nsx, nks, cls, (int)NN);
-        HIPOTF_CHECK(hipGetLastError());
-        ++ab_timing().mma_launches;
+    const size_t lds = std::min<size_t>(lds_budget(), 160 * 1024);
+    auto go = [&](auto moc, auto mcc, auto ksc, auto nwc, auto wpc) {
+        constexpr int MO = decltype(moc)::value, MC = decltype(mcc)::value, KS = decltype(ksc)::value;
+        constexpr int NWV = decltype(nwc)::value;
+        const i64 nn = MC ? NN : NB;
+        const size_t smem = ab_mma_lds<T, MO + MC, KS>(MC ? std::max(NN, NB - NN) : NB);
+        const int rows = MC ? n + (n - 1) * (n - 2) / 2 : n * (n + 1) / 2;
+        if (smem > lds || A.nsx + 1 > 4 * KS || rows > 16 * MO || n > 4 * MO || (MC && n - 1 > 16 * MC)) return false;
+        const uint2 *tab = ab_target_table<T>(B, n, (int)nn, MO, MC, st);
+        const T *dw = diag_w_table<T>(H, st);
+        auto kern = k_ab_mma<T, MO, MC, KS, NWV, decltype(wpc)::value>;
+        HIPOTF_CHECK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
+        for (int cls = 0; cls < (MC ? 2 : 1); ++cls) {
+            if (MC && (cls ? NB - NN : NN) == 0) continue;
+            hipLaunchKernelGGL(kern, dim3((unsigned)nblocks), dim3(NWV * 64), smem, st, xt, s1, nvst, v0,
+                               A.sx.as<u32>(), tab, eri, dw, ab_src_nw(n), n, A.N, (int)NB, A.nsx, cls, (int)nn);
+            HIPOTF_CHECK(hipGetLastError());
+            ++ab_timing().mma_launches;
+        }
+        return true;
+    };
+#define IC(x) std::integral_constant<int, x>{}
+    // row tiles and k-steps of the orbital count's half-filled spaces; eight waves where two
+    // workgroups share a CU
+    if (n <= 9) return go(IC(3), IC(0), IC(6), IC(8), IC(4));
+    if (n == 10) return go(IC(4), IC(0), IC(7), IC(8), IC(4));
+    if (n <= 12) return go(IC(5), IC(0), IC(10), IC(8), IC(4));
+    if (n == 13) return go(IC(6), IC(0), IC(11), IC(8), IC(4));
+    if (n == 14) return go(IC(7), IC(0), IC(13), IC(8), IC(4));
+    if (n == 15) return go(IC(8), IC(0), IC(15), IC(16), IC(4));
+    if (n == 16 && go(IC(9), IC(0), IC(17), IC(16), IC(4))) return true;
+    if constexpr (sizeof(T) == 8) {
+        if (n == 16) return go(IC(8), IC(1), IC(17), IC(16), IC(4));
+        if (n == 17) return go(IC(9), IC(1), IC(17), IC(8), IC(2));
+        if (n == 18) return go(IC(10), IC(2), IC(17), IC(8), IC(2));
     }
-    return true;
+#undef IC
+    return false;
 }
 
 // the class-split FP32 kernel for vectors v0, v0 + 1 (ab_cls.hpp): 256-entry integral rows
@@ -916,7 +952,7 @@ static void launch_ab(DevHam *H, const T *xt, T *s1, int nv, const T *eri, hipSt
     const int pref = ab_kernel_pref(sizeof(T) == 4);
     if (pref <= 1 || pref >= 4) {
         while (v0 < nv) {
-            if (ab_mma_first(pref, H->n) && try_ab_mma<T>(H, xt, s1, nv, v0, eri, st)) {
+            if (ab_mma_first(pref, sizeof(T) == 4, H->n) && try_ab_mma<T>(H, xt, s1, nv, v0, eri, st)) {
                 v0 += 1;
                 continue;
             }
