@@ -330,6 +330,10 @@ DevHam *make_dev_ham(DevBasis *b, int n, const std::vector<double> &h, const std
     // the default row blocks now, so that the first sigma does not pay for them
     for (int prec = 0; prec < 2; ++prec) {
         const int rb = tuning(prec).rs_block;
+        if (prec == 0 && rb == MB_RB && tuning(prec).rs_passes == 0) {
+            mfma_blocks(*H->ptA);
+            mfma_blocks(*H->ptB);
+        }
         if (rb == 4 || rb == 8 || rb == 16) {
             row_blocks(*H->ptA, rb);
             row_blocks(*H->ptB, rb);

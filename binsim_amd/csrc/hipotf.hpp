@@ -168,6 +168,18 @@ struct RowBlockTable {
     DevBuf c64, c32;          // double / float [entries][rb]
 };
 
+// the row blocks of MB_RB strings in MFMA-operand order for the FP64 matrix-core row SpMM
+// (k_mbspmm): each block's sources in nr source ranges, each range padded to whole groups of
+// MB_GRP batches of 4 sources (coefficient 0, a valid source)
+constexpr int MB_RB = 8, MB_GRP = 4;
+struct MfmaBlockTable {
+    int nr = 1;               // source ranges: passes of the kernel
+    i64 nblk = 0, batches = 0;
+    DevBuf P;                 // int32[nblk][nr + 1]: first batch of each range, end
+    DevBuf J;                 // int32[batches][4]: sources
+    DevBuf c64;               // double[batches][4 sources][4][2]: coefficients of rows i and i + 4
+};
+
 struct SameSpinTable {
     i64 N = 0;
     int L = 0;                // 1 + nsx + ndx entries per dest string, ascending source index
@@ -180,6 +192,7 @@ struct SameSpinTable {
     std::vector<double> hC;   // built on the host (row blocks are then built from them)
     bool dev_built = false;   // built on the device (tables.hip): row blocks too
     std::unique_ptr<RowBlockTable> blocks[3];  // rb = 4, 8, 16
+    std::unique_ptr<MfmaBlockTable> mfma;
 };
 
 // row-block table of T for rb in {4, 8, 16}, built (and uploaded) on first use
@@ -189,6 +202,8 @@ const RowBlockTable &row_blocks(SameSpinTable &T, int rb);
 struct DevSpin;
 bool build_same_spin_dev(SameSpinTable &T, const DevSpin &S, const DevBuf &h64, const DevBuf &eri64, int n);
 void row_blocks_dev(SameSpinTable &T, RowBlockTable &R, int rb);
+// matrix-core row-SpMM table of T, built on first use; NULL for tables built on the host
+const MfmaBlockTable *mfma_blocks(SameSpinTable &T);
 void build_jab_dev(DevBuf &jab, const DevSpin &A, int n, const DevBuf &eri64);
 void build_sx_dev(DevSpin &D);  // single-excitation table of one spin (n <= 32)
 

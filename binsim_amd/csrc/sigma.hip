@@ -199,6 +199,96 @@ __global__ __launch_bounds__(256) void k_rbspmm(const T *__restrict__ X, T *__re
 }
 
 // ---------------------------------------------------------------------------------------
+// K2/K3 on the matrix cores (FP64, the default): the row blocks of k_rbspmm with 8 strings, one
+// wave = one block x 32 NP columns.  Per batch of 4 of the block's sources the 8 x 4 coefficients
+// times the 4 source slices as 4x4x4 MFMAs (two row quads x 2 NP groups of 16 columns; each lane
+// loads 2 consecutive columns, 16 bytes).  The coefficients come as a vector load in operand order
+// and, like the slices and the source indices, MB_GRP batches ahead in registers.
+//
+// Why: k_rbspmm's coefficients are scalar loads, 64 bytes per 16 FMAs, which cannot be held ahead
+// in the SGPRs: its FP64 VALU was 63% busy, and one wave's chain of waits set the pace in small
+// spaces.  16-row tiles (16x16x4 MFMAs) would need 4.8 times the useful products instead of 3.4.
+// Operand layout (measured): lane l holds A[l % 4][l / 16], B[l / 16][l % 16], D[l / 16][l % 16].
+// Measured, FP64, per spin: 16 orbitals / 8 electrons 28.5 -> 24.5 ms, 12 orbitals / 6 electrons
+// 157 -> 39 us.  Bound now by the gathered bytes (480 GB per spin at 16 orbitals, 19.6 TB/s into the
+// CUs; the matrix cores are 50% busy).  Measured and not faster: 96 or 256 columns per wave, 2
+// batches ahead, and the slices staged in LDS for 64 strings (147 GB staged instead of 480
+// gathered, but 49 ms with scalar coefficients and 76 ms on the matrix cores: too few loads in
+// flight beside the LDS buffers).
+// ---------------------------------------------------------------------------------------
+constexpr size_t MB_SLACK = 1024;  // bytes after the source vector that k_mbspmm may read
+template <int NP>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NP == 4 ? 3 : 4)))
+void k_mbspmm(const double *__restrict__ X, double *__restrict__ Y,
+                                                const int32_t *__restrict__ J, const int32_t *__restrict__ P,
+                                                const double2 *__restrict__ C, i64 nrows, i64 ncols, i64 nblk,
+                                                i64 nwork, i64 per_xcd, int nr, int r, int accumulate) {
+    typedef double V2 __attribute__((ext_vector_type(2), aligned(8)));
+    const int lane = threadIdx.x & 63, k = lane >> 4, j = lane & 15;
+    // contiguous ranges of wave items per XCD (tile-major: all blocks of a column tile, then the next)
+    const i64 w = (i64)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if ((blockIdx.x >> 3) * 4 + (threadIdx.x >> 6) >= per_xcd || w >= nwork) return;
+    const i64 tile = w / nblk, blk = w - tile * nblk;
+    // (lanes past the last column read into the next row, or the slack after the last one)
+    const i64 col0 = tile * (32 * NP) + 2 * j;
+    const char *Xc = reinterpret_cast<const char *>(X + (col0 < ncols ? col0 : 0));
+    int b = P[blk * (nr + 1) + r];
+    const int e = P[blk * (nr + 1) + r + 1];
+    double acc[2][2 * NP];
+#pragma unroll
+    for (int q = 0; q < 2 * NP; ++q) acc[0][q] = acc[1][q] = 0.0;
+    const u32 jo = (u32)k * 4, co = (u32)(k * 4 + (lane & 3)) * 16, rowb = (u32)ncols * 8;
+    auto src = [&](int at) { return *reinterpret_cast<const u32 *>(reinterpret_cast<const char *>(J + (i64)at * 4) + jo); };
+    u32 jn[MB_GRP];
+    double2 a[MB_GRP];
+    V2 x[MB_GRP][NP];
+    auto fetch = [&](int q, int at) {  // batch `at` into slot q, then the indices MB_GRP further on
+        a[q] = *reinterpret_cast<const double2 *>(reinterpret_cast<const char *>(C + (i64)at * 16) + co);
+        const char *xr = Xc + (u64)jn[q] * rowb;
+#pragma unroll
+        for (int p = 0; p < NP; ++p) x[q][p] = *reinterpret_cast<const V2 *>(xr + 256 * p);
+        jn[q] = src(at + MB_GRP);
+    };
+    if (b < e) {
+#pragma unroll
+        for (int q = 0; q < MB_GRP; ++q) jn[q] = src(b + q);
+#pragma unroll
+        for (int q = 0; q < MB_GRP; ++q) fetch(q, b + q);
+    }
+    for (; b < e; b += MB_GRP) {
+#pragma unroll
+        for (int q = 0; q < MB_GRP; ++q) {
+            const double2 av = a[q];
+            V2 xv[NP];
+#pragma unroll
+            for (int p = 0; p < NP; ++p) xv[p] = x[q][p];
+#pragma unroll
+            for (int p = 0; p < NP; ++p)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    acc[0][2 * p + h] = __builtin_amdgcn_mfma_f64_4x4x4f64(av.x, xv[p][h], acc[0][2 * p + h], 0, 0, 0);
+                    acc[1][2 * p + h] = __builtin_amdgcn_mfma_f64_4x4x4f64(av.y, xv[p][h], acc[1][2 * p + h], 0, 0, 0);
+                }
+            __builtin_amdgcn_sched_barrier(0);  // (the scheduler would sink the loads to their uses)
+            fetch(q, b + MB_GRP + q);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const i64 row = blk * MB_RB + 4 * h + k;
+        if (row >= nrows) continue;
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+            const i64 col = col0 + 32 * p;
+            double *y = Y + row * ncols + col;
+            if (col < ncols) y[0] = accumulate ? y[0] + acc[h][2 * p] : acc[h][2 * p];
+            if (col + 1 < ncols) y[1] = accumulate ? y[1] + acc[h][2 * p + 1] : acc[h][2 * p + 1];
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------------------
 // K4: alpha-beta part.  Workgroup = destination alpha row Ia.  For each alpha connection
 // (its nsxA single excitations Ja = Ia - p + q, then Ia itself) the source row x~[Ja, :] is
 // staged in LDS (in chunks if it does not fit) together with the integral row
@@ -538,12 +628,38 @@ static int rs_npass(i64 nrows, int tile_cols) {
     return p;
 }
 
+template <int NP>
+static void launch_mbspmm_n(const double *X, double *Y, const MfmaBlockTable &M, i64 nrows, i64 ncols, hipStream_t st) {
+    const i64 ntiles = (ncols + 32 * NP - 1) / (32 * NP), nwork = ntiles * M.nblk, per_xcd = (nwork + 7) / 8;
+    const i64 nwg = (per_xcd + 3) / 4 * 8;
+    HIPOTF_REQUIRE(nwg < (1ll << 31), "row-block SpMM grid too large");
+    for (int r = 0; r < M.nr; ++r)
+        hipLaunchKernelGGL(k_mbspmm<NP>, dim3((unsigned)nwg), dim3(256), 0, st, X, Y, M.J.as<int32_t>(),
+                           M.P.as<int32_t>(), M.c64.as<double2>(), nrows, ncols, M.nblk, nwork, per_xcd, M.nr, r,
+                           r > 0 ? 1 : 0);
+    HIPOTF_CHECK(hipGetLastError());
+}
+
+// 128 columns per wave (the fewest coefficient and index loads per product), fewer where that leaves
+// the chip short of waves.  FP64 sigma with 128 / 64 / 32 columns: 8 orbitals / 4 + 4 electrons 24.9 /
+// 23.2 / 22.8 us, 10 / 5 + 5 45 / 40 / 36 us, 12 / 6 + 6 207 / 216 / 240 us, 16 / 8 + 8 109 / 118 / 136 ms
+static void launch_mbspmm(const double *X, double *Y, const MfmaBlockTable &M, i64 nrows, i64 ncols, hipStream_t st) {
+    auto waves = [&](int np) { return (ncols + 32 * np - 1) / (32 * np) * M.nblk; };
+    const int np = waves(4) >= 768 ? 4 : (waves(2) >= 384 ? 2 : 1);
+    if (np == 4) launch_mbspmm_n<4>(X, Y, M, nrows, ncols, st);
+    else if (np == 2) launch_mbspmm_n<2>(X, Y, M, nrows, ncols, st);
+    else launch_mbspmm_n<1>(X, Y, M, nrows, ncols, st);
+}
+
 template <typename T>
 static void launch_rowspmm(const T *X, T *Y, SameSpinTable &tab, const T *C, i64 nrows,
                            i64 ncols, hipStream_t st) {
     if (nrows == 0 || ncols == 0) return;
     HIPOTF_REQUIRE(nrows == tab.N, "internal: same-spin table does not match the row count");
     const int rb = tuning(sizeof(T) == 4).rs_block;
+    if constexpr (sizeof(T) == 8)
+        if (rb == MB_RB && tuning(0).rs_passes == 0)  // the defaults
+            if (const MfmaBlockTable *M = mfma_blocks(tab)) return launch_mbspmm(X, Y, *M, nrows, ncols, st);
     if (rb == 4 || rb == 8 || rb == 16) {
         const int npass = rs_npass<T>(nrows, 256 * rs_cpl<T>(ncols));
         const RowBlockTable &rt = row_blocks(tab, rb);
@@ -997,8 +1113,8 @@ static void sigma_group(DevHam *H, const SrcPack &src, const DstPack &dst, hipSt
         s1 = reinterpret_cast<T *>(work + 2 * stride);
         s2T = reinterpret_cast<T *>(work + 3 * stride);
     } else {
-        B->xt.ensure(bytes);
-        B->xtT.ensure(bytes);
+        B->xt.ensure(bytes + MB_SLACK);
+        B->xtT.ensure(bytes + MB_SLACK);
         B->s1.ensure(bytes);
         B->s2T.ensure(bytes);
         xt = B->xt.as<T>(), xtT = B->xtT.as<T>(), s1 = B->s1.as<T>(), s2T = B->s2T.as<T>();

@@ -340,6 +340,80 @@ void row_blocks_dev(SameSpinTable &T, RowBlockTable &R, int rb) {
     HIPOTF_CHECK(hipDeviceSynchronize());
 }
 
+// ---------------------------------------------------------------------------------------
+// matrix-core row-SpMM table (MfmaBlockTable) from the blocks of MB_RB rows, one workgroup per
+// block; FILL = false: its batches
+// ---------------------------------------------------------------------------------------
+template <bool FILL>
+__global__ __launch_bounds__(256) void k_mb(const int32_t *__restrict__ J, const int32_t *__restrict__ P,
+                                            const double *__restrict__ C, i64 N, int nr, int32_t *__restrict__ cnt,
+                                            const int32_t *__restrict__ first, int32_t *__restrict__ Pm,
+                                            int32_t *__restrict__ Jm, double *__restrict__ cm) {
+    const i64 b = blockIdx.x;
+    const int32_t e0 = P[b * (SS_RANGES + 1)];
+    int at = FILL ? first[b] : 0;
+    for (int r = 0; r < nr; ++r) {
+        const int32_t s = P[b * (SS_RANGES + 1) + r * (SS_RANGES / nr)], e = P[b * (SS_RANGES + 1) + (r + 1) * (SS_RANGES / nr)];
+        const int nb = (e - s + 4 * MB_GRP - 1) / (4 * MB_GRP) * MB_GRP;
+        if (FILL) {
+            if (threadIdx.x == 0) Pm[b * (nr + 1) + r] = at;
+            for (int i = threadIdx.x; i < nb * 4; i += blockDim.x) {
+                const bool in = s + i < e;
+                const i64 d = (i64)at * 4 + i, src = in ? s + i : (e > s ? e - 1 : e0);
+                Jm[d] = J[src];
+                for (int q = 0; q < MB_RB; ++q) cm[(d * 4 + q % 4) * 2 + q / 4] = in ? C[src * MB_RB + q] : 0.0;
+            }
+        }
+        at += nb;
+    }
+    if (threadIdx.x == 0) {
+        if (FILL) Pm[b * (nr + 1) + nr] = at;
+        else cnt[b] = at;
+    }
+}
+
+const MfmaBlockTable *mfma_blocks(SameSpinTable &T) {
+    if (T.mfma) return T.mfma.get();
+    if (!T.dev_built || T.N < 1) return nullptr;
+    const RowBlockTable &R = row_blocks(T, MB_RB);
+    auto M = std::make_unique<MfmaBlockTable>();
+    // as many source ranges as keep the gathered slice of 128 columns about within an XCD's 4 MB L2
+    // (FP64 sigma, 16 orbitals / 8 + 8 electrons, slice 13.2 MB: 146 / 115 / 109 / 115 ms with 1 / 2 /
+    // 4 / 8 ranges; 18 orbitals / 5 + 5, 8.8 MB: 60.7 / 52.5 / 53.0 / 56.0 ms)
+    while (M->nr < SS_RANGES && (double)T.N * 128 * 8 > 4.5e6 * M->nr) M->nr *= 2;
+    const i64 nblk = R.nblk;
+    M->nblk = nblk;
+    DevBuf cnt, first;
+    cnt.alloc((size_t)nblk * 4);
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(256), 0, 0, R.J.as<int32_t>(), R.P.as<int32_t>(),
+                           R.c64.as<double>(), T.N, M->nr, cnt.as<int32_t>(), first.as<int32_t>(), M->P.as<int32_t>(),
+                           M->J.as<int32_t>(), M->c64.as<double>());
+        HIPOTF_CHECK(hipGetLastError());
+    };
+    go(k_mb<false>);
+    std::vector<int32_t> h(nblk), f(nblk);
+    HIPOTF_CHECK(hipMemcpy(h.data(), cnt.p, (size_t)nblk * 4, hipMemcpyDeviceToHost));
+    i64 t = 0;
+    for (i64 b = 0; b < nblk; ++b) {
+        f[b] = (int32_t)t;
+        t += h[b];
+        HIPOTF_REQUIRE(t < (1ll << 31) - 64, "matrix-core row-block table too large for 32-bit offsets");
+    }
+    M->batches = t;
+    first.upload(f);
+    const size_t E = (size_t)t + 4 * MB_GRP;  // (the kernel reads up to 3 groups past a range's end)
+    M->P.alloc((size_t)nblk * (M->nr + 1) * 4);
+    M->J.alloc(E * 16);
+    M->c64.alloc(E * 4 * MB_RB * sizeof(double));
+    HIPOTF_CHECK(hipMemset((char *)M->J.p + (size_t)t * 16, 0, 4 * MB_GRP * 16));
+    HIPOTF_CHECK(hipMemset((char *)M->c64.p + (size_t)t * 256, 0, 4 * MB_GRP * 256));
+    go(k_mb<true>);
+    HIPOTF_CHECK(hipDeviceSynchronize());
+    T.mfma = std::move(M);
+    return T.mfma.get();
+}
+
 void build_jab_dev(DevBuf &jab, const DevSpin &A, int n, const DevBuf &eri64) {
     const i64 tot = A.N * n;
     jab.alloc((size_t)tot * sizeof(double));
