@@ -302,7 +302,7 @@ DavidsonOut davidson(DevHam *H, int nroots, int mode, int block, double tol, dou
                 out.sigma64++;
             }
         } else {
-            sigma(H, count, (const double *const *)&V[first], &AV[first], phase, st, nv_sigma);
+            sigma(H, count, (const double *const *)&V[first], &AV[first], phase, st, nv_sigma, false);
             if (phase == 1) out.sigma32 += count;
             else out.sigma64 += count;
         }

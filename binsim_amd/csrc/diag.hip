@@ -143,28 +143,6 @@ __global__ __launch_bounds__(256) void k_scale_inv(double *__restrict__ y, const
     stream_for(n, [&](i64 i) { y[i] *= s; });
 }
 
-// out[j] = <V_j, a> for j < M (M <= 8): each block accumulates M partials
-template <int M>
-__global__ __launch_bounds__(256) void k_multidot(VecPack V, const double *__restrict__ a,
-                                                  double *__restrict__ partial, int ldp, i64 n) {
-    double acc[M];
-#pragma unroll
-    for (int j = 0; j < M; ++j) acc[j] = 0.0;
-    for (i64 i = (i64)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (i64)gridDim.x * blockDim.x) {
-        const double av = a[i];
-        double v[M];
-#pragma unroll
-        for (int j = 0; j < M; ++j) v[j] = V.v[j][i];
-#pragma unroll
-        for (int j = 0; j < M; ++j) acc[j] += v[j] * av;
-    }
-#pragma unroll
-    for (int j = 0; j < M; ++j) {
-        const double t = block_sum_d(acc[j]);
-        if (threadIdx.x == 0) partial[j * ldp + blockIdx.x] = t;
-    }
-}
-
 struct DiagScratch {
     DevBuf partial, scal;
     DiagScratch() {
@@ -271,31 +249,12 @@ double dot(i64 N, const double *a, const double *b, hipStream_t st) {
     return d2h(d, st);
 }
 
+void block_dots(i64 N, int na, const double *const *A, int nbv, const double *const *B, double *G, hipStream_t st);
 // out[j] = <V_j, a>, j < dim, written to host memory
-void multidot(i64 N, int dim, const double *const *V, const double *a, double *out_host,
-              hipStream_t st) {
-    auto &S = scratch();
-    const int nb = nblk(N);
-    std::vector<double> res(dim);
-    for (int j0 = 0; j0 < dim; j0 += 8) {
-        const int m = std::min(8, dim - j0);
-        VecPack P{};
-        pack(P, V + j0, nullptr, m);
-        dispatch_m8(m, [&](auto mc) {
-            hipLaunchKernelGGL(k_multidot<decltype(mc)::value>, dim3(nb), dim3(256), 0, st, P, a,
-                               S.partial.as<double>(), 2048, N);
-        });
-        HIPOTF_CHECK(hipGetLastError());
-        for (int j = 0; j < m; ++j) {
-            hipLaunchKernelGGL(k_reduce, dim3(1), dim3(256), 0, st, S.partial.as<double>() + j * 2048,
-                               N > 0 ? nb : 0, S.scal.as<double>() + 16 + j, 0);
-            HIPOTF_CHECK(hipGetLastError());
-        }
-        HIPOTF_CHECK(hipMemcpyAsync(res.data() + j0, S.scal.as<double>() + 16, m * sizeof(double),
-                                    hipMemcpyDeviceToHost, st));
-        HIPOTF_CHECK(hipStreamSynchronize(st));
-    }
-    std::copy(res.begin(), res.end(), out_host);
+void multidot(i64 N, int dim, const double *const *V, const double *a, double *out_host, hipStream_t st) {
+    HIPOTF_REQUIRE(dim >= 0 && dim <= DMAX, "subspace dimension must be in [0, 64]");
+    for (int j = 0; j < dim; ++j) HIPOTF_REQUIRE(V[j] != nullptr, "NULL subspace vector");
+    block_dots(N, dim, V, 1, &a, out_host, st);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -304,6 +263,7 @@ void multidot(i64 N, int dim, const double *const *V, const double *a, double *o
 // instead of once per (root, vector) pair; reductions stay two-stage and deterministic.
 // ------------------------------------------------------------------------------------------
 constexpr int BK = 8;  // outputs per launch
+constexpr int DOT_BLOCKS = 1024;  // workgroups of the dot products
 
 struct Ptr64 { const double *p[DMAX]; };
 struct Out8 { double *p[BK]; };
@@ -386,35 +346,89 @@ __global__ __launch_bounds__(256) void k_block_subtract(Ptr64 V, int m, const do
     }
 }
 
-// partial[(a * NB + b) * nblk + blk] = block sums of A_a . B_b   (a < NA, b < NB, NA * NB <= 32);
-// every pointer is loaded (the host repeats a vector to fill a partial group)
-constexpr int DOT_ACC = 32;
-template <int NA, int NB>
-__global__ __launch_bounds__(256) void k_block_dots(Ptr64 A, Ptr64 B, double *__restrict__ partial, i64 n) {
-    static_assert(NA * NB <= DOT_ACC, "accumulator budget");
-    double acc[NA][NB];
+// Sums of A_a . B_b over the elements, for all a < na <= DMAX and NB vectors B in one pass: a thread
+// holds DOT_EL elements of every B and streams the A through; per a, the wave adds its NB sums
+// up with VALU moves (wave_sum4) into its own row of LDS, so no accumulator lives across vectors.
+// (One launch per 8 x 4 sums re-read the B and added each sum up over the block with two barriers:
+// 8 launches of 55 us at 854,000 elements, 64 x 4 sums, bound by those reductions.)  HBM bound:
+// 8 N (na + NB) bytes.
+// partial[(a * NB + b) * gridDim.x + block]
+constexpr int DOT_THREADS = 256;
+template <int NB>
+constexpr int dot_el() { return NB <= 4 ? 8 : 4; }
+
+// sums over the wave of four values: lanes 12..15 end with those of a[0..3]
+__device__ __forceinline__ double dot_wave_sum4(const double (&a)[4]) {
+    const int lane = threadIdx.x & 63;
+    auto dpp = [](double v, auto ctrl) {
+        constexpr int CT = decltype(ctrl)::value;
+        const long long b = __double_as_longlong(v);
+        const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CT, 0xf, 0xf, false);
+        const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CT, 0xf, 0xf, false);
+        return __longlong_as_double(((long long)hi << 32) | (u32)lo);
+    };
+    const bool o1 = lane & 1, o2 = lane & 2;
+    const double u = (o1 ? a[1] : a[0]) + dpp(o1 ? a[0] : a[1], std::integral_constant<int, 0xb1>{});
+    const double v = (o1 ? a[3] : a[2]) + dpp(o1 ? a[2] : a[3], std::integral_constant<int, 0xb1>{});
+    double w = (o2 ? v : u) + dpp(o2 ? u : v, std::integral_constant<int, 0x4e>{});
+    w += dpp(w, std::integral_constant<int, 0x114>{});
+    w += dpp(w, std::integral_constant<int, 0x118>{});
+    w += __shfl_xor(w, 16, 64);
+    w += __shfl_xor(w, 32, 64);
+    return w;
+}
+
+template <int NB>
+__global__ __launch_bounds__(DOT_THREADS) void k_dots(Ptr64 A, int na, Out8 B, double *__restrict__ partial, i64 n) {
+    constexpr int EL = dot_el<NB>(), NQ = (NB + 3) / 4, W = DOT_THREADS / 64;
+    extern __shared__ double sums[];  // [W][na * NB]
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, no = na * NB;
+    for (int i = tid; i < W * no; i += DOT_THREADS) sums[i] = 0.0;
+    __syncthreads();
+    double *mine = sums + wave * no;
+    for (i64 base = (i64)blockIdx.x * DOT_THREADS * EL + tid; base - tid < n; base += (i64)gridDim.x * DOT_THREADS * EL) {
+        double bv[NB][EL];
 #pragma unroll
-    for (int a = 0; a < NA; ++a)
+        for (int b = 0; b < NB; ++b)
 #pragma unroll
-        for (int b = 0; b < NB; ++b) acc[a][b] = 0.0;
-    for (i64 i = (i64)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (i64)gridDim.x * blockDim.x) {
-        double bv[NB], av[NA];
+            for (int q = 0; q < EL; ++q) {
+                const i64 i = base + q * DOT_THREADS;
+                bv[b][q] = i < n ? B.p[b][i] : 0.0;
+            }
+        double av[EL], nx[EL];
+        auto load = [&](double (&d)[EL], int a) {
+            const double *p = A.p[a];
 #pragma unroll
-        for (int b = 0; b < NB; ++b) bv[b] = B.p[b][i];
+            for (int q = 0; q < EL; ++q) {
+                const i64 i = base + q * DOT_THREADS;
+                d[q] = i < n ? p[i] : 0.0;
+            }
+        };
+        load(av, 0);
+        for (int a = 0; a < na; ++a) {
+            load(nx, a + 1 < na ? a + 1 : a);
 #pragma unroll
-        for (int a = 0; a < NA; ++a) av[a] = A.p[a][i];
+            for (int g = 0; g < NQ; ++g) {
+                double s[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-        for (int a = 0; a < NA; ++a)
+                for (int b = 0; b < 4; ++b)
+                    if (g * 4 + b < NB)
 #pragma unroll
-            for (int b = 0; b < NB; ++b) acc[a][b] += av[a] * bv[b];
-    }
+                        for (int q = 0; q < EL; ++q) s[b] += av[q] * bv[g * 4 + b < NB ? g * 4 + b : 0][q];
+                const double t = dot_wave_sum4(s);
+                const int b = g * 4 + lane - 12;
+                if (lane >= 12 && lane < 16 && b < NB) mine[a * NB + b] += t;
+            }
 #pragma unroll
-    for (int a = 0; a < NA; ++a)
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            const double t = block_sum_d(acc[a][b]);
-            if (threadIdx.x == 0) partial[(a * NB + b) * gridDim.x + blockIdx.x] = t;
+            for (int q = 0; q < EL; ++q) av[q] = nx[q];
         }
+    }
+    __syncthreads();
+    for (int o = tid; o < no; o += DOT_THREADS) {
+        double t = 0.0;
+        for (int w = 0; w < W; ++w) t += sums[w * no + o];
+        partial[(i64)o * gridDim.x + blockIdx.x] = t;
+    }
 }
 
 // out[o] = sum of partial[o * nparts .. + nparts) for o = blockIdx.x
@@ -429,7 +443,7 @@ __global__ __launch_bounds__(256) void k_multi_reduce(const double *__restrict__
 struct BlockScratch {
     DevBuf partial, coef, small;
     BlockScratch() {
-        partial.alloc((size_t)DOT_ACC * 2048 * sizeof(double));
+        partial.alloc((size_t)DMAX * BK * DOT_BLOCKS * sizeof(double));
         coef.alloc((size_t)DMAX * DMAX * sizeof(double));
         small.alloc((size_t)4 * DMAX * BK * sizeof(double));
     }
@@ -498,15 +512,13 @@ void block_combine(i64 N, int m, int k, const double *C, const double *w, const 
 // In place X_r <- sum_j C[j][r] X_j for r < keep <= m <= DMAX: the subspace restart without a
 // second copy of the kept vectors.  Each thread loads all m elements of its index before it
 // writes any, and no two threads share an index, so reading and writing the same vectors is
-// safe.  C sits in LDS (uniform reads, broadcast).  M = m rounded up to a multiple of 8.
+// safe.  C is [keep][M], read by scalar loads (from LDS, 64 broadcast reads per output and thread
+// were the bound: 669 us at 854,000 elements, 64 -> 32 vectors).  M = m rounded up to a multiple of 8.
 struct PtrMut64 { double *p[DMAX]; };
 
 template <int M>
 __global__ __launch_bounds__(256) void k_rotate_inplace(PtrMut64 X, int m, int keep, const double *__restrict__ C,
                                                         i64 n) {
-    __shared__ double cs[M * DMAX];
-    for (int t = threadIdx.x; t < m * keep; t += blockDim.x) cs[(t / keep) * DMAX + t % keep] = C[t];
-    __syncthreads();
     for (i64 i = (i64)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (i64)gridDim.x * blockDim.x) {
         double x[M];
 #pragma unroll
@@ -514,8 +526,7 @@ __global__ __launch_bounds__(256) void k_rotate_inplace(PtrMut64 X, int m, int k
         for (int r = 0; r < keep; ++r) {
             double acc = 0.0;
 #pragma unroll
-            for (int j = 0; j < M; ++j)
-                if (j < m) acc += cs[j * DMAX + r] * x[j];
+            for (int j = 0; j < M; ++j) acc += C[r * M + j] * x[j];
             X.p[r][i] = acc;
         }
     }
@@ -525,10 +536,13 @@ __global__ __launch_bounds__(256) void k_rotate_inplace(PtrMut64 X, int m, int k
 void rotate_inplace(i64 N, int m, int keep, const double *C, double *const *X, hipStream_t st) {
     HIPOTF_REQUIRE(m >= 1 && m <= DMAX && keep >= 1 && keep <= m, "rotate_inplace: bad sizes");
     auto &S = bscratch();
-    HIPOTF_CHECK(hipMemcpyAsync(S.coef.p, C, (size_t)m * keep * sizeof(double), hipMemcpyHostToDevice, st));
     PtrMut64 P{};
     for (int j = 0; j < m; ++j) P.p[j] = X[j];
     const int mm = (m + 7) / 8 * 8;
+    std::vector<double> Ct((size_t)keep * mm, 0.0);
+    for (int j = 0; j < m; ++j)
+        for (int r = 0; r < keep; ++r) Ct[(size_t)r * mm + j] = C[(size_t)j * keep + r];
+    HIPOTF_CHECK(hipMemcpyAsync(S.coef.p, Ct.data(), Ct.size() * sizeof(double), hipMemcpyHostToDevice, st));
     auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, dim3(nblk_block(N)), dim3(256), 0, st, P, m, keep, S.coef.as<double>(), N);
     };
@@ -571,48 +585,28 @@ void block_dots(i64 N, int na, const double *const *A, int nbv, const double *co
     HIPOTF_REQUIRE(na >= 0 && na <= DMAX && nbv >= 1 && nbv <= BK, "block_dots: bad sizes");
     if (na == 0) return;
     auto &S = bscratch();
-    const int nb = nblk_block(N);
-    Ptr64 PB{};
-    for (int b = 0; b < nbv; ++b) PB.p[b] = B[b];
-    // A vectors per launch: a power of two with NA * nbv <= 32 (at most 16); the groups are
-    // balanced, and a group smaller than its NA repeats its first vector (results dropped)
-    int cap = 16;
-    while (cap * nbv > DOT_ACC) cap /= 2;
-    const int ngroups = (na + cap - 1) / cap, per = (na + ngroups - 1) / ngroups;
-    int NA = 1;
-    while (NA < per) NA *= 2;
-    HIPOTF_REQUIRE(NA * nbv <= DOT_ACC, "block_dots: group too large");
-    std::vector<double> h((size_t)DOT_ACC);
-    for (int a0 = 0; a0 < na; a0 += per) {
-        const int ka = std::min(per, na - a0);
-        Ptr64 PA{};
-        for (int a = 0; a < NA; ++a) PA.p[a] = A[a0 + (a < ka ? a : 0)];
-        double *part = S.partial.as<double>();
+    Ptr64 PA{};
+    Out8 PB{};
+    for (int a = 0; a < na; ++a) PA.p[a] = A[a];
+    for (int b = 0; b < nbv; ++b) PB.p[b] = const_cast<double *>(B[b]);
+    const int no = na * nbv;
+    std::vector<double> h((size_t)no, 0.0);
+    if (N > 0) {
+        int nb = 1;
         dispatch_m8(nbv, [&](auto bc) {
             constexpr int NB = decltype(bc)::value;
-            switch (NA) {
-            case 1: hipLaunchKernelGGL((k_block_dots<1, NB>), dim3(nb), dim3(256), 0, st, PA, PB, part, N); break;
-            case 2: hipLaunchKernelGGL((k_block_dots<2, NB>), dim3(nb), dim3(256), 0, st, PA, PB, part, N); break;
-            case 4: hipLaunchKernelGGL((k_block_dots<4, (NB <= 8 ? NB : 8)>), dim3(nb), dim3(256), 0, st, PA, PB,
-                                       part, N); break;
-            case 8:
-                if constexpr (NB <= 4)
-                    hipLaunchKernelGGL((k_block_dots<8, NB>), dim3(nb), dim3(256), 0, st, PA, PB, part, N);
-                break;
-            default:
-                if constexpr (NB <= 2)
-                    hipLaunchKernelGGL((k_block_dots<16, NB>), dim3(nb), dim3(256), 0, st, PA, PB, part, N);
-                break;
-            }
+            const i64 per = (i64)DOT_THREADS * dot_el<NB>();
+            nb = (int)std::max<i64>(1, std::min<i64>((N + per - 1) / per, DOT_BLOCKS));
+            hipLaunchKernelGGL(k_dots<NB>, dim3(nb), dim3(DOT_THREADS), (size_t)(DOT_THREADS / 64) * no * sizeof(double),
+                               st, PA, na, PB, S.partial.as<double>(), N);
         });
         HIPOTF_CHECK(hipGetLastError());
-        hipLaunchKernelGGL(k_multi_reduce, dim3(NA * nbv), dim3(256), 0, st, part, nb, S.small.as<double>());
+        hipLaunchKernelGGL(k_multi_reduce, dim3(no), dim3(256), 0, st, S.partial.as<double>(), nb, S.small.as<double>());
         HIPOTF_CHECK(hipGetLastError());
-        HIPOTF_CHECK(hipMemcpyAsync(h.data(), S.small.p, (size_t)NA * nbv * sizeof(double), hipMemcpyDeviceToHost, st));
+        HIPOTF_CHECK(hipMemcpyAsync(h.data(), S.small.p, (size_t)no * sizeof(double), hipMemcpyDeviceToHost, st));
         HIPOTF_CHECK(hipStreamSynchronize(st));
-        for (int a = 0; a < ka; ++a)
-            for (int b = 0; b < nbv; ++b) G[(size_t)(a0 + a) * nbv + b] = h[(size_t)a * nbv + b];
     }
+    std::copy(h.begin(), h.end(), G);
 }
 
 // T_j -= sum_i P[i][j] V_i  (P host row-major [m][nt], nt <= BK)

@@ -714,8 +714,12 @@ constexpr int ab_eptmax() { return (sizeof(T) == 8 && NVS >= 4) ? 4 : 8; }
 // launch, n <= 16) first.  The matrix-core kernel's default range is where it was measured
 // faster: at 12 orbitals its FP64 sigma is 8% slower (0.66 vs 0.61 ms), at 14 and 16 it is 1.4
 // and 1.6 times faster.
-static bool ab_mma_first(int pref, int prec, int n) {
-    return pref == 5 || (pref == 0 && (prec == 0 || (n >= 14 && n <= 16)));
+// FP32 calls that promise the caller a fixed rounding (fixed = true: hipotf_hvec_block, whose FP32
+// results below 14 orbitals are those of the class-split and source-lane kernels) keep them there;
+// the Davidson driver's FP32 phase takes the matrix cores at every size (12 orbitals, 4 vectors:
+// 1.36 -> 0.37 ms)
+static bool ab_mma_first(int pref, int prec, int n, bool fixed) {
+    return pref == 5 || (pref == 0 && (prec == 0 || !fixed || (n >= 14 && n <= 16)));
 }
 static int ab_kernel_pref(int prec) {
     const int p = tuning(prec).ab_kernel;
@@ -1058,7 +1062,7 @@ static void launch_ab_nvs(DevHam *H, const T *xt, T *s1, int nvst, int v0, const
 // processes the nv interleaved vectors in sub-blocks of NVS so that a staged source row fits
 // LDS and the per-lane accumulators stay within ~64 VGPRs
 template <typename T>
-static void launch_ab(DevHam *H, const T *xt, T *s1, int nv, const T *eri, hipStream_t st) {
+static void launch_ab(DevHam *H, const T *xt, T *s1, int nv, const T *eri, hipStream_t st, bool fixed) {
     DevBasis *B = H->basis;
     const i64 NB = B->pB->N;
     if (B->pA->N == 0 || NB == 0) return;
@@ -1068,7 +1072,7 @@ static void launch_ab(DevHam *H, const T *xt, T *s1, int nv, const T *eri, hipSt
     const int pref = ab_kernel_pref(sizeof(T) == 4);
     if (pref <= 1 || pref >= 4) {
         while (v0 < nv) {
-            if (ab_mma_first(pref, sizeof(T) == 4, H->n) && try_ab_mma<T>(H, xt, s1, nv, v0, eri, st)) {
+            if (ab_mma_first(pref, sizeof(T) == 4, H->n, fixed) && try_ab_mma<T>(H, xt, s1, nv, v0, eri, st)) {
                 v0 += 1;
                 continue;
             }
@@ -1098,7 +1102,7 @@ static void launch_ab(DevHam *H, const T *xt, T *s1, int nv, const T *eri, hipSt
 // work: NULL (the basis's own work buffers, grown as needed) or 4 consecutive 256-byte aligned
 // regions of round_up(dim * NV * sizeof(T), 256) bytes each
 template <typename T, int NV>
-static void sigma_group(DevHam *H, const SrcPack &src, const DstPack &dst, hipStream_t st,
+static void sigma_group(DevHam *H, const SrcPack &src, const DstPack &dst, hipStream_t st, bool fixed = true,
                         unsigned char *work = nullptr) {
     DevBasis *B = H->basis;
     const DevSpin &A = *B->pA, &Bs = *B->pB;
@@ -1132,7 +1136,7 @@ static void sigma_group(DevHam *H, const SrcPack &src, const DstPack &dst, hipSt
     const T *eri = f32 ? (const T *)H->eri32.p : (const T *)H->eri64.p;
     AbTiming &tm = ab_timing();
     if (tm.on) HIPOTF_CHECK(hipEventRecord(tm.e0, st));
-    launch_ab<T>(H, xt, s1, NV, eri, st);
+    launch_ab<T>(H, xt, s1, NV, eri, st, fixed);
     if (tm.on) {
         HIPOTF_CHECK(hipEventRecord(tm.e1, st));
         HIPOTF_CHECK(hipEventSynchronize(tm.e1));
@@ -1148,7 +1152,7 @@ static void sigma_group(DevHam *H, const SrcPack &src, const DstPack &dst, hipSt
 
 template <typename T>
 static void sigma_t(DevHam *H, int nv, const double *const *src, double *const *dst, hipStream_t st,
-                    int maxnv) {
+                    int maxnv, bool fixed) {
     for (int g0 = 0; g0 < nv; g0 += maxnv) {
         const int m = std::min(maxnv, nv - g0);
         SrcPack sp{};
@@ -1159,25 +1163,25 @@ static void sigma_t(DevHam *H, int nv, const double *const *src, double *const *
             dp.p[i] = dst[g0 + i];
         }
         switch (m) {
-            case 1: sigma_group<T, 1>(H, sp, dp, st); break;
-            case 2: sigma_group<T, 2>(H, sp, dp, st); break;
-            case 3: sigma_group<T, 3>(H, sp, dp, st); break;
-            case 4: sigma_group<T, 4>(H, sp, dp, st); break;
-            case 5: sigma_group<T, 5>(H, sp, dp, st); break;
-            case 6: sigma_group<T, 6>(H, sp, dp, st); break;
-            case 7: sigma_group<T, 7>(H, sp, dp, st); break;
-            default: sigma_group<T, 8>(H, sp, dp, st); break;
+            case 1: sigma_group<T, 1>(H, sp, dp, st, fixed); break;
+            case 2: sigma_group<T, 2>(H, sp, dp, st, fixed); break;
+            case 3: sigma_group<T, 3>(H, sp, dp, st, fixed); break;
+            case 4: sigma_group<T, 4>(H, sp, dp, st, fixed); break;
+            case 5: sigma_group<T, 5>(H, sp, dp, st, fixed); break;
+            case 6: sigma_group<T, 6>(H, sp, dp, st, fixed); break;
+            case 7: sigma_group<T, 7>(H, sp, dp, st, fixed); break;
+            default: sigma_group<T, 8>(H, sp, dp, st, fixed); break;
         }
     }
 }
 
 void sigma(DevHam *H, int nv, const double *const *src, double *const *dst, int prec, hipStream_t st,
-           int maxnv) {
+           int maxnv, bool fixed) {
     HIPOTF_REQUIRE(H != nullptr, "Hamiltonian handle is NULL");
     HIPOTF_REQUIRE(nv >= 1, "need at least one vector");
     HIPOTF_REQUIRE(maxnv >= 1 && maxnv <= MAXNV, "vectors per sigma pass out of range");
-    if (prec == 0) sigma_t<double>(H, nv, src, dst, st, maxnv);
-    else sigma_t<float>(H, nv, src, dst, st, maxnv);
+    if (prec == 0) sigma_t<double>(H, nv, src, dst, st, maxnv, fixed);
+    else sigma_t<float>(H, nv, src, dst, st, maxnv, fixed);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1217,7 +1221,7 @@ void sigma_noalloc(DevHam *H, const double *src, double *dst, hipStream_t st) {
     DstPack dp{};
     sp.p[0] = src;
     dp.p[0] = dst;
-    sigma_group<double, 1>(H, sp, dp, st, work);
+    sigma_group<double, 1>(H, sp, dp, st, true, work);
 }
 
 void diag_elements(DevHam *H, double *diags, hipStream_t st) {
