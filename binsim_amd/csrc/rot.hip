@@ -1175,7 +1175,7 @@ static void sweeps(DevPool *P, i64 n, const i64 *idxs, const double *thetas, con
             a.list = s.lv->list.as<u32>();
             if (back) a.partial = pend_add(s);
             const i64 nblk = (a.nunit * a.nbins + 7) / 8 * 8;
-            const int np = lv_words(*s.lv, back, nblk), bd = lv_threads(*s.lv, np);
+            const int np = lv_words(*s.lv, back, grad, nblk), bd = lv_threads(*s.lv, np);
             const size_t smem = lv_lds(*s.lv, back, bd);
             HIPOTF_REQUIRE(nblk < (1ll << 31), "rotation sweep grid too large");
             auto go = [&](auto kern) {

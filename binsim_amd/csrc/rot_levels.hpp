@@ -511,14 +511,17 @@ static LevelPlan *level_plan(DevPool *P, int spin, bool pair, int kb) {
 // Two words per thread share the descriptor work, but where few waves are in flight on a CU (a
 // bin that fills the LDS, or a small grid) a generator's phase is latency and one word on twice the
 // waves is faster (12 orbitals: adjoint runs 31 -> 24 us, forward 24 -> 18; 14 orbitals, nine bins
-// per CU: forward 12.2 ms per sweep with two words, 13.5 with one).  More than four waves
-// come in whole rounds of the CU's four SIMDs.
+// per CU: forward 12.2 ms per sweep with two words, 13.5 with one).  The gradient-only pass has no
+// barrier between generators, its waves run ahead on their own, and two words are never slower
+// (whole pool at 14 orbitals 7.5 -> 6.7 ms).  More than four waves come in whole rounds of the
+// CU's four SIMDs.
 static int lv_threads(const LevelPlan &L, int np) {
     const int t = (L.maxlen + np - 1) / np, m = t > 256 ? 256 : 64;
     return std::max(64, (t + m - 1) / m * m);
 }
-static int lv_words(const LevelPlan &L, bool back, i64 nblk) {
+static int lv_words(const LevelPlan &L, bool back, bool grad, i64 nblk) {
     if (L.maxlen > 2048) return 4;
+    if (grad) return L.maxlen > 64 ? 2 : 1;
     if (L.maxlen > 1024) return 2;
     const int bd = lv_threads(L, 2);
     const i64 perCU = std::min<i64>((i64)(seg_lds_budget() / lv_lds(L, back, bd)), (nblk + 255) / 256);
