@@ -27,7 +27,8 @@ double ritz_and_residual(i64 N, int dim, const double *coeffs, double min_e, con
 void ritz_vector(i64 N, int dim, const double *coeffs, const double *const *V, double *xt, hipStream_t st);
 void precondition(i64 N, double *axt, const double *diags, double min_e, double shift, hipStream_t st);
 double mgs(i64 N, int dim, const double *const *V, double *vt, hipStream_t st);
-double normalize(i64 N, double *vec, hipStream_t st);
+void scale_inv(i64 N, double *vec, double nrm, hipStream_t st);
+void norms(i64 N, int k, double *const *T, double *out, hipStream_t st);
 double dot(i64 N, const double *a, const double *b, hipStream_t st);
 void multidot(i64 N, int dim, const double *const *V, const double *a, double *out_host, hipStream_t st);
 void block_combine(i64 N, int m, int k, const double *C, const double *w, const double *const *X,
@@ -266,7 +267,7 @@ DavidsonOut davidson(DevHam *H, int nroots, int mode, int block, double tol, dou
             HIPOTF_REQUIRE(!required, "initial guesses are linearly dependent");
             return;
         }
-        normalize(N, V[m], st);
+        scale_inv(N, V[m], na, st);
         ++m;
     };
     size_t next_low = 0;
@@ -436,8 +437,7 @@ DavidsonOut davidson(DevHam *H, int nroots, int mode, int block, double tol, dou
                 }
                 m = 0;
                 for (int i = 0; i < kk; ++i) {
-                    mgs(N, m, (const double *const *)V.data(), V[i], st);
-                    normalize(N, V[i], st);
+                    scale_inv(N, V[i], mgs(N, m, (const double *const *)V.data(), V[i], st), st);
                     ++m;
                 }
                 phase = 0;
@@ -473,9 +473,10 @@ DavidsonOut davidson(DevHam *H, int nroots, int mode, int block, double tol, dou
                 std::swap(V[m + b], V[m + i]);  // i >= b: earlier swaps only touched lower slots
                 double *t = V[m + b];
                 precondition(N, t, diag.as<double>(), w[i], std::max(rn[i] * 1e-2, 1e-4), st);
-                nb0.push_back(std::sqrt(dot(N, t, t, st)));
                 ++b;
             }
+            nb0.resize(b);
+            norms(N, b, &V[m], nb0.data(), st);
             if (b > 0 && m > 0) {
                 std::vector<double> G((size_t)m * b);
                 for (int pass = 0; pass < 2; ++pass) {
@@ -490,7 +491,7 @@ DavidsonOut davidson(DevHam *H, int nroots, int mode, int block, double tol, dou
                 double na = mgs(N, kept, (const double *const *)&V[m], t, st);
                 if (kept > 0 && na < 0.717 * nb0[j]) na = mgs(N, kept, (const double *const *)&V[m], t, st);
                 if (na < 1e-12 * std::max(1.0, nb0[j])) continue;  // lies in the subspace
-                normalize(N, t, st);
+                scale_inv(N, t, na, st);
                 ++kept;
             }
             m += kept;
@@ -505,7 +506,7 @@ DavidsonOut davidson(DevHam *H, int nroots, int mode, int block, double tol, dou
             double na = mgs(N, m, (const double *const *)V.data(), t, st);
             if (na < 0.717 * nb) na = mgs(N, m, (const double *const *)V.data(), t, st);
             if (na < 1e-12 * std::max(1.0, nb)) continue;  // lies in the subspace
-            normalize(N, t, st);
+            scale_inv(N, t, na, st);
             ++m;
         }
         if (m == first) {

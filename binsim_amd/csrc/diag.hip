@@ -156,6 +156,11 @@ __global__ __launch_bounds__(256) void k_mgs_step(double *__restrict__ y, const 
     if (threadIdx.x == 0) pout[blockIdx.x] = t;
 }
 
+// y *= s
+__global__ __launch_bounds__(256) void k_scale(double *__restrict__ y, double s, i64 n) {
+    stream_for(n, [&](i64 i) { y[i] *= s; });
+}
+
 // y *= 1 / *nrm
 __global__ __launch_bounds__(256) void k_scale_inv(double *__restrict__ y, const double *__restrict__ nrm,
                                                    i64 n) {
@@ -272,6 +277,25 @@ double normalize(i64 N, double *vec, hipStream_t st) {
     hipLaunchKernelGGL(k_scale_inv, dim3(nb), dim3(256), 0, st, vec, nrm, N);
     HIPOTF_CHECK(hipGetLastError());
     return d2h(nrm, st);  // (waits for the scaling too)
+}
+
+// vec /= nrm for a norm the caller already has (mgs returns it): no further dot product or wait
+void scale_inv(i64 N, double *vec, double nrm, hipStream_t st) {
+    hipLaunchKernelGGL(k_scale, dim3(nblk(N)), dim3(256), 0, st, vec, 1.0 / nrm, N);
+    HIPOTF_CHECK(hipGetLastError());
+}
+
+// out[j] = |T_j|, j < k <= 8, with one synchronisation
+void norms(i64 N, int k, double *const *T, double *out, hipStream_t st) {
+    HIPOTF_REQUIRE(k >= 0 && k <= 8, "norms: at most 8 vectors");
+    if (k == 0) return;
+    auto &S = scratch();
+    double *d = S.scal.as<double>() + 16;
+    for (int j = 0; j < k; ++j) dot_dev(N, T[j], T[j], d + j, st);
+    double h[8];
+    HIPOTF_CHECK(hipMemcpyAsync(h, d, k * sizeof(double), hipMemcpyDeviceToHost, st));
+    HIPOTF_CHECK(hipStreamSynchronize(st));
+    for (int j = 0; j < k; ++j) out[j] = std::sqrt(h[j]);
 }
 
 double dot(i64 N, const double *a, const double *b, hipStream_t st) {
