@@ -200,9 +200,10 @@ __global__ __launch_bounds__(256) void k_rbspmm(const T *__restrict__ X, T *__re
 
 // ---------------------------------------------------------------------------------------
 // K2/K3 on the matrix cores (FP64, the default): the row blocks of k_rbspmm with 8 strings, one
-// wave = one block x 32 NP columns.  Per batch of 4 of the block's sources the 8 x 4 coefficients
-// times the 4 source slices as 4x4x4 MFMAs (two row quads x 2 NP groups of 16 columns; each lane
-// loads 2 consecutive columns, 16 bytes).  The coefficients come as a vector load in operand order
+// wave = one block x 32 NP columns (FP32: 64 NP).  Per batch of 4 of the block's sources the 8 x 4
+// coefficients times the 4 source slices as FP64 4x4x4 MFMAs (two row quads x groups of 16 columns;
+// each lane loads 2 or 4 consecutive columns, 16 bytes).  FP32 vectors are widened on the way in,
+// summed in FP64 and rounded once per source range.  The coefficients come as a vector load in operand order
 // and, like the slices and the source indices, MB_GRP batches ahead in registers.
 //
 // Why: k_rbspmm's coefficients are scalar loads, 64 bytes per 16 FMAs, which cannot be held ahead
@@ -214,39 +215,41 @@ __global__ __launch_bounds__(256) void k_rbspmm(const T *__restrict__ X, T *__re
 // CUs; the matrix cores are 50% busy).  Measured and not faster: 96 or 256 columns per wave, 2
 // batches ahead, and the slices staged in LDS for 64 strings (147 GB staged instead of 480
 // gathered, but 49 ms with scalar coefficients and 76 ms on the matrix cores: too few loads in
-// flight beside the LDS buffers).
+// flight beside the LDS buffers).  FP32, blocks of 4 vectors, 12 orbitals / 6 electrons: 173 (k_rbspmm)
+// -> 121 us per spin; 256 columns per wave the same.
 // ---------------------------------------------------------------------------------------
 constexpr size_t MB_SLACK = 1024;  // bytes after the source vector that k_mbspmm may read
-template <int NP>
+template <typename T, int NP>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NP == 4 ? 3 : 4)))
-void k_mbspmm(const double *__restrict__ X, double *__restrict__ Y,
+void k_mbspmm(const T *__restrict__ X, T *__restrict__ Y,
                                                 const int32_t *__restrict__ J, const int32_t *__restrict__ P,
                                                 const double2 *__restrict__ C, i64 nrows, i64 ncols, i64 nblk,
                                                 i64 nwork, i64 per_xcd, int nr, int r, int accumulate) {
-    typedef double V2 __attribute__((ext_vector_type(2), aligned(8)));
+    constexpr int W = 16 / sizeof(T);  // consecutive columns per lane and load
+    typedef T VW __attribute__((ext_vector_type(16 / sizeof(T)), aligned(sizeof(T))));
     const int lane = threadIdx.x & 63, k = lane >> 4, j = lane & 15;
     // contiguous ranges of wave items per XCD (tile-major: all blocks of a column tile, then the next)
     const i64 w = (i64)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if ((blockIdx.x >> 3) * 4 + (threadIdx.x >> 6) >= per_xcd || w >= nwork) return;
     const i64 tile = w / nblk, blk = w - tile * nblk;
     // (lanes past the last column read into the next row, or the slack after the last one)
-    const i64 col0 = tile * (32 * NP) + 2 * j;
+    const i64 col0 = tile * (16 * W * NP) + W * j;
     const char *Xc = reinterpret_cast<const char *>(X + (col0 < ncols ? col0 : 0));
     int b = P[blk * (nr + 1) + r];
     const int e = P[blk * (nr + 1) + r + 1];
-    double acc[2][2 * NP];
+    double acc[2][W * NP];
 #pragma unroll
-    for (int q = 0; q < 2 * NP; ++q) acc[0][q] = acc[1][q] = 0.0;
-    const u32 jo = (u32)k * 4, co = (u32)(k * 4 + (lane & 3)) * 16, rowb = (u32)ncols * 8;
+    for (int q = 0; q < W * NP; ++q) acc[0][q] = acc[1][q] = 0.0;
+    const u32 jo = (u32)k * 4, co = (u32)(k * 4 + (lane & 3)) * 16, rowb = (u32)ncols * (u32)sizeof(T);
     auto src = [&](int at) { return *reinterpret_cast<const u32 *>(reinterpret_cast<const char *>(J + (i64)at * 4) + jo); };
     u32 jn[MB_GRP];
     double2 a[MB_GRP];
-    V2 x[MB_GRP][NP];
+    VW x[MB_GRP][NP];
     auto fetch = [&](int q, int at) {  // batch `at` into slot q, then the indices MB_GRP further on
         a[q] = *reinterpret_cast<const double2 *>(reinterpret_cast<const char *>(C + (i64)at * 16) + co);
         const char *xr = Xc + (u64)jn[q] * rowb;
 #pragma unroll
-        for (int p = 0; p < NP; ++p) x[q][p] = *reinterpret_cast<const V2 *>(xr + 256 * p);
+        for (int p = 0; p < NP; ++p) x[q][p] = *reinterpret_cast<const VW *>(xr + 256 * p);
         jn[q] = src(at + MB_GRP);
     };
     if (b < e) {
@@ -259,15 +262,16 @@ void k_mbspmm(const double *__restrict__ X, double *__restrict__ Y,
 #pragma unroll
         for (int q = 0; q < MB_GRP; ++q) {
             const double2 av = a[q];
-            V2 xv[NP];
+            VW xv[NP];
 #pragma unroll
             for (int p = 0; p < NP; ++p) xv[p] = x[q][p];
 #pragma unroll
             for (int p = 0; p < NP; ++p)
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    acc[0][2 * p + h] = __builtin_amdgcn_mfma_f64_4x4x4f64(av.x, xv[p][h], acc[0][2 * p + h], 0, 0, 0);
-                    acc[1][2 * p + h] = __builtin_amdgcn_mfma_f64_4x4x4f64(av.y, xv[p][h], acc[1][2 * p + h], 0, 0, 0);
+                for (int h = 0; h < W; ++h) {
+                    const double v = (double)xv[p][h];
+                    acc[0][W * p + h] = __builtin_amdgcn_mfma_f64_4x4x4f64(av.x, v, acc[0][W * p + h], 0, 0, 0);
+                    acc[1][W * p + h] = __builtin_amdgcn_mfma_f64_4x4x4f64(av.y, v, acc[1][W * p + h], 0, 0, 0);
                 }
             __builtin_amdgcn_sched_barrier(0);  // (the scheduler would sink the loads to their uses)
             fetch(q, b + MB_GRP + q);
@@ -280,10 +284,11 @@ void k_mbspmm(const double *__restrict__ X, double *__restrict__ Y,
         if (row >= nrows) continue;
 #pragma unroll
         for (int p = 0; p < NP; ++p) {
-            const i64 col = col0 + 32 * p;
-            double *y = Y + row * ncols + col;
-            if (col < ncols) y[0] = accumulate ? y[0] + acc[h][2 * p] : acc[h][2 * p];
-            if (col + 1 < ncols) y[1] = accumulate ? y[1] + acc[h][2 * p + 1] : acc[h][2 * p + 1];
+            const i64 col = col0 + 16 * W * p;
+            T *y = Y + row * ncols + col;
+#pragma unroll
+            for (int c = 0; c < W; ++c)
+                if (col + c < ncols) y[c] = (T)(accumulate ? (double)y[c] + acc[h][W * p + c] : acc[h][W * p + c]);
         }
     }
 }
@@ -628,13 +633,14 @@ static int rs_npass(i64 nrows, int tile_cols) {
     return p;
 }
 
-template <int NP>
-static void launch_mbspmm_n(const double *X, double *Y, const MfmaBlockTable &M, i64 nrows, i64 ncols, hipStream_t st) {
-    const i64 ntiles = (ncols + 32 * NP - 1) / (32 * NP), nwork = ntiles * M.nblk, per_xcd = (nwork + 7) / 8;
+template <typename T, int NP>
+static void launch_mbspmm_n(const T *X, T *Y, const MfmaBlockTable &M, i64 nrows, i64 ncols, hipStream_t st) {
+    constexpr int cols = 256 / sizeof(T) * NP;
+    const i64 ntiles = (ncols + cols - 1) / cols, nwork = ntiles * M.nblk, per_xcd = (nwork + 7) / 8;
     const i64 nwg = (per_xcd + 3) / 4 * 8;
     HIPOTF_REQUIRE(nwg < (1ll << 31), "row-block SpMM grid too large");
     for (int r = 0; r < M.nr; ++r)
-        hipLaunchKernelGGL(k_mbspmm<NP>, dim3((unsigned)nwg), dim3(256), 0, st, X, Y, M.J.as<int32_t>(),
+        hipLaunchKernelGGL((k_mbspmm<T, NP>), dim3((unsigned)nwg), dim3(256), 0, st, X, Y, M.J.as<int32_t>(),
                            M.P.as<int32_t>(), M.c64.as<double2>(), nrows, ncols, M.nblk, nwork, per_xcd, M.nr, r,
                            r > 0 ? 1 : 0);
     HIPOTF_CHECK(hipGetLastError());
@@ -643,25 +649,31 @@ static void launch_mbspmm_n(const double *X, double *Y, const MfmaBlockTable &M,
 // 128 columns per wave (the fewest coefficient and index loads per product), fewer where that leaves
 // the chip short of waves.  FP64 sigma with 128 / 64 / 32 columns: 8 orbitals / 4 + 4 electrons 24.9 /
 // 23.2 / 22.8 us, 10 / 5 + 5 45 / 40 / 36 us, 12 / 6 + 6 207 / 216 / 240 us, 16 / 8 + 8 109 / 118 / 136 ms
-static void launch_mbspmm(const double *X, double *Y, const MfmaBlockTable &M, i64 nrows, i64 ncols, hipStream_t st) {
-    auto waves = [&](int np) { return (ncols + 32 * np - 1) / (32 * np) * M.nblk; };
-    const int np = waves(4) >= 768 ? 4 : (waves(2) >= 384 ? 2 : 1);
-    if (np == 4) launch_mbspmm_n<4>(X, Y, M, nrows, ncols, st);
-    else if (np == 2) launch_mbspmm_n<2>(X, Y, M, nrows, ncols, st);
-    else launch_mbspmm_n<1>(X, Y, M, nrows, ncols, st);
+template <typename T>
+static void launch_mbspmm(const T *X, T *Y, const MfmaBlockTable &M, i64 nrows, i64 ncols, hipStream_t st) {
+    auto waves = [&](int cols) { return (ncols + cols - 1) / cols * M.nblk; };
+    const int cols = waves(128) >= 768 ? 128 : (waves(64) >= 384 ? 64 : 32);
+    if constexpr (sizeof(T) == 4) {
+        if (cols == 128) launch_mbspmm_n<T, 2>(X, Y, M, nrows, ncols, st);
+        else launch_mbspmm_n<T, 1>(X, Y, M, nrows, ncols, st);
+    } else {
+        if (cols == 128) launch_mbspmm_n<T, 4>(X, Y, M, nrows, ncols, st);
+        else if (cols == 64) launch_mbspmm_n<T, 2>(X, Y, M, nrows, ncols, st);
+        else launch_mbspmm_n<T, 1>(X, Y, M, nrows, ncols, st);
+    }
 }
 
 template <typename T>
 static void launch_rowspmm(const T *X, T *Y, SameSpinTable &tab, const T *C, i64 nrows,
-                           i64 ncols, hipStream_t st) {
+                           i64 ncols, bool fixed, hipStream_t st) {
     if (nrows == 0 || ncols == 0) return;
     HIPOTF_REQUIRE(nrows == tab.N, "internal: same-spin table does not match the row count");
     int rb = tuning(sizeof(T) == 4).rs_block;
     if (rb == MB_RB && tuning(sizeof(T) == 4).rs_passes == 0) {  // the defaults
-        if constexpr (sizeof(T) == 8) {
+        if (sizeof(T) == 8 || !fixed)
             if (const MfmaBlockTable *M = mfma_blocks(tab)) return launch_mbspmm(X, Y, *M, nrows, ncols, st);
-        } else {
-            // FP32: blocks of 4 strings, the same sums in the same order (FP32 sigma, 4 vectors: 12
+        if constexpr (sizeof(T) == 4) {
+            // FP32 of a fixed rounding (hipotf_hvec_block): blocks of 4 strings, the same sums in the same order (FP32 sigma, 4 vectors: 12
             // orbitals 1.77 -> 1.67 ms, 14 orbitals 12.1 -> 11.5 ms)
             rb = 4;
         }
@@ -1137,8 +1149,8 @@ static void sigma_group(DevHam *H, const SrcPack &src, const DstPack &dst, hipSt
     const bool f32 = sizeof(T) == 4;
     const T *CA = f32 ? (const T *)H->ptA->c32.p : (const T *)H->ptA->c64.p;
     const T *CB = f32 ? (const T *)H->ptB->c32.p : (const T *)H->ptB->c64.p;
-    launch_rowspmm<T>(xt, s1, *H->ptA, CA, NA, NB * NV, st);
-    launch_rowspmm<T>(xtT, s2T, *H->ptB, CB, NB, NA * NV, st);
+    launch_rowspmm<T>(xt, s1, *H->ptA, CA, NA, NB * NV, fixed, st);
+    launch_rowspmm<T>(xtT, s2T, *H->ptB, CB, NB, NA * NV, fixed, st);
     const T *eri = f32 ? (const T *)H->eri32.p : (const T *)H->eri64.p;
     AbTiming &tm = ab_timing();
     if (tm.on) HIPOTF_CHECK(hipEventRecord(tm.e0, st));
