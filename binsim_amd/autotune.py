@@ -13,13 +13,16 @@ Tuned per precision (FP64 sigma of one vector; FP32 block sigma of ``k`` vectors
   4 source-lane with FP32 vector pairs on the class-split form (the beta strings split by the
   top orbital; one class's FP64 destination elements of both vectors in LDS), 5 matrix-core
   (per destination alpha row, the dense product of the integral block with the source rows on
-  the MFMA units, scattered into an FP64 LDS row; up to 16 orbitals, one vector per launch);
+  the MFMA units, scattered into an FP64 LDS row; FP64 up to 18 orbitals, FP32 up to 16, one
+  vector per launch);
 * ``ab_split``: lanes per source string in the source-lane kernel, i.e. waves per CU
   (1: 512-thread workgroups, 8 waves per CU; 2: 1024-thread workgroups, 16 waves per CU);
 * ``ab_db``: one or two LDS copies of the replicated integral row (source-lane);
 * ``ab_nvs``: vectors per source-lane launch in FP32 (1 or 2);
 * ``rs_block``: destination alpha (beta) strings per workgroup of the same-spin row SpMM that
-  share each gathered source row (4, 8, 16; 0 = one destination row per wave);
+  share each gathered source row (4, 8, 16; 0 = one destination row per wave; 8 with
+  ``rs_passes`` 0, the library's default, runs on the matrix cores in FP64 and in blocks of 4 in
+  FP32);
 * ``rs_passes``: the same-spin row SpMM gathers its sources in 1, 2, 4 or 8 alpha-string
   ranges (source alpha block of N/passes strings per launch; the library's default, 0, takes
   the fewest that keep a column tile's gathered slice within an XCD's 4 MB L2);

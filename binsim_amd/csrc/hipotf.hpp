@@ -238,8 +238,10 @@ DevHam *make_dev_ham(DevBasis *b, int n, const std::vector<double> &h, const std
 // launch choices of the sigma kernels (process-wide; set by hipotf_set_tuning, chosen by the
 // autotuner in binsim_amd/autotune.py)
 struct SigmaTuning {
-    int ab_kernel = 0;      // alpha-beta kernel: 0 first that applies (source-lane, register,
-                            // chunked), 1 source-lane, 2 register-descriptor, 3 chunked
+    int ab_kernel = 0;      // alpha-beta kernel: 0 the default for the precision and size (the
+                            // matrix-core kernel up to 18 orbitals in FP64; sigma.hip), 1
+                            // source-lane, 2 register-descriptor, 3 chunked, 4 class-split FP32
+                            // pairs, 5 matrix-core
     int ab_split = 1;       // source-lane: threads per source string (1: 8 waves/CU, 2: 16)
     int ab_db = 1;          // source-lane: integral-row buffers (1, or 2 where LDS allows)
     int ab_nvs = 2;         // source-lane, FP32: vectors per launch (1 or 2)
@@ -247,8 +249,10 @@ struct SigmaTuning {
                             // for which a column tile's gathered slice fits an XCD's L2)
     int deterministic = 0;  // 1: alpha-beta scatter wave by wave (bitwise reproducible)
     int rs_block = 8;       // row SpMM: destination rows sharing each gathered source row
-                            // (4, 8, 16), or 0 for one row per wave
-    int sweep_mode = 4;     // VQE rotation sweeps (FP64 table): 0 fused segments with as many
+                            // (4, 8, 16), or 0 for one row per wave; 8 with rs_passes 0, the
+                            // defaults, is the matrix-core form in FP64 and blocks of 4 in FP32
+    int sweep_mode = 4;     // VQE rotation sweeps (FP64 table): 0 fused, on excitation levels in
+                            // LDS where the pool allows (rot_levels.hpp), else with as many
                             // rows (and the leading part of one more) in LDS as fit, the
                             // others in global memory; 1 fused, rows
                             // always in global memory; 2 one launch per generator; 3 fused,

@@ -3,11 +3,13 @@
 // Replaces cuda_hvec / hvec_gather_*_kernel (src/include/cuda/hvec.cuh:6-446) and the CPU
 // contract_network_otf (src/include/op/hvec.hpp:481-496).  Pipeline per block of nv vectors:
 //   K1 k_gauge_in   x -> x~ = E x, written alpha-major (xt) and beta-major (xtT), T precision
-//   K2 k_rowspmm    s1  = G_alpha x~          rows = alpha strings, coalesced row streams
-//   K3 k_rowspmm    s2T = G_beta  x~^T        same kernel on the beta-major copy
-//   K4 k_ab         s1 += H_ab x~              one workgroup per destination alpha row; each
-//                                               source row staged in LDS, beta connectivity
-//                                               read per lane, integrals (pq|rs) row in LDS
+//   K2 k_mbspmm     s1  = G_alpha x~          rows = alpha strings, 8 per wave on the matrix cores
+//                                               (k_rbspmm: FP32 blocks of 4; k_rowspmm: one per wave)
+//   K3 k_mbspmm     s2T = G_beta  x~^T        same kernel on the beta-major copy
+//   K4 k_ab_mma     s1 += H_ab x~              one workgroup per destination alpha row: the dense
+//                                               product of its integral block with its source rows
+//                                               on the matrix cores, scattered into an FP64 LDS row
+//                                               (k_ab_cls, k_ab_src, k_ab_reg, k_ab: other sizes)
 //   K5 k_finalize   sigma = E (s1 + s2T^T + E_core x~)   tiled transpose, FP64 output
 // T = double (drop-in FP64) or float (mixed precision).  Sum order differs from the
 // reference, so FP64 results agree to rounding (~1e-15 relative), not bit-for-bit.
@@ -673,8 +675,9 @@ static void launch_rowspmm(const T *X, T *Y, SameSpinTable &tab, const T *C, i64
         if (sizeof(T) == 8 || !fixed)
             if (const MfmaBlockTable *M = mfma_blocks(tab)) return launch_mbspmm(X, Y, *M, nrows, ncols, st);
         if constexpr (sizeof(T) == 4) {
-            // FP32 of a fixed rounding (hipotf_hvec_block): blocks of 4 strings, the same sums in the same order (FP32 sigma, 4 vectors: 12
-            // orbitals 1.77 -> 1.67 ms, 14 orbitals 12.1 -> 11.5 ms)
+            // FP32 of a fixed rounding (hipotf_hvec_block): blocks of 4 strings, the same sums in
+            // the same order (FP32 sigma, 4 vectors: 12 orbitals 1.77 -> 1.67 ms, 14 orbitals
+            // 12.1 -> 11.5 ms)
             rb = 4;
         }
     }
@@ -725,13 +728,13 @@ static void launch_ab_ept(DevHam *H, const T *xt, T *s1, int nvst, int v0, const
 template <typename T, int NVS>
 constexpr int ab_eptmax() { return (sizeof(T) == 8 && NVS >= 4) ? 4 : 8; }
 
-// alpha-beta kernel family (SigmaTuning::ab_kernel): 0 takes the first of matrix-core (14 to 16
-// orbitals), class-split (FP32 vector pairs, ab_cls.hpp), source-lane, register, chunked that
+// alpha-beta kernel family (SigmaTuning::ab_kernel): 0 takes the first of matrix-core (FP64 up
+// to 18 orbitals; FP32 of a fixed rounding 14 to 16), class-split (FP32 vector pairs, ab_cls.hpp), source-lane, register, chunked that
 // applies; 1..3 start the search at source-lane, register, chunked; 4 is 1 with FP32 vector
 // pairs on the class-split kernel; 5 puts the matrix-core kernel (ab_mma.hpp, one vector per
-// launch, n <= 16) first.  The matrix-core kernel's default range is where it was measured
-// faster: at 12 orbitals its FP64 sigma is 8% slower (0.66 vs 0.61 ms), at 14 and 16 it is 1.4
-// and 1.6 times faster.
+// launch) first.  The matrix-core kernel's FP64 range is all it can hold: it is the fastest at
+// every size measured (whole FP64 sigma against the source-lane kernel beside the same row SpMM: 12
+// orbitals 6 + 6 0.22 / 0.51 ms, 14 / 7 + 7 4.1 / 9.8 ms, 16 / 8 + 8 109 / 198 ms).
 // FP32 calls that promise the caller a fixed rounding (fixed = true: hipotf_hvec_block, whose FP32
 // results below 14 orbitals are those of the class-split and source-lane kernels) keep them there;
 // the Davidson driver's FP32 phase takes the matrix cores at every size (12 orbitals, 4 vectors:

@@ -131,14 +131,15 @@ int64_t hipotf_num_generators(void *net);
 int hipotf_prepare(void *basis, void *net);
 /* launch choices of the sigma kernels, process-wide (no reference counterpart; the
  * reference's tiles are compile-time, src/include/ham/otf.hpp:6-9 and cuda/common.cuh:7-12):
- * v[8] = {alpha-beta kernel 0 auto (matrix-core at 14-16 orbitals, else class-split FP32 pairs,
- * source-lane, register, chunked) | 1 source-lane | 2 register | 3 chunked | 4 source-lane with
- * FP32 vector pairs on the class-split kernel | 5 matrix-core (16 orbitals or fewer), threads per
+ * v[8] = {alpha-beta kernel 0 auto (matrix-core: FP64 up to 18 orbitals, FP32 at 14-16; else
+ * class-split FP32 pairs, source-lane, register, chunked) | 1 source-lane | 2 register | 3 chunked | 4 source-lane with
+ * FP32 vector pairs on the class-split kernel | 5 matrix-core (where it applies), threads per
  * source string 1|2, integral-row buffers 1|2, FP32 vectors per alpha-beta launch 1|2,
  * row-SpMM source-range passes 1|2|4|8 (0: as many as keep a column tile's gathered slice
  * within an XCD's L2), deterministic 0|1, same-spin destination rows per
- * gathered source row 4|8|16 (0: one row per wave), VQE rotation sweeps 0 fused (as many rows
- * in LDS as fit, the others in global memory) | 1 fused with rows in global memory | 2 one
+ * gathered source row 4|8|16 (0: one row per wave; 8 with 0 passes, the defaults: FP64 on the
+ * matrix cores, FP32 in blocks of 4), VQE rotation sweeps 0 fused (runs of particle-hole
+ * generators on excitation levels in LDS; else as many rows in LDS as fit, the others in global memory) | 1 fused with rows in global memory | 2 one
  * launch per generator | 3 fused with at most one row and half of the next in LDS, +4 (4..7)
  * the same with the adjoint sweep's alpha-pair segments on interleaved (l, r) rows (default 4;
  * FP64 table only)},
