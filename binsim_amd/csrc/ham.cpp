@@ -330,10 +330,14 @@ DevHam *make_dev_ham(DevBasis *b, int n, const std::vector<double> &h, const std
     // the default row blocks now, so that the first sigma does not pay for them
     for (int prec = 0; prec < 2; ++prec) {
         const int rb = tuning(prec).rs_block;
-        if (prec == 0 && rb == MB_RB && tuning(prec).rs_passes == 0) {
+        // the matrix-core tables in FP64; FP32 has blocks of 4, built when used.  The blocks of 8
+        // beside them where hipotf_hvec_noalloc, which builds none, may be called with other passes
+        const bool mb = rb == MB_RB && tuning(prec).rs_passes == 0, small = hb.dim <= NOALLOC_MAX_DIM;
+        if (prec == 0 && (mb || (rb == MB_RB && small))) {
             mfma_blocks(*H->ptA);
             mfma_blocks(*H->ptB);
         }
+        if (mb && !small && H->tA.dev_built && H->ptB->dev_built) continue;
         if (rb == 4 || rb == 8 || rb == 16) {
             row_blocks(*H->ptA, rb);
             row_blocks(*H->ptB, rb);

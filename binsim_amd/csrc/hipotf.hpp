@@ -168,16 +168,18 @@ struct RowBlockTable {
     DevBuf c64, c32;          // double / float [entries][rb]
 };
 
-// the row blocks of MB_RB strings in MFMA-operand order for the FP64 matrix-core row SpMM
+// the row blocks of 8 or 16 strings in MFMA-operand order for the FP64 matrix-core row SpMM
 // (k_mbspmm): each block's sources in nr source ranges, each range padded to whole groups of
 // MB_GRP batches of 4 sources (coefficient 0, a valid source)
 constexpr int MB_RB = 8, MB_GRP = 4;
 struct MfmaBlockTable {
+    int rb = MB_RB;           // strings per block: 8 or 16
     int nr = 1;               // source ranges: passes of the kernel
     i64 nblk = 0, batches = 0;
     DevBuf P;                 // int32[nblk][nr + 1]: first batch of each range, end
     DevBuf J;                 // int32[batches][4]: sources
-    DevBuf c64;               // double[batches][4 sources][4][2]: coefficients of rows i and i + 4
+    DevBuf c64;               // rb 8: double[batches][4 sources][4][2]: coefficients of rows i and
+                              // i + 4; rb 16: double[batches][4 sources][16]
 };
 
 struct SameSpinTable {

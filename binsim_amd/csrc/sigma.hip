@@ -201,31 +201,33 @@ __global__ __launch_bounds__(256) void k_rbspmm(const T *__restrict__ X, T *__re
 }
 
 // ---------------------------------------------------------------------------------------
-// K2/K3 on the matrix cores (FP64, the default): the row blocks of k_rbspmm with 8 strings, one
-// wave = one block x 32 NP columns (FP32: 64 NP).  Per batch of 4 of the block's sources the 8 x 4
-// coefficients times the 4 source slices as FP64 4x4x4 MFMAs (two row quads x groups of 16 columns;
-// each lane loads 2 or 4 consecutive columns, 16 bytes).  FP32 vectors are widened on the way in,
+// K2/K3 on the matrix cores (FP64, the default): the row blocks of k_rbspmm with RB = 8 or 16
+// strings, one wave = one block x 32 NP columns (FP32: 64 NP).  Per batch of 4 of the block's sources
+// the RB x 4 coefficients times the 4 source slices as FP64 MFMAs (8: 4x4x4, two row quads x groups of
+// 16 columns; 16: 16x16x4; each lane loads 2 or 4 consecutive columns, 16 bytes).  FP32 vectors are widened on the way in,
 // summed in FP64 and rounded once per source range.  The coefficients come as a vector load in operand order
 // and, like the slices and the source indices, MB_GRP batches ahead in registers.
 //
 // Why: k_rbspmm's coefficients are scalar loads, 64 bytes per 16 FMAs, which cannot be held ahead
 // in the SGPRs: its FP64 VALU was 63% busy, and one wave's chain of waits set the pace in small
-// spaces.  16-row tiles (16x16x4 MFMAs) would need 4.8 times the useful products instead of 3.4.
-// Operand layout (measured): lane l holds A[l % 4][l / 16], B[l / 16][l % 16], D[l / 16][l % 16].
-// Measured, FP64, per spin: 16 orbitals / 8 electrons 28.5 -> 24.5 ms, 12 orbitals / 6 electrons
-// 157 -> 39 us.  Bound now by the gathered bytes (480 GB per spin at 16 orbitals, 19.6 TB/s into the
-// CUs; the matrix cores are 50% busy).  Measured and not faster: 96 or 256 columns per wave, 2
+// spaces.  Blocks of 16 need 4.8 times the useful products, blocks of 8 3.4 times, but gather 30% less
+// (mfma_blocks has the rule).  Operand layouts (measured): lane l holds B[l / 16][l % 16] in both;
+// 4x4x4: A[l % 4][l / 16], D[l / 16][l % 16]; 16x16x4: A[l % 16][l / 16], element v D[4 v + l / 16][l % 16].
+// Measured, FP64, per spin: 16 orbitals / 8 electrons 28.5 -> 24.5 (blocks of 8) -> 22.6 ms (16), 12
+// orbitals / 6 electrons 157 -> 39 us (8).  Bound by the gathered bytes (16 orbitals: blocks of 8
+// 480 GB per spin, 19.6 TB/s into the CUs, matrix cores 47% busy; of 16 335 GB) and, with blocks
+// of 16, as much by the matrix cores.  Measured and not faster: 96 or 256 columns per wave, 2
 // batches ahead, and the slices staged in LDS for 64 strings (147 GB staged instead of 480
 // gathered, but 49 ms with scalar coefficients and 76 ms on the matrix cores: too few loads in
 // flight beside the LDS buffers).  FP32, blocks of 4 vectors, 12 orbitals / 6 electrons: 173 (k_rbspmm)
 // -> 121 us per spin; 256 columns per wave the same.
 // ---------------------------------------------------------------------------------------
 constexpr size_t MB_SLACK = 1024;  // bytes after the source vector that k_mbspmm may read
-template <typename T, int NP>
+template <typename T, int NP, int RB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NP == 4 ? 3 : 4)))
 void k_mbspmm(const T *__restrict__ X, T *__restrict__ Y,
                                                 const int32_t *__restrict__ J, const int32_t *__restrict__ P,
-                                                const double2 *__restrict__ C, i64 nrows, i64 ncols, i64 nblk,
+                                                const double *__restrict__ C, i64 nrows, i64 ncols, i64 nblk,
                                                 i64 nwork, i64 per_xcd, int nr, int r, int accumulate) {
     constexpr int W = 16 / sizeof(T);  // consecutive columns per lane and load
     typedef T VW __attribute__((ext_vector_type(16 / sizeof(T)), aligned(sizeof(T))));
@@ -239,16 +241,21 @@ void k_mbspmm(const T *__restrict__ X, T *__restrict__ Y,
     const char *Xc = reinterpret_cast<const char *>(X + (col0 < ncols ? col0 : 0));
     int b = P[blk * (nr + 1) + r];
     const int e = P[blk * (nr + 1) + r + 1];
-    double acc[2][W * NP];
+    typedef double V4 __attribute__((ext_vector_type(4)));
+    typedef typename std::conditional<RB == 16, double, double2>::type CF;  // a lane's coefficients of a batch
+    double acc[2][RB == 8 ? W * NP : 1];
+    V4 acc4[RB == 16 ? W * NP : 1];
 #pragma unroll
-    for (int q = 0; q < W * NP; ++q) acc[0][q] = acc[1][q] = 0.0;
-    const u32 jo = (u32)k * 4, co = (u32)(k * 4 + (lane & 3)) * 16, rowb = (u32)ncols * (u32)sizeof(T);
+    for (int q = 0; q < W * NP; ++q)
+        if constexpr (RB == 8) acc[0][q] = acc[1][q] = 0.0;
+        else acc4[q] = V4{};
+    const u32 jo = (u32)k * 4, co = RB == 16 ? (u32)lane * 8 : (u32)(k * 4 + (lane & 3)) * 16, rowb = (u32)ncols * (u32)sizeof(T);
     auto src = [&](int at) { return *reinterpret_cast<const u32 *>(reinterpret_cast<const char *>(J + (i64)at * 4) + jo); };
     u32 jn[MB_GRP];
-    double2 a[MB_GRP];
+    CF a[MB_GRP];
     VW x[MB_GRP][NP];
     auto fetch = [&](int q, int at) {  // batch `at` into slot q, then the indices MB_GRP further on
-        a[q] = *reinterpret_cast<const double2 *>(reinterpret_cast<const char *>(C + (i64)at * 16) + co);
+        a[q] = *reinterpret_cast<const CF *>(reinterpret_cast<const char *>(C + (i64)at * (4 * RB)) + co);
         const char *xr = Xc + (u64)jn[q] * rowb;
 #pragma unroll
         for (int p = 0; p < NP; ++p) x[q][p] = *reinterpret_cast<const VW *>(xr + 256 * p);
@@ -263,7 +270,7 @@ void k_mbspmm(const T *__restrict__ X, T *__restrict__ Y,
     for (; b < e; b += MB_GRP) {
 #pragma unroll
         for (int q = 0; q < MB_GRP; ++q) {
-            const double2 av = a[q];
+            const CF av = a[q];
             VW xv[NP];
 #pragma unroll
             for (int p = 0; p < NP; ++p) xv[p] = x[q][p];
@@ -272,8 +279,13 @@ void k_mbspmm(const T *__restrict__ X, T *__restrict__ Y,
 #pragma unroll
                 for (int h = 0; h < W; ++h) {
                     const double v = (double)xv[p][h];
-                    acc[0][W * p + h] = __builtin_amdgcn_mfma_f64_4x4x4f64(av.x, v, acc[0][W * p + h], 0, 0, 0);
-                    acc[1][W * p + h] = __builtin_amdgcn_mfma_f64_4x4x4f64(av.y, v, acc[1][W * p + h], 0, 0, 0);
+                    const int c = W * p + h;
+                    if constexpr (RB == 8) {
+                        acc[0][c] = __builtin_amdgcn_mfma_f64_4x4x4f64(av.x, v, acc[0][c], 0, 0, 0);
+                        acc[1][c] = __builtin_amdgcn_mfma_f64_4x4x4f64(av.y, v, acc[1][c], 0, 0, 0);
+                    } else {
+                        acc4[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, v, acc4[c], 0, 0, 0);
+                    }
                 }
             __builtin_amdgcn_sched_barrier(0);  // (the scheduler would sink the loads to their uses)
             fetch(q, b + MB_GRP + q);
@@ -281,8 +293,8 @@ void k_mbspmm(const T *__restrict__ X, T *__restrict__ Y,
         }
     }
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const i64 row = blk * MB_RB + 4 * h + k;
+    for (int h = 0; h < RB / 4; ++h) {
+        const i64 row = blk * RB + 4 * h + k;
         if (row >= nrows) continue;
 #pragma unroll
         for (int p = 0; p < NP; ++p) {
@@ -290,7 +302,12 @@ void k_mbspmm(const T *__restrict__ X, T *__restrict__ Y,
             T *y = Y + row * ncols + col;
 #pragma unroll
             for (int c = 0; c < W; ++c)
-                if (col + c < ncols) y[c] = (T)(accumulate ? (double)y[c] + acc[h][W * p + c] : acc[h][W * p + c]);
+                if (col + c < ncols) {
+                    double v;
+                    if constexpr (RB == 8) v = acc[h][W * p + c];
+                    else v = acc4[W * p + c][h];
+                    y[c] = (T)(accumulate ? (double)y[c] + v : v);
+                }
         }
     }
 }
@@ -635,15 +652,15 @@ static int rs_npass(i64 nrows, int tile_cols) {
     return p;
 }
 
-template <typename T, int NP>
+template <typename T, int NP, int RB>
 static void launch_mbspmm_n(const T *X, T *Y, const MfmaBlockTable &M, i64 nrows, i64 ncols, hipStream_t st) {
     constexpr int cols = 256 / sizeof(T) * NP;
     const i64 ntiles = (ncols + cols - 1) / cols, nwork = ntiles * M.nblk, per_xcd = (nwork + 7) / 8;
     const i64 nwg = (per_xcd + 3) / 4 * 8;
     HIPOTF_REQUIRE(nwg < (1ll << 31), "row-block SpMM grid too large");
     for (int r = 0; r < M.nr; ++r)
-        hipLaunchKernelGGL((k_mbspmm<T, NP>), dim3((unsigned)nwg), dim3(256), 0, st, X, Y, M.J.as<int32_t>(),
-                           M.P.as<int32_t>(), M.c64.as<double2>(), nrows, ncols, M.nblk, nwork, per_xcd, M.nr, r,
+        hipLaunchKernelGGL((k_mbspmm<T, NP, RB>), dim3((unsigned)nwg), dim3(256), 0, st, X, Y, M.J.as<int32_t>(),
+                           M.P.as<int32_t>(), M.c64.as<double>(), nrows, ncols, M.nblk, nwork, per_xcd, M.nr, r,
                            r > 0 ? 1 : 0);
     HIPOTF_CHECK(hipGetLastError());
 }
@@ -655,14 +672,14 @@ template <typename T>
 static void launch_mbspmm(const T *X, T *Y, const MfmaBlockTable &M, i64 nrows, i64 ncols, hipStream_t st) {
     auto waves = [&](int cols) { return (ncols + cols - 1) / cols * M.nblk; };
     const int cols = waves(128) >= 768 ? 128 : (waves(64) >= 384 ? 64 : 32);
-    if constexpr (sizeof(T) == 4) {
-        if (cols == 128) launch_mbspmm_n<T, 2>(X, Y, M, nrows, ncols, st);
-        else launch_mbspmm_n<T, 1>(X, Y, M, nrows, ncols, st);
-    } else {
-        if (cols == 128) launch_mbspmm_n<T, 4>(X, Y, M, nrows, ncols, st);
-        else if (cols == 64) launch_mbspmm_n<T, 2>(X, Y, M, nrows, ncols, st);
-        else launch_mbspmm_n<T, 1>(X, Y, M, nrows, ncols, st);
-    }
+    auto go = [&](auto rb) {
+        constexpr int RB = decltype(rb)::value, W = 16 / sizeof(T);
+        if (cols == 128) launch_mbspmm_n<T, 8 / W, RB>(X, Y, M, nrows, ncols, st);
+        else if (cols == 64 || W == 4) launch_mbspmm_n<T, 4 / W, RB>(X, Y, M, nrows, ncols, st);
+        else launch_mbspmm_n<T, 1, RB>(X, Y, M, nrows, ncols, st);
+    };
+    if (M.rb == 16) go(std::integral_constant<int, 16>{});
+    else go(std::integral_constant<int, 8>{});
 }
 
 template <typename T>

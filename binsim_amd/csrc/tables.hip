@@ -341,12 +341,12 @@ void row_blocks_dev(SameSpinTable &T, RowBlockTable &R, int rb) {
 }
 
 // ---------------------------------------------------------------------------------------
-// matrix-core row-SpMM table (MfmaBlockTable) from the blocks of MB_RB rows, one workgroup per
+// matrix-core row-SpMM table (MfmaBlockTable) from the blocks of rb rows, one workgroup per
 // block; FILL = false: its batches
 // ---------------------------------------------------------------------------------------
 template <bool FILL>
 __global__ __launch_bounds__(256) void k_mb(const int32_t *__restrict__ J, const int32_t *__restrict__ P,
-                                            const double *__restrict__ C, i64 N, int nr, int32_t *__restrict__ cnt,
+                                            const double *__restrict__ C, int rb, int nr, int32_t *__restrict__ cnt,
                                             const int32_t *__restrict__ first, int32_t *__restrict__ Pm,
                                             int32_t *__restrict__ Jm, double *__restrict__ cm) {
     const i64 b = blockIdx.x;
@@ -361,7 +361,8 @@ __global__ __launch_bounds__(256) void k_mb(const int32_t *__restrict__ J, const
                 const bool in = s + i < e;
                 const i64 d = (i64)at * 4 + i, src = in ? s + i : (e > s ? e - 1 : e0);
                 Jm[d] = J[src];
-                for (int q = 0; q < MB_RB; ++q) cm[(d * 4 + q % 4) * 2 + q / 4] = in ? C[src * MB_RB + q] : 0.0;
+                for (int q = 0; q < rb; ++q)
+                    cm[d * rb + (rb == 16 ? q : (q % 4) * 2 + q / 4)] = in ? C[src * rb + q] : 0.0;
             }
         }
         at += nb;
@@ -375,11 +376,17 @@ __global__ __launch_bounds__(256) void k_mb(const int32_t *__restrict__ J, const
 const MfmaBlockTable *mfma_blocks(SameSpinTable &T) {
     if (T.mfma) return T.mfma.get();
     if (!T.dev_built || T.N < 1) return nullptr;
-    const RowBlockTable &R = row_blocks(T, MB_RB);
     auto M = std::make_unique<MfmaBlockTable>();
+    // blocks of 16 strings from 2,048 strings: 30% fewer gathered bytes than blocks of 8 for 1.4 times
+    // the products.  FP64 sigma, blocks of 8 / 16: 16 orbitals / 8 + 8 electrons 110.9 / 104.5 ms, 18 / 5
+    // + 5 52.7 / 50.2 ms, 14 / 7 + 7 (3,432 strings) 4.02 / 3.87 ms; but 13 / 5 + 7 (1,287 and 1,716)
+    // 0.66 / 0.71 ms, 10 / 5 + 5 36 / 40 us: there half the waves, and the slices come from L2 anyway
+    M->rb = T.N >= 2048 ? 16 : 8;
+    const bool own = M->rb == 16 && !T.blocks[2];  // blocks of 16 serve only to make these
+    const RowBlockTable &R = row_blocks(T, M->rb);
     // as many source ranges as keep the gathered slice of 128 columns about within an XCD's 4 MB L2
-    // (FP64 sigma, 16 orbitals / 8 + 8 electrons, slice 13.2 MB: 146 / 115 / 109 / 115 ms with 1 / 2 /
-    // 4 / 8 ranges; 18 orbitals / 5 + 5, 8.8 MB: 60.7 / 52.5 / 53.0 / 56.0 ms)
+    // (FP64 sigma, 16 orbitals / 8 + 8 electrons, slice 13.2 MB: 106.4 / 104.5 / 109.3 ms with 2 / 4 /
+    // 8 ranges; 18 orbitals / 5 + 5, 8.8 MB: 54.4 / 50.2 / 50.7 ms with 1 / 2 / 4)
     while (M->nr < SS_RANGES && (double)T.N * 128 * 8 > 4.5e6 * M->nr) M->nr *= 2;
     const i64 nblk = R.nblk;
     M->nblk = nblk;
@@ -387,7 +394,7 @@ const MfmaBlockTable *mfma_blocks(SameSpinTable &T) {
     cnt.alloc((size_t)nblk * 4);
     auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(256), 0, 0, R.J.as<int32_t>(), R.P.as<int32_t>(),
-                           R.c64.as<double>(), T.N, M->nr, cnt.as<int32_t>(), first.as<int32_t>(), M->P.as<int32_t>(),
+                           R.c64.as<double>(), M->rb, M->nr, cnt.as<int32_t>(), first.as<int32_t>(), M->P.as<int32_t>(),
                            M->J.as<int32_t>(), M->c64.as<double>());
         HIPOTF_CHECK(hipGetLastError());
     };
@@ -405,11 +412,12 @@ const MfmaBlockTable *mfma_blocks(SameSpinTable &T) {
     const size_t E = (size_t)t + 4 * MB_GRP;  // (the kernel reads up to 3 groups past a range's end)
     M->P.alloc((size_t)nblk * (M->nr + 1) * 4);
     M->J.alloc(E * 16);
-    M->c64.alloc(E * 4 * MB_RB * sizeof(double));
+    M->c64.alloc(E * 4 * M->rb * sizeof(double));
     HIPOTF_CHECK(hipMemset((char *)M->J.p + (size_t)t * 16, 0, 4 * MB_GRP * 16));
-    HIPOTF_CHECK(hipMemset((char *)M->c64.p + (size_t)t * 256, 0, 4 * MB_GRP * 256));
+    HIPOTF_CHECK(hipMemset((char *)M->c64.p + (size_t)t * 32 * M->rb, 0, 4 * MB_GRP * 32 * (size_t)M->rb));
     go(k_mb<true>);
     HIPOTF_CHECK(hipDeviceSynchronize());
+    if (own) T.blocks[2].reset();
     T.mfma = std::move(M);
     return T.mfma.get();
 }
