@@ -305,7 +305,9 @@ struct PairList {            // pattern within one spin: strings u with ann subs
 struct LevelPlan {
     bool ok = false;
     int nbins = 0, maxslot = 0, maxlen = 0;
-    DevBuf slots, soff, list;
+    DevBuf data;             // slots (uint2), then the pair lists (u32), then soff (int): one upload
+    size_t list_at = 0, soff_at = 0;  // their first bytes
+    template <typename T> T *at(size_t byte) const { return reinterpret_cast<T *>(data.as<unsigned char>() + byte); }
     std::vector<int> pat;    // pattern id -> row of ol, -1 if of another rank or spin
     std::vector<int2> ol;    // [row][bin]: first word in list, words
 };

@@ -1167,12 +1167,12 @@ static void sweeps(DevPool *P, i64 n, const i64 *idxs, const double *thetas, con
             a.nel = rowB ? NA : NB;
             a.nbins = s.lv->nbins;
             a.ng = s.count;
-            a.slots = s.lv->slots.as<uint2>();
-            a.soff = s.lv->soff.as<int>();
+            a.slots = s.lv->at<uint2>(0);
+            a.soff = s.lv->at<int>(s.lv->soff_at);
             a.rword = rowB ? B->pB->strs.as<u64>() : B->gaugeM.as<u64>();
             a.gens = P->lvdesc.as<LvGen>() + s.first;
             a.gstride = n;
-            a.list = s.lv->list.as<u32>();
+            a.list = s.lv->at<u32>(s.lv->list_at);
             if (back) a.partial = pend_add(s);
             const i64 nblk = (a.nunit * a.nbins + 7) / 8 * 8;
             const int np = lv_words(*s.lv, back, grad, nblk), bd = lv_threads(*s.lv, np);

@@ -500,9 +500,14 @@ static LevelPlan *level_plan(DevPool *P, int spin, bool pair, int kb) {
     if (L.maxlen > 4 * 1024) return nullptr;
     list.resize(list.size() + LV_PAD, 0u);
     HIPOTF_REQUIRE(list.size() < (1u << 29), "internal: level lists too long");
-    L.slots.upload(slots);
-    L.soff.upload(soff);
-    L.list.upload(list);
+    // (one allocation and copy: of a small pool's first pass they are most of the cost)
+    L.list_at = slots.size() * sizeof(uint2);
+    L.soff_at = L.list_at + list.size() * sizeof(u32);
+    std::vector<unsigned char> all(L.soff_at + soff.size() * sizeof(int));
+    std::memcpy(all.data(), slots.data(), L.list_at);
+    std::memcpy(all.data() + L.list_at, list.data(), list.size() * sizeof(u32));
+    std::memcpy(all.data() + L.soff_at, soff.data(), soff.size() * sizeof(int));
+    L.data.upload(all);
     L.ok = true;
     return &L;
 }
