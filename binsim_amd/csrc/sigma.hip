@@ -678,8 +678,11 @@ static void launch_mbspmm(const T *X, T *Y, const MfmaBlockTable &M, i64 nrows, 
         else if (cols == 64 || W == 4) launch_mbspmm_n<T, 4 / W, RB>(X, Y, M, nrows, ncols, st);
         else launch_mbspmm_n<T, 1, RB>(X, Y, M, nrows, ncols, st);
     };
-    if (M.rb == 16) go(std::integral_constant<int, 16>{});
-    else go(std::integral_constant<int, 8>{});
+    if constexpr (sizeof(T) == 8) {
+        if (M.rb == 16) return go(std::integral_constant<int, 16>{});
+    }
+    HIPOTF_REQUIRE(M.rb == 8, "internal: FP32 rows in blocks of 16 strings");
+    go(std::integral_constant<int, 8>{});
 }
 
 template <typename T>
@@ -689,12 +692,16 @@ static void launch_rowspmm(const T *X, T *Y, SameSpinTable &tab, const T *C, i64
     HIPOTF_REQUIRE(nrows == tab.N, "internal: same-spin table does not match the row count");
     int rb = tuning(sizeof(T) == 4).rs_block;
     if (rb == MB_RB && tuning(sizeof(T) == 4).rs_passes == 0) {  // the defaults
-        if (sizeof(T) == 8 || !fixed)
+        // FP32 without a fixed rounding (the Davidson driver's): the matrix cores below 2,048 strings
+        // (4 vectors, 12 orbitals: 173 -> 121 us per spin), blocks of 4 on the VALU from there, where
+        // the FP64 products take longer (mixed Davidson, blocks of 4: 40 iterations at 14 orbitals
+        // 0.94 s on the matrix cores, 0.89 s on the VALU; 16 iterations at 16 orbitals 7.3 / 6.6 s)
+        if (sizeof(T) == 8 || (!fixed && tab.N < 2048))
             if (const MfmaBlockTable *M = mfma_blocks(tab)) return launch_mbspmm(X, Y, *M, nrows, ncols, st);
         if constexpr (sizeof(T) == 4) {
-            // FP32 of a fixed rounding (hipotf_hvec_block): blocks of 4 strings, the same sums in
-            // the same order (FP32 sigma, 4 vectors: 12 orbitals 1.77 -> 1.67 ms, 14 orbitals
-            // 12.1 -> 11.5 ms)
+            // FP32 otherwise: blocks of 4 strings, of hipotf_hvec_block's fixed rounding: the same
+            // sums in the same order as blocks of 8 (FP32 sigma, 4 vectors: 12 orbitals 1.77 -> 1.67
+            // ms, 14 orbitals 12.1 -> 11.5 ms)
             rb = 4;
         }
     }
