@@ -216,7 +216,7 @@ __global__ __launch_bounds__(256) void k_rbspmm(const T *__restrict__ X, T *__re
 // Measured, FP64, per spin: 16 orbitals / 8 electrons 28.5 -> 24.5 (blocks of 8) -> 22.6 ms (16), 12
 // orbitals / 6 electrons 157 -> 39 us (8).  Bound by the gathered bytes (16 orbitals: blocks of 8
 // 480 GB per spin, 19.6 TB/s into the CUs, matrix cores 47% busy; of 16 335 GB) and, with blocks
-// of 16, as much by the matrix cores.  Measured and not faster: 96 or 256 columns per wave, 2
+// of 16, by the matrix cores (76% busy).  Measured and not faster: 96 or 256 columns per wave, 2
 // batches ahead, and the slices staged in LDS for 64 strings (147 GB staged instead of 480
 // gathered, but 49 ms with scalar coefficients and 76 ms on the matrix cores: too few loads in
 // flight beside the LDS buffers).  FP32, blocks of 4 vectors, 12 orbitals / 6 electrons: 173 (k_rbspmm)
