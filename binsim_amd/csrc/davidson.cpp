@@ -309,7 +309,11 @@ DavidsonOut davidson(DevHam *H, int nroots, int mode, int block, double tol, dou
                 rn[i] = ritz_and_residual(N, m, coef[i].data(), w[i], (const double *const *)V.data(),
                                           (const double *const *)AV.data(), R[i].as<double>(), st);
         }
-        for (int i = 0; i < std::min(nroots, kk); ++i) rmax = std::max(rmax, rn[i]);
+        for (int i = 0; i < std::min(nroots, kk); ++i) {
+            HIPOTF_REQUIRE(std::isfinite(rn[i]), "residual is not finite: an infinity or NaN in the guess, the "
+                                                 "integrals or the subspace");
+            rmax = std::max(rmax, rn[i]);
+        }
         for (int i = 0; i < nroots; ++i) energies[i] = w[i];  // current estimates
         out.max_residual = rmax;
         if (verbose) {  // progress goes to stderr: stdout belongs to the caller
