@@ -306,11 +306,11 @@ double dot(i64 N, const double *a, const double *b, hipStream_t st) {
 }
 
 void block_dots(i64 N, int na, const double *const *A, int nbv, const double *const *B, double *G, hipStream_t st);
-// out[j] = <V_j, a>, j < dim, written to host memory
+// out[j] = <V_j, a>, j < dim (any number), written to host memory
 void multidot(i64 N, int dim, const double *const *V, const double *a, double *out_host, hipStream_t st) {
-    HIPOTF_REQUIRE(dim >= 0 && dim <= DMAX, "subspace dimension must be in [0, 64]");
+    HIPOTF_REQUIRE(dim >= 0, "subspace dimension must not be negative");
     for (int j = 0; j < dim; ++j) HIPOTF_REQUIRE(V[j] != nullptr, "NULL subspace vector");
-    block_dots(N, dim, V, 1, &a, out_host, st);
+    for (int j = 0; j < dim; j += DMAX) block_dots(N, std::min(DMAX, dim - j), V + j, 1, &a, out_host + j, st);
 }
 
 // ------------------------------------------------------------------------------------------

@@ -3,6 +3,7 @@ import numpy as np
 import pytest
 
 from binsim_amd import davidson as D
+from binsim_amd import lib as L
 from tests.conftest import gpu_vec
 from tests.helpers import seeded_vector
 from tests.test_gpu_sigma import _dev
@@ -19,3 +20,18 @@ def test_a_guess_that_is_not_finite_is_an_error(torch_cuda, mixed, bad):
     x[7] = bad
     with pytest.raises(RuntimeError, match="finite|infinities"):
         D.solve(B, H, nroots=1, mixed=mixed, guess=gpu_vec(torch_cuda, x))
+
+
+@pytest.mark.parametrize("m", [64, 65, 130])
+def test_subspace_matrix_beyond_64_vectors(torch_cuda, m):
+    """Dot products of unit vectors of 500 elements: off by a few units of rounding, 1e-13."""
+    N, lib = 500, L.load()
+    V = np.stack([seeded_vector(N, 10 + j) for j in range(m)])
+    Vd = [gpu_vec(torch_cuda, v) for v in V]
+    t = seeded_vector(N, 5)
+    td, col, heff = gpu_vec(torch_cuda, t), np.full(m, np.nan), np.zeros(m * m)
+    lib.compute_heff_col_f64(N, m, D._pp(Vd), td.data_ptr(), col.ctypes.data_as(L._dp))
+    assert np.max(np.abs(col - V @ t)) < 1e-13
+    if m < 130:
+        lib.rebuild_heff_f64(N, m, D._pp(Vd), D._pp(Vd), heff.ctypes.data_as(L._dp), m)
+        assert np.max(np.abs(heff.reshape(m, m) - V @ V.T)) < 1e-13
