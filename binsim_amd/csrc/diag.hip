@@ -134,7 +134,8 @@ __global__ __launch_bounds__(256) void k_dotp(const double *__restrict__ a, cons
 // z . y (NORM: y . y) for the next; the rounding of every operation is that of a dot, a sum and a
 // subtraction done one after the other.  Those moved five vectors per step in three launches, this
 // moves four in one, at 6.2 TB/s (x was the z of the step before, and partly still in the Infinity
-// Cache): 20 steps on 10.3M elements 1.34 -> 1.07 ms.
+// Cache): 20 steps on 10.3M elements 1.34 -> 1.07 ms.  z may be y itself (a subspace that holds the
+// vector): then, as everywhere, its new values count.
 template <bool NORM>
 __global__ __launch_bounds__(256) void k_mgs_step(double *__restrict__ y, const double *__restrict__ x,
                                                   const double *__restrict__ z, const double *__restrict__ pin,
@@ -146,11 +147,12 @@ __global__ __launch_bounds__(256) void k_mgs_step(double *__restrict__ y, const 
     if (threadIdx.x == 0) ps = s;
     __syncthreads();
     const double p = ps;
+    const bool own = NORM || z == y;
     double acc = 0.0;
     stream_for(n, [&](i64 i) {
-        const double v = y[i] - p * x[i];
+        const double zv = NORM ? 0.0 : z[i], v = y[i] - p * x[i];
         y[i] = v;
-        acc += NORM ? v * v : z[i] * v;
+        acc += (own ? v : zv) * v;
     });
     const double t = block_sum_d(acc);
     if (threadIdx.x == 0) pout[blockIdx.x] = t;
