@@ -445,16 +445,28 @@ static LevelPlan *level_plan(DevPool *P, int spin, bool pair, int kb) {
     std::stable_sort(bl.begin(), bl.end(), [](const auto &a, const auto &b) { return a.size() > b.size(); });
     if (bl.empty() || (i64)bl[0].size() > lv_cap(false)) return nullptr;
     // bins: largest blocks first, smaller ones added while a bin stays within 5/4 of the largest
-    // block (a bin of a few elements takes as long per generator as a full one) and the LDS
+    // block (a bin of a few elements takes as long per generator as a full one) and the LDS.  The
+    // blocks of a pool on a window of the orbitals hold a few elements each: where that makes more
+    // workgroups than the chip holds at a time, bins of 512 elements (14 orbitals / 7 + 7, excitations
+    // among orbitals 4 to 9, forward: 6.04 ms; 0.85 / 0.75 / 0.76 / 0.78 ms with 256 / 512 / 1024 / 2048.
+    // Not in small spaces: 10 orbitals / 4 + 6, energy and gradient 0.91 -> 0.98 ms)
     const i64 big = (i64)bl[0].size(), capb = lv_cap(big <= lv_cap(true));
-    const i64 cap = std::min(capb, big + big / 4);
+    i64 cap = big + big / 4, held = 0;
+    for (const auto &v : bl) held += (i64)v.size();
+    if ((spin == 0 ? hb.B : hb.A).N * (held / cap) > 2048) cap = std::max<i64>(cap, 512);
+    cap = std::min(cap, capb);
     std::vector<std::vector<u32>> bins;
+    std::vector<int> blocks_of;
     for (auto &v : bl) {
         size_t b = 0;
         while (b < bins.size() && (i64)(bins[b].size() + v.size()) > cap) ++b;
-        if (b == bins.size()) bins.emplace_back();
+        if (b == bins.size()) bins.emplace_back(), blocks_of.push_back(0);
         bins[b].insert(bins[b].end(), v.begin(), v.end());
+        ++blocks_of[b];
     }
+    // (many small blocks: in the order of the rows and elements, for coalesced loads)
+    for (size_t b = 0; b < bins.size(); ++b)
+        if (blocks_of[b] > 8) std::sort(bins[b].begin(), bins[b].end());
     L.nbins = (int)bins.size();
     // slot of an element: [row side][element]
     std::vector<int> bin_of[2], loc[2];
