@@ -890,8 +890,10 @@ static size_t seg_lds_budget() {
 
 // group the sweep (generator indices in order) into fusable segments; nvec rows per element
 // (1 for the forward expm sweep, 2 for the adjoint sweep) decide what fits LDS.  il: the
-// adjoint sweep's pair segments on interleaved (l, r) rows (two rows of 16-byte elements)
-static std::vector<Segment> plan_sweep(DevPool *P, const i64 *idxs, i64 n, int nvec, bool il = false) {
+// adjoint sweep's pair segments on interleaved (l, r) rows (two rows of 16-byte elements); grad: the
+// gradient-only pass
+static std::vector<Segment> plan_sweep(DevPool *P, const i64 *idxs, i64 n, int nvec, bool il = false,
+                                       bool grad = false) {
     const DevBasis *B = P->basis;
     const i64 NA = B->pA->N, NB = B->pB->N;
     const size_t budget = seg_lds_budget();
@@ -947,34 +949,72 @@ static std::vector<Segment> plan_sweep(DevPool *P, const i64 *idxs, i64 n, int n
             segs.push_back(s);
             continue;
         }
-        // runs of one rank of the moved spin that fit the LDS level by level; what does not stays
-        // on the segment's own form
-        const bool pair = s.kind == SEG_PAIR;
+        // runs of one rank of the moved spin on excitation levels (rot_levels.hpp), where they fit and
+        // are long enough to pay for their loads by slot; the rest on the segment's own form
+        const bool pair = s.kind == SEG_PAIR, back = nvec == 2;
         const int spin = s.kind == SEG_ROW_B ? 0 : 1;
+        const i64 nel = spin == 0 ? NA : NB;
         auto rank = [&](i64 j) {
             return __builtin_popcountll(P->lists[spin == 0 ? gen(j).pa : gen(j).pb].cre);
         };
-        auto plan_of = [&](int k) -> LevelPlan * {
-            LevelPlan *lp = k > 0 ? level_plan(P, spin, pair, k) : nullptr;
-            return lp && (nvec == 1 || (lp->maxslot <= lv_cap(true) && lp->maxlen <= 2048)) ? lp : nullptr;
-        };
+        std::vector<Segment> runs;
+        int moved = 0, nzero = 0;
         for (i64 j = s.first, end = s.first + s.count; j < end;) {
-            const int k = rank(j);
             Segment t = s;
             t.first = (int)j;
             t.count = 1;
-            LevelPlan *lp = plan_of(k);
+            const int k = rank(j);
             if (pair && k == 0) {
                 t.kind = SEG_LV0;
-            } else if (lp) {
+                ++nzero;
+            } else {
+                while (j + t.count < end && rank(j + t.count) == k) ++t.count;
+                moved += t.count;
+            }
+            runs.push_back(t);
+            j += t.count;
+        }
+        // A pair segment goes either way as a whole: on levels an alpha single (rank 0) is a launch of
+        // its own, and the segment's adjoint form holds (l, r) interleaved.  Generators that pay for a
+        // run, at 8, 10, 12, 14 and 16 orbitals: adjoint 1, 1, 1, 1, 2; forward 1, 3, 4, 2, 3; with an
+        // alpha single adjoint 2, 3, 6, 2, 4 and forward 4, 6, 8, 3, 7.  The gradient-only pass has no
+        // generator after generator to wait for: always
+        const int nrun = (int)runs.size() - nzero;
+        bool all = !pair || (nrun > 0 && (grad || moved >= (back ? nrun + 3 * nzero : 3 * nrun + 5 * nzero)));
+        const i64 units = pair ? P->lists[s.pa].len : (spin == 0 ? NB : NA);
+        auto longest = [&](const LevelPlan &lp) -> i64 {  // generators per launch
+            return back ? LV_PART / std::max<i64>(1, units * lp.nbins) : 4096;
+        };
+        for (Segment &t : runs) {
+            if (!all) break;
+            if (t.kind == SEG_LV0) continue;
+            const int k = rank(t.first);
+            // rows: run lengths that pay at 8, 10, 12, 14 and 16 orbitals: adjoint 1, 1, 1, 1, 8; forward
+            // singles 4, 5, 8, 6, -, doubles 3, 4, 8, 20, 4
+            if (!pair && !grad && t.count < (back ? (nel <= lv_cap(true) ? 1 : 8) : (k == 1 ? 8 : 16))) continue;
+            LevelPlan *lp = level_plan(P, spin, pair, k);
+            const bool fits = lp && !(back && (lp->maxslot > lv_cap(true) || lp->maxlen > 2048)) &&
+                              longest(*lp) >= 16 && units * lp->nbins < 1ll << 22;  // (less than 2^32 threads)
+            if (fits) {
                 t.kind = pair ? SEG_LV_PAIR : (spin == 0 ? SEG_LV_ROW_B : SEG_LV_ROW_A);
                 t.lv = lp;
-                while (j + t.count < end && rank(j + t.count) == k) ++t.count;
-            } else {
-                while (j + t.count < end && rank(j + t.count) > 0 && !plan_of(rank(j + t.count))) ++t.count;
+            } else if (pair) {
+                all = false;
             }
-            segs.push_back(t);
-            j += t.count;
+        }
+        if (!all) {  // (a generalised pool, whose runs have no plan, at 14 orbitals: energy and gradient
+            segs.push_back(s);  // 34.6 ms with the alpha singles split off, 19.4 without)
+            continue;
+        }
+        for (size_t q = 0; q < runs.size();) {
+            Segment t = runs[q++];
+            if (!pair && !t.lv)  // neighbours on the segment's form go together
+                for (; q < runs.size() && !runs[q].lv; ++q) t.count += runs[q].count;
+            const int most = t.lv ? (int)std::min<i64>(t.count, longest(*t.lv)) : t.count;
+            for (int left = t.count; left > 0; left -= t.count, t.first += t.count) {
+                t.count = std::min(left, most);
+                segs.push_back(t);
+            }
         }
     }
     return segs;
@@ -1120,7 +1160,7 @@ static void sweeps(DevPool *P, i64 n, const i64 *idxs, const double *thetas, con
                     cap = std::max(cap, need);
                     tot += need;
                 }
-            cap = std::max(cap, std::min<i64>(tot, 32ll << 20));
+            cap = std::max(cap, std::min<i64>(tot, LV_PART));
             if (cap) P->lvpart.ensure(cap * sizeof(double));
         }
         LvPend pend{};
@@ -1386,7 +1426,7 @@ static void sweeps(DevPool *P, i64 n, const i64 *idxs, const double *thetas, con
         if (back) pend_flush();
     };
     if (grad) {
-        run(plan_sweep(P, idxs, n, 2), true, false);
+        run(plan_sweep(P, idxs, n, 2, false, true), true, false);
         return;
     }
     if (forward) run(plan_sweep(P, idxs, n, 1), false, false);

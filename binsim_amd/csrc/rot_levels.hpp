@@ -32,6 +32,7 @@
 
 constexpr int LV_SLOT_BITS = 14;
 constexpr int LV_PAD = 4096; // words after the last list that idle threads may read
+constexpr i64 LV_PART = 32ll << 20;  // gradient partials that one launch may write (256 MB)
 constexpr int LV_RED = 64;  // generators between two flushes of the gradient sums
 
 struct LvGen {              // one generator as one bin sees it

@@ -1,8 +1,10 @@
-"""Rotation runs on excitation levels (csrc/rot_levels.hpp) against one launch per generator
-(sweep_mode 2): pools on a window of the orbitals (blocks of a few elements, many to a bin).
+"""Which rotation runs go to excitation levels (csrc/rot.hip plan_sweep, csrc/rot_levels.hpp), against
+one launch per generator (sweep_mode 2): pools on a window of the orbitals (blocks of a few elements,
+many to a bin), run lengths on both sides of the rules, alpha singles in segments with and without a
+plan, and runs cut where their gradient partials would pass the limit.
 
 Tolerance: m rotations in another order of additions differ by a few m units of rounding relative to
-the norm 1; 1e-12 covers m up to 1,000 with a factor of 4."""
+the norm 1; 1e-12 covers m up to 1,000 with a factor of 4, 4e-12 the 2,352 of the longest case."""
 import time
 
 import numpy as np
@@ -26,6 +28,12 @@ def _functions(n, na, nb, sos):
 
 def _window(n, na, nb, lo, hi):
     return [so for so in ucc_spin_orbitals(n, na, nb) if all(lo <= p // 2 < hi for p in so)]
+
+
+def _spins(so):
+    """(alpha, beta) excitation ranks"""
+    a = sum(p % 2 == 0 for p in so) // 2
+    return a, len(so) // 2 - a
 
 
 def _compare(torch, n, na, nb, sos, modes=(0, 4), tol=1e-12):
@@ -60,6 +68,38 @@ def test_pools_on_a_window_of_the_orbitals(torch_cuda, n, na, nb, lo, hi):
     sos = _window(n, na, nb, lo, hi)
     assert sos
     _compare(torch_cuda, n, na, nb, sos[:120] + sos[120:][-120:])
+
+
+@pytest.mark.parametrize("m", [1, 2, 3, 7, 8, 9, 15, 16, 17])
+@pytest.mark.parametrize("n,na,nb", [(8, 4, 4), (9, 3, 4)])
+def test_run_lengths_around_the_rules(torch_cuda, n, na, nb, m):
+    """m beta excitations of one rank after each alpha single, with and without the alpha single
+    itself, and m of one spin alone between others."""
+    u = ucc_spin_orbitals(n, na, nb)
+    sos = []
+    for p in [so for so in u if _spins(so) == (1, 0)][:4]:
+        mixed = [so for so in u if _spins(so) == (1, 1) and so[0] == p[0] and so[2] == p[1]]
+        sos += [p] + mixed[:m] + [so for so in u if _spins(so) == (0, 2)][:m] + mixed[-m:]
+        sos += [so for so in u if _spins(so) == (0, 1)][:m] + [so for so in u if _spins(so) == (2, 0)][:m]
+    _compare(torch_cuda, n, na, nb, sos[:240])
+
+
+def test_alpha_singles_of_a_generalised_pool(torch_cuda):
+    """Alpha singles before mixed generators that have no level plan."""
+    n = 7
+    sos = []
+    for p in range(1, 4):
+        sos.append([2 * p, 0])
+        sos += [[2 * p, 2 * r + 1, 0, 2 * t + 1] for r in range(n) for t in range(r)]
+    sos += [[2 * p + 1, 2 * q + 1] for p in range(n) for q in range(p)]
+    _compare(torch_cuda, n, 3, 3, sos)
+
+
+def test_run_longer_than_its_gradient_partials_allow(torch_cuda):
+    """8,008 rows in two bins: at most 2,095 generators to a launch."""
+    doubles = [so for so in ucc_spin_orbitals(16, 6, 8) if _spins(so) == (0, 2)]
+    assert len(doubles) == 784
+    _compare(torch_cuda, 16, 6, 8, doubles * 3, modes=(4,), tol=4e-12)
 
 
 @pytest.mark.parametrize("lo,hi", [(6, 8), (5, 9)])
