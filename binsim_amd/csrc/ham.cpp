@@ -130,23 +130,21 @@ static void build_same_spin(SameSpinTable &T, const SpinSpace &S, const std::vec
     T.hC = std::move(C);
 }
 
-const RowBlockTable &row_blocks(SameSpinTable &T, int rb) {
+const RowBlockTable &row_blocks(SameSpinTable &T, int rb, int prec) {
     HIPOTF_REQUIRE(rb == 4 || rb == 8 || rb == 16, "row block size must be 4, 8 or 16");
     const int slot = rb == 4 ? 0 : (rb == 8 ? 1 : 2);
-    if (T.blocks[slot]) return *T.blocks[slot];
+    if (T.blocks[prec][slot]) return *T.blocks[prec][slot];
     if (T.dev_built) {
         auto R = std::make_unique<RowBlockTable>();
-        row_blocks_dev(T, *R, rb);
-        T.blocks[slot] = std::move(R);
-        return *T.blocks[slot];
+        row_blocks_dev(T, *R, rb, prec);
+        T.blocks[prec][slot] = std::move(R);
+        return *T.blocks[prec][slot];
     }
+    // from the host's tables: both precisions at once (the unions are the cost)
     const i64 N = T.N;
     const size_t L = T.L;
     HIPOTF_REQUIRE(T.hJ.size() == (size_t)N * L, "internal: same-spin host table missing");
-    auto R = std::make_unique<RowBlockTable>();
-    R->rb = rb;
-    R->nblk = (N + rb - 1) / rb;
-    const i64 nblk = R->nblk;
+    const i64 nblk = (N + rb - 1) / rb;
     // the ascending, duplicate-free union of the sources of rows [g*rb, g*rb + rb)
     auto block_union = [&](i64 g, std::vector<int32_t> &u) {
         const i64 r0 = g * rb, r1 = std::min<i64>(N, r0 + rb);
@@ -163,7 +161,6 @@ const RowBlockTable &row_blocks(SameSpinTable &T, int rb) {
     for (i64 g = 0; g < nblk; ++g) off[g + 1] += off[g];
     const i64 E = off[nblk];
     HIPOTF_REQUIRE(E < (1ll << 31), "row-block table too large for 32-bit offsets");
-    R->entries = E;
     std::vector<int32_t> J((size_t)E);
     std::vector<double> C((size_t)E * rb, 0.0);
     std::vector<int32_t> P((size_t)nblk * (SS_RANGES + 1));
@@ -185,13 +182,17 @@ const RowBlockTable &row_blocks(SameSpinTable &T, int rb) {
             P[(size_t)g * (SS_RANGES + 1) + rg] = (int32_t)(off[g] + (i64)pos);
         }
     });
-    R->J.upload(J);
-    R->P.upload(P);
-    R->c64.upload(C);
-    std::vector<float> C32(C.begin(), C.end());
-    R->c32.upload(C32);
-    T.blocks[slot] = std::move(R);
-    return *T.blocks[slot];
+    for (int q = 0; q < 2; ++q) {
+        auto R = std::make_unique<RowBlockTable>();
+        R->rb = rb;
+        R->nblk = nblk;
+        R->J.upload(J);
+        R->P.upload(P);
+        if (q == 0) R->c.upload(C);
+        else R->c.upload(std::vector<float>(C.begin(), C.end()));
+        T.blocks[q][slot] = std::move(R);
+    }
+    return *T.blocks[prec][slot];
 }
 
 // Determinants as interleaved spin-orbital occupations: bit 2p = alpha p, bit 2p+1 = beta p
@@ -327,21 +328,17 @@ DevHam *make_dev_ham(DevBasis *b, int n, const std::vector<double> &h, const std
             build_same_spin(H->tB, hb.B, H->h, H->eri, n);
         H->ptB = &H->tB;
     }
-    // the default row blocks now, so that the first sigma does not pay for them
-    for (int prec = 0; prec < 2; ++prec) {
-        const int rb = tuning(prec).rs_block;
-        // the matrix-core tables in FP64; FP32 has blocks of 4, built when used.  The blocks of 8
-        // beside them where hipotf_hvec_noalloc, which builds none, may be called with other passes
-        const bool mb = rb == MB_RB && tuning(prec).rs_passes == 0, small = hb.dim <= NOALLOC_MAX_DIM;
-        if (prec == 0 && (mb || (rb == MB_RB && small))) {
-            mfma_blocks(*H->ptA);
-            mfma_blocks(*H->ptB);
+    // the row tables of the chosen forms now, so that the first sigma does not pay for them (the
+    // default's FP32 blocks of 4 when an FP32 sigma first needs them); where hipotf_hvec_noalloc,
+    // which builds none, may be called with other choices later, the matrix-core tables too
+    for (SameSpinTable *T : {H->ptA, H->ptB}) {
+        for (int prec = 0; prec < 2; ++prec) {
+            const int rb = tuning(prec).rs_block;
+            const bool mb = rb == MB_RB && tuning(prec).rs_passes == 0 && T->dev_built;
+            if (mb && prec == 0) mfma_blocks(*T);
+            if (!mb && (rb == 4 || rb == 8 || rb == 16)) row_blocks(*T, rb, prec);
         }
-        if (mb && !small && H->tA.dev_built && H->ptB->dev_built) continue;
-        if (rb == 4 || rb == 8 || rb == 16) {
-            row_blocks(*H->ptA, rb);
-            row_blocks(*H->ptB, rb);
-        }
+        if (hb.dim <= NOALLOC_MAX_DIM) mfma_blocks(*T);
     }
     build_jab_dev(H->jab, *b->pA, n, H->eri64);
     return H.release();

@@ -161,21 +161,21 @@ constexpr int SS_RANGES = 8;  // source-index ranges the same-spin rows are spli
 struct RowBlockTable {
     int rb = 0;
     i64 nblk = 0;             // ceil(N / rb)
-    i64 entries = 0;
-    DevBuf J;                 // int32[entries]: sources of block 0, then block 1, ...
+    DevBuf J;                 // int32[entries]: sources of block 0, block 1, ... (gaps between blocks
+                              // are not read)
     DevBuf P;                 // int32[nblk][SS_RANGES + 1]: entry offset (absolute) of the
                               // first source >= g * N / SS_RANGES; P[.][SS_RANGES] = block end
-    DevBuf c64, c32;          // double / float [entries][rb]
+    DevBuf c;                 // double or float [entries][rb]
 };
 
 // the row blocks of 8 or 16 strings in MFMA-operand order for the FP64 matrix-core row SpMM
 // (k_mbspmm): each block's sources in nr source ranges, each range padded to whole groups of
-// MB_GRP batches of 4 sources (coefficient 0, a valid source)
+// MB_GRP batches of 4 sources (coefficient 0, a valid source), and two groups after the last
 constexpr int MB_RB = 8, MB_GRP = 4;
 struct MfmaBlockTable {
     int rb = MB_RB;           // strings per block: 8 or 16
     int nr = 1;               // source ranges: passes of the kernel
-    i64 nblk = 0, batches = 0;
+    i64 nblk = 0;
     DevBuf P;                 // int32[nblk][nr + 1]: first batch of each range, end
     DevBuf J;                 // int32[batches][4]: sources
     DevBuf c64;               // rb 8: double[batches][4 sources][4][2]: coefficients of rows i and
@@ -193,17 +193,17 @@ struct SameSpinTable {
     std::vector<int32_t> hJ;  // host copies of J and the FP64 coefficients when the table was
     std::vector<double> hC;   // built on the host (row blocks are then built from them)
     bool dev_built = false;   // built on the device (tables.hip): row blocks too
-    std::unique_ptr<RowBlockTable> blocks[3];  // rb = 4, 8, 16
+    std::unique_ptr<RowBlockTable> blocks[2][3];  // [FP64, FP32][rb = 4, 8, 16]
     std::unique_ptr<MfmaBlockTable> mfma;
 };
 
-// row-block table of T for rb in {4, 8, 16}, built (and uploaded) on first use
-const RowBlockTable &row_blocks(SameSpinTable &T, int rb);
+// row-block table of T for rb in {4, 8, 16} and a precision, built (and uploaded) on first use
+const RowBlockTable &row_blocks(SameSpinTable &T, int rb, int prec);
 // device construction (tables.hip): false when a row is too long for its in-LDS sort (then the
 // host build applies)
 struct DevSpin;
 bool build_same_spin_dev(SameSpinTable &T, const DevSpin &S, const DevBuf &h64, const DevBuf &eri64, int n);
-void row_blocks_dev(SameSpinTable &T, RowBlockTable &R, int rb);
+void row_blocks_dev(SameSpinTable &T, RowBlockTable &R, int rb, int prec);
 // matrix-core row-SpMM table of T, built on first use; NULL for tables built on the host
 const MfmaBlockTable *mfma_blocks(SameSpinTable &T);
 void build_jab_dev(DevBuf &jab, const DevSpin &A, int n, const DevBuf &eri64);

@@ -619,7 +619,7 @@ static void launch_rbspmm_c(const T *X, T *Y, const RowBlockTable &rt, i64 nrows
     const i64 nwork = ntiles * rt.nblk;
     const i64 per_xcd = (nwork + 7) / 8;
     HIPOTF_REQUIRE(per_xcd * 8 < (1ll << 31), "row-block SpMM grid too large");
-    const T *C = sizeof(T) == 4 ? (const T *)rt.c32.p : (const T *)rt.c64.p;
+    const T *C = rt.c.as<T>();
     for (int p = 0; p < npass; ++p)
         hipLaunchKernelGGL((k_rbspmm<T, RB, CPL>), dim3((unsigned)(per_xcd * 8)), dim3(256), 0, st, X, Y,
                            rt.J.as<int32_t>(), rt.P.as<int32_t>(), C, nrows, ncols, rt.nblk, nwork,
@@ -699,15 +699,19 @@ static void launch_rowspmm(const T *X, T *Y, SameSpinTable &tab, const T *C, i64
         if (sizeof(T) == 8 || (!fixed && tab.N < 2048))
             if (const MfmaBlockTable *M = mfma_blocks(tab)) return launch_mbspmm(X, Y, *M, nrows, ncols, st);
         if constexpr (sizeof(T) == 4) {
-            // FP32 otherwise: blocks of 4 strings, of hipotf_hvec_block's fixed rounding: the same
-            // sums in the same order as blocks of 8 (FP32 sigma, 4 vectors: 12 orbitals 1.77 -> 1.67
-            // ms, 14 orbitals 12.1 -> 11.5 ms)
-            rb = 4;
+            // FP32 otherwise: blocks of 4 strings, the same sums in the same order as blocks of 8 (FP32
+            // sigma, 4 vectors: 12 orbitals 1.77 -> 1.67 ms, 14 orbitals 12.1 -> 11.5 ms).  Tables from
+            // the host have the blocks of 8 in both precisions, and another set costs seconds
+            if (tab.dev_built) rb = 4;
         }
     }
+    // an allocation-free call with other passes than at its preparation: the matrix-core tables
+    if constexpr (sizeof(T) == 8)
+        if (rb == MB_RB && g_forbid_alloc && !tab.blocks[0][1] && tab.mfma)
+            return launch_mbspmm(X, Y, *tab.mfma, nrows, ncols, st);
     if (rb == 4 || rb == 8 || rb == 16) {
         const int npass = rs_npass<T>(nrows, 256 * rs_cpl<T>(ncols));
-        const RowBlockTable &rt = row_blocks(tab, rb);
+        const RowBlockTable &rt = row_blocks(tab, rb, sizeof(T) == 4);
         if (rb == 4) launch_rbspmm<T, 4>(X, Y, rt, nrows, ncols, npass, st);
         else if (rb == 8) launch_rbspmm<T, 8>(X, Y, rt, nrows, ncols, npass, st);
         else launch_rbspmm<T, 16>(X, Y, rt, nrows, ncols, npass, st);

@@ -6,7 +6,7 @@
 // build_same_spin forms them from h_pq and (pq|rs)), its source strings as colex ranks, the row
 // sorted by source in LDS; then the row-block tables of the same-spin SpMM -- per block of rb
 // consecutive strings the ascending union of their sources and an rb-wide coefficient column per
-// union entry -- with the union sorted in LDS.  Replaces the host construction of
+// union entry -- with the union as a bit set in LDS.  Replaces the host construction of
 // src/include/ham/ham.hpp:635-996 / :998-1069 (JW terms and SVD groups) with a direct build.
 #include "hipotf.hpp"
 
@@ -163,68 +163,101 @@ __global__ __launch_bounds__(256) void k_ss_rows(const u64 *__restrict__ strs, i
         P[I * (SS_RANGES + 1) + tid] = tid == SS_RANGES ? L : tb_lower(key, L, (i64)tid * N / SS_RANGES);
 }
 
-// per block of rb rows: the ascending union of their sources.  FILL = false: its size into
-// cnt[g]; FILL = true: the union into Jr[off[g]..], the rb-wide coefficient columns and the
-// range offsets.  LP (power of two) >= rb * L keys in LDS.
-template <bool FILL>
+// The set of sources of a block of rows, in LDS: a bit per string, and the count of bits before each
+// 256 (ascending order and positions come from the bits: no sort)
+struct TbSet {
+    u32 *bits;   // [8 groups]
+    int *pre;    // [groups + 1]
+    int groups;
+};
+static int tb_groups(i64 N) { return (int)((N + 255) / 256); }
+static size_t tb_set_bytes(i64 N) { return ((size_t)tb_groups(N) * 9 + 1 + 16) * 4; }
+
+// number of members below x
+__device__ __forceinline__ int tb_below(const TbSet &s, i64 x) {
+    if (x >= (i64)s.groups * 256) return s.pre[s.groups];
+    const int g = (int)(x >> 8), w1 = (int)(x >> 5);
+    int p = s.pre[g];
+    for (int w = g * 8; w < w1; ++w) p += __popc(s.bits[w]);
+    return p + __popc(s.bits[w1] & ((1u << (x & 31)) - 1));
+}
+
+// the set of J[0..m), by the whole workgroup
+__device__ TbSet tb_union(u32 *lds, const int32_t *__restrict__ J, int m, i64 N) {
+    const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wave = tid >> 6, G = (int)((N + 255) / 256);
+    TbSet s{lds, reinterpret_cast<int *>(lds + 8 * G), G};
+    int *wsum = s.pre + G + 1;  // up to 16 waves
+    for (int i = tid; i < 8 * G; i += nt) s.bits[i] = 0;
+    __syncthreads();
+    for (int i = tid; i < m; i += nt) {
+        const int j = J[i];
+        atomicOr(&s.bits[j >> 5], 1u << (j & 31));
+    }
+    __syncthreads();
+    auto count = [&](int g) {
+        int c = 0;
+        for (int w = 0; w < 8; ++w) c += __popc(s.bits[g * 8 + w]);
+        return c;
+    };
+    const int per = (G + nt - 1) / nt, g0 = min(G, tid * per), g1 = min(G, g0 + per);
+    int mine = 0;
+    for (int g = g0; g < g1; ++g) mine += count(g);
+    int x = mine;  // inclusive scan over the wave, then over the waves
+    for (int d = 1; d < 64; d <<= 1) {
+        const int y = __shfl_up(x, d, 64);
+        if (lane >= d) x += y;
+    }
+    if (lane == 63) wsum[wave] = x;
+    __syncthreads();
+    int at = x - mine;
+    for (int w = 0; w < wave; ++w) at += wsum[w];
+    for (int g = g0; g < g1; ++g) {
+        s.pre[g] = at;
+        at += count(g);
+    }
+    if (tid == nt - 1) s.pre[G] = at;
+    __syncthreads();
+    return s;
+}
+
+// f(position, member) for every member, ascending positions
+template <typename F>
+__device__ __forceinline__ void tb_members(const TbSet &s, F &&f) {
+    for (int w = threadIdx.x; w < 8 * s.groups; w += blockDim.x) {
+        u32 v = s.bits[w];
+        int p = v ? tb_below(s, (i64)w * 32) : 0;
+        for (; v; v &= v - 1) f(p++, w * 32 + __builtin_ctz(v));
+    }
+}
+
+// per block of rb rows: the ascending union of their sources.  FILL = false: its size into cnt[g];
+// FILL = true: the union into Jr[o..], the rb-wide coefficient columns and the range offsets, with
+// o = off[g], or g * stride without a count
+template <bool FILL, typename T>
 __global__ __launch_bounds__(1024) void k_rb_union(const int32_t *__restrict__ J, const double *__restrict__ c64,
-                                                   i64 N, int L, int rb, int LP, int32_t *__restrict__ cnt,
-                                                   const i64 *__restrict__ off, int32_t *__restrict__ Jr,
-                                                   double *__restrict__ cr64, float *__restrict__ cr32,
-                                                   int32_t *__restrict__ Pr) {
-    extern __shared__ int lds[];
-    int *key = lds;              // LP keys
-    int *tsum = lds + LP;        // per-thread unique counts, then their exclusive scan
+                                                   i64 N, int L, int rb, int32_t *__restrict__ cnt,
+                                                   const i64 *__restrict__ off, i64 stride, int32_t *__restrict__ Jr,
+                                                   T *__restrict__ cr, int32_t *__restrict__ Pr) {
+    extern __shared__ u32 lds[];
     const int tid = threadIdx.x, nt = blockDim.x;
     const i64 g = blockIdx.x, r0 = g * rb, r1 = r0 + rb < N ? r0 + rb : N;
     const int m = (int)((r1 - r0) * L);
-    for (int i = tid; i < LP; i += nt) key[i] = i < m ? J[r0 * L + i] : INT_MAX;
-    __syncthreads();
-    tb_bitonic<false, int>(key, nullptr, LP, tid, nt);
-    // each thread owns a contiguous chunk of the sorted keys
-    const int per = LP / nt, c0 = tid * per;
-    int mine[32];
-    int u = 0;
-    for (int i = 0; i < per; ++i) {
-        const int x = key[c0 + i];
-        const bool first = x != INT_MAX && (c0 + i == 0 || key[c0 + i - 1] != x);
-        mine[i] = first ? x : INT_MAX;
-        u += first ? 1 : 0;
-    }
-    tsum[tid] = u;
-    __syncthreads();
-    if (tid == 0) {
-        int acc = 0;
-        for (int t = 0; t < nt; ++t) {
-            const int c = tsum[t];
-            tsum[t] = acc;
-            acc += c;
-        }
-        tsum[nt] = acc;
-    }
-    __syncthreads();
-    const int U = tsum[nt];
+    const TbSet s = tb_union(lds, J + r0 * L, m, N);
+    const int U = s.pre[s.groups];
     if (!FILL) {
         if (tid == 0) cnt[g] = U;
         return;
     }
-    // compact the union in place (every thread has read its chunk before the barrier above)
-    int pos = tsum[tid];
-    for (int i = 0; i < per; ++i)
-        if (mine[i] != INT_MAX) key[pos++] = mine[i];
+    const i64 o = stride ? g * stride : off[g];
+    tb_members(s, [&](int p, int j) { Jr[o + p] = j; });
+    for (int i = tid; i < U * rb; i += nt) cr[o * rb + i] = T(0);
     __syncthreads();
-    const i64 o = off[g];
-    for (int i = tid; i < U; i += nt) Jr[o + i] = key[i];
     for (int i = tid; i < m; i += nt) {
-        const int row = i / L;
         const i64 src = r0 * L + i;
-        const int p = tb_lower(key, U, J[src]);
-        cr64[(o + p) * rb + row] = c64[src];
-        cr32[(o + p) * rb + row] = (float)c64[src];
+        cr[(o + tb_below(s, J[src])) * rb + i / L] = (T)c64[src];
     }
     if (tid <= SS_RANGES)
-        Pr[g * (SS_RANGES + 1) + tid] =
-            (int32_t)(o + (tid == SS_RANGES ? U : tb_lower(key, U, (i64)tid * N / SS_RANGES)));
+        Pr[g * (SS_RANGES + 1) + tid] = (int32_t)(o + (tid == SS_RANGES ? U : tb_below(s, (i64)tid * N / SS_RANGES)));
 }
 
 // single-excitation table of one spin: sx[slot][I], slot = io (n - k) + iv, r = io-th occupied and
@@ -300,76 +333,122 @@ bool build_same_spin_dev(SameSpinTable &T, const DevSpin &S, const DevBuf &hdev,
     return true;
 }
 
-void row_blocks_dev(SameSpinTable &T, RowBlockTable &R, int rb) {
-    const i64 N = T.N, nblk = (N + rb - 1) / rb;
-    const int L = T.L;
-    int LP = 1024;
-    while (LP < rb * L) LP <<= 1;
-    HIPOTF_REQUIRE(LP <= 32768, "internal: row block too long for the in-LDS union");
-    const size_t smem = ((size_t)LP + 1024 + 1) * sizeof(int);
-    DevBuf cnt, off;
-    cnt.alloc((size_t)nblk * sizeof(int32_t));
-    HIPOTF_CHECK(hipFuncSetAttribute((const void *)k_rb_union<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     (int)smem));
-    HIPOTF_CHECK(hipFuncSetAttribute((const void *)k_rb_union<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     (int)smem));
-    hipLaunchKernelGGL(k_rb_union<false>, dim3((unsigned)nblk), dim3(1024), smem, 0, T.J.as<int32_t>(),
-                       T.c64.as<double>(), N, L, rb, LP, cnt.as<int32_t>(), nullptr, nullptr, nullptr, nullptr,
-                       nullptr);
+// Launch of a table kernel, one workgroup per row block.  (1024 threads where a block has many
+// entries to place; LDS: the bits of the N strings, 144 KB at the limit of 2^20)
+template <typename K, typename... Args>
+static void launch_blocks(K kern, i64 nblk, i64 N, i64 entries, Args... args) {
+    const size_t smem = tb_set_bytes(N);
+    if (smem > 48 * 1024)
+        HIPOTF_CHECK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
+    hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(entries > 4096 ? 1024 : 256), smem, 0, args...);
     HIPOTF_CHECK(hipGetLastError());
-    std::vector<int32_t> hc(nblk);
-    HIPOTF_CHECK(hipMemcpy(hc.data(), cnt.p, (size_t)nblk * sizeof(int32_t), hipMemcpyDeviceToHost));
-    std::vector<i64> ho(nblk + 1, 0);
-    for (i64 g = 0; g < nblk; ++g) ho[g + 1] = ho[g] + hc[g];
-    const i64 E = ho[nblk];
-    HIPOTF_REQUIRE(E < (1ll << 31), "row-block table too large for 32-bit offsets");
-    off.upload(ho);
+}
+
+// Sizes of the blocks' parts of a table, as first places and the total: counted on the device, or,
+// where all blocks at their largest take no more than 16 MB, that many each without a count (a
+// count, its two copies and their waits are most of the time of a small table)
+struct TbPlaces {
+    i64 stride = 0, total = 0;
+    std::vector<i64> first;
+};
+template <typename K>
+static TbPlaces tb_places(i64 nblk, i64 most, size_t bytes_each, K &&count) {
+    TbPlaces p;
+    if ((size_t)nblk * most * bytes_each <= 16u << 20) {
+        p.stride = most;
+        p.total = nblk * most;
+        return p;
+    }
+    DevBuf cnt((size_t)nblk * sizeof(int32_t));
+    count(cnt.as<int32_t>());
+    std::vector<int32_t> h(nblk);
+    HIPOTF_CHECK(hipMemcpy(h.data(), cnt.p, (size_t)nblk * sizeof(int32_t), hipMemcpyDeviceToHost));
+    p.first.resize(nblk);
+    for (i64 g = 0; g < nblk; ++g) {
+        p.first[g] = p.total;
+        p.total += h[g];
+    }
+    return p;
+}
+
+template <typename T>
+static void row_blocks_t(SameSpinTable &S, RowBlockTable &R, int rb) {
+    const i64 N = S.N, nblk = (N + rb - 1) / rb, most = std::min<i64>(N, (i64)rb * S.L);
+    const int32_t *J = S.J.as<int32_t>();
+    const double *c = S.c64.as<double>();
+    const TbPlaces p = tb_places(nblk, most, 4 + rb * sizeof(T), [&](int32_t *cnt) {
+        launch_blocks(k_rb_union<false, T>, nblk, N, (i64)rb * S.L, J, c, N, S.L, rb, cnt, (const i64 *)nullptr, (i64)0,
+                      (int32_t *)nullptr, (T *)nullptr, (int32_t *)nullptr);
+    });
+    HIPOTF_REQUIRE(p.total < (1ll << 31), "row-block table too large for 32-bit offsets");
+    DevBuf off;
+    if (!p.stride) off.upload(p.first);
     R.rb = rb;
     R.nblk = nblk;
-    R.entries = E;
-    R.J.alloc((size_t)E * sizeof(int32_t));
-    R.c64.alloc((size_t)E * rb * sizeof(double));
-    R.c32.alloc((size_t)E * rb * sizeof(float));
+    R.J.alloc((size_t)p.total * sizeof(int32_t));
+    R.c.alloc((size_t)p.total * rb * sizeof(T));
     R.P.alloc((size_t)nblk * (SS_RANGES + 1) * sizeof(int32_t));
-    HIPOTF_CHECK(hipMemset(R.c64.p, 0, (size_t)E * rb * sizeof(double)));
-    HIPOTF_CHECK(hipMemset(R.c32.p, 0, (size_t)E * rb * sizeof(float)));
-    hipLaunchKernelGGL(k_rb_union<true>, dim3((unsigned)nblk), dim3(1024), smem, 0, T.J.as<int32_t>(),
-                       T.c64.as<double>(), N, L, rb, LP, nullptr, off.as<i64>(), R.J.as<int32_t>(),
-                       R.c64.as<double>(), R.c32.as<float>(), R.P.as<int32_t>());
-    HIPOTF_CHECK(hipGetLastError());
-    HIPOTF_CHECK(hipDeviceSynchronize());
+    launch_blocks(k_rb_union<true, T>, nblk, N, (i64)rb * S.L, J, c, N, S.L, rb, (int32_t *)nullptr,
+                  off.as<const i64>(), p.stride, R.J.as<int32_t>(), R.c.as<T>(), R.P.as<int32_t>());
+}
+void row_blocks_dev(SameSpinTable &S, RowBlockTable &R, int rb, int prec) {
+    if (prec == 0) row_blocks_t<double>(S, R, rb);
+    else row_blocks_t<float>(S, R, rb);
 }
 
 // ---------------------------------------------------------------------------------------
-// matrix-core row-SpMM table (MfmaBlockTable) from the blocks of rb rows, one workgroup per
-// block; FILL = false: its batches
+// matrix-core row-SpMM table (MfmaBlockTable), one workgroup per block of rb rows: the union of its
+// sources cut into nr ranges, each padded to whole groups of MB_GRP batches of 4 with its last
+// source and coefficients 0; after the last range 2 more groups of source 0, which the kernel reads
+// ahead but does not use.  FILL = false: the block's batches into cnt[g]; first place: first[g], or
+// g * stride.  (From the same-spin rows themselves: by way of a row-block table of 16, filled in
+// both precisions, converted and dropped again, preparing 18 orbitals / 2 + 7 took 19.4 ms, now
+// 5.2; 14 / 7 + 7 1.60 -> 0.73, 8 / 4 + 4 0.35 -> 0.19)
 // ---------------------------------------------------------------------------------------
 template <bool FILL>
-__global__ __launch_bounds__(256) void k_mb(const int32_t *__restrict__ J, const int32_t *__restrict__ P,
-                                            const double *__restrict__ C, int rb, int nr, int32_t *__restrict__ cnt,
-                                            const int32_t *__restrict__ first, int32_t *__restrict__ Pm,
-                                            int32_t *__restrict__ Jm, double *__restrict__ cm) {
-    const i64 b = blockIdx.x;
-    const int32_t e0 = P[b * (SS_RANGES + 1)];
-    int at = FILL ? first[b] : 0;
-    for (int r = 0; r < nr; ++r) {
-        const int32_t s = P[b * (SS_RANGES + 1) + r * (SS_RANGES / nr)], e = P[b * (SS_RANGES + 1) + (r + 1) * (SS_RANGES / nr)];
-        const int nb = (e - s + 4 * MB_GRP - 1) / (4 * MB_GRP) * MB_GRP;
-        if (FILL) {
-            if (threadIdx.x == 0) Pm[b * (nr + 1) + r] = at;
-            for (int i = threadIdx.x; i < nb * 4; i += blockDim.x) {
-                const bool in = s + i < e;
-                const i64 d = (i64)at * 4 + i, src = in ? s + i : (e > s ? e - 1 : e0);
-                Jm[d] = J[src];
-                for (int q = 0; q < rb; ++q)
-                    cm[d * rb + (rb == 16 ? q : (q % 4) * 2 + q / 4)] = in ? C[src * rb + q] : 0.0;
-            }
-        }
-        at += nb;
+__global__ __launch_bounds__(1024) void k_mb_union(const int32_t *__restrict__ J, const double *__restrict__ c64,
+                                                   i64 N, int L, int rb, int nr, int32_t *__restrict__ cnt,
+                                                   const i64 *__restrict__ first, i64 stride,
+                                                   int32_t *__restrict__ Pm, int32_t *__restrict__ Jm,
+                                                   double *__restrict__ cm) {
+    extern __shared__ u32 lds[];
+    __shared__ int start[SS_RANGES + 1], base[SS_RANGES + 1];  // of each range: union position, batch
+    const int tid = threadIdx.x, nt = blockDim.x;
+    const i64 g = blockIdx.x, r0 = g * rb, r1 = r0 + rb < N ? r0 + rb : N;
+    const int m = (int)((r1 - r0) * L);
+    const TbSet s = tb_union(lds, J + r0 * L, m, N);
+    if (tid <= nr) start[tid] = tid == nr ? s.pre[s.groups] : tb_below(s, (i64)(tid * (SS_RANGES / nr)) * N / SS_RANGES);
+    __syncthreads();
+    if (tid == 0) {
+        base[0] = 0;
+        for (int r = 0; r < nr; ++r)
+            base[r + 1] = base[r] + (start[r + 1] - start[r] + 4 * MB_GRP - 1) / (4 * MB_GRP) * MB_GRP;
+        if (!FILL) cnt[g] = base[nr] + 2 * MB_GRP;
     }
-    if (threadIdx.x == 0) {
-        if (FILL) Pm[b * (nr + 1) + nr] = at;
-        else cnt[b] = at;
+    if (!FILL) return;
+    __syncthreads();
+    const i64 o = stride ? g * stride : first[g];
+    if (tid <= nr) Pm[g * (nr + 1) + tid] = (int32_t)(o + base[tid]);
+    auto place = [&](int p) {  // entry of union position p
+        int r = 0;
+        while (r + 1 < nr && start[r + 1] <= p) ++r;
+        return base[r] * 4 + p - start[r];
+    };
+    tb_members(s, [&](int p, int j) {
+        const int d = place(p);
+        Jm[o * 4 + d] = j;
+        int r = 0;  // the last of its range: the padding too
+        while (r + 1 < nr && start[r + 1] <= p) ++r;
+        if (p + 1 == start[r + 1])
+            for (int q = d + 1; q < base[r + 1] * 4; ++q) Jm[o * 4 + q] = j;
+    });
+    if (tid < 8 * MB_GRP) Jm[(o + base[nr]) * 4 + tid] = 0;
+    for (int i = tid; i < (base[nr] + 2 * MB_GRP) * 4 * rb; i += nt) cm[o * 4 * rb + i] = 0.0;
+    __syncthreads();
+    for (int i = tid; i < m; i += nt) {
+        const i64 src = r0 * L + i;
+        const int q = i / L;
+        cm[(o * 4 + place(tb_below(s, J[src]))) * rb + (rb == 16 ? q : (q % 4) * 2 + q / 4)] = c64[src];
     }
 }
 
@@ -381,43 +460,27 @@ const MfmaBlockTable *mfma_blocks(SameSpinTable &T) {
     // the products.  FP64 sigma, blocks of 8 / 16: 16 orbitals / 8 + 8 electrons 110.9 / 104.5 ms, 18 / 5
     // + 5 52.7 / 50.2 ms, 14 / 7 + 7 (3,432 strings) 4.02 / 3.87 ms; but 13 / 5 + 7 (1,287 and 1,716)
     // 0.66 / 0.71 ms, 10 / 5 + 5 36 / 40 us: there half the waves, and the slices come from L2 anyway
-    M->rb = T.N >= 2048 ? 16 : 8;
-    const bool own = M->rb == 16 && !T.blocks[2];  // blocks of 16 serve only to make these
-    const RowBlockTable &R = row_blocks(T, M->rb);
+    const int rb = M->rb = T.N >= 2048 ? 16 : 8;
     // as many source ranges as keep the gathered slice of 128 columns about within an XCD's 4 MB L2
     // (FP64 sigma, 16 orbitals / 8 + 8 electrons, slice 13.2 MB: 106.4 / 104.5 / 109.3 ms with 2 / 4 /
     // 8 ranges; 18 orbitals / 5 + 5, 8.8 MB: 54.4 / 50.2 / 50.7 ms with 1 / 2 / 4)
     while (M->nr < SS_RANGES && (double)T.N * 128 * 8 > 4.5e6 * M->nr) M->nr *= 2;
-    const i64 nblk = R.nblk;
-    M->nblk = nblk;
-    DevBuf cnt, first;
-    cnt.alloc((size_t)nblk * 4);
-    auto go = [&](auto kern) {
-        hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(256), 0, 0, R.J.as<int32_t>(), R.P.as<int32_t>(),
-                           R.c64.as<double>(), M->rb, M->nr, cnt.as<int32_t>(), first.as<int32_t>(), M->P.as<int32_t>(),
-                           M->J.as<int32_t>(), M->c64.as<double>());
-        HIPOTF_CHECK(hipGetLastError());
-    };
-    go(k_mb<false>);
-    std::vector<int32_t> h(nblk), f(nblk);
-    HIPOTF_CHECK(hipMemcpy(h.data(), cnt.p, (size_t)nblk * 4, hipMemcpyDeviceToHost));
-    i64 t = 0;
-    for (i64 b = 0; b < nblk; ++b) {
-        f[b] = (int32_t)t;
-        t += h[b];
-        HIPOTF_REQUIRE(t < (1ll << 31) - 64, "matrix-core row-block table too large for 32-bit offsets");
-    }
-    M->batches = t;
-    first.upload(f);
-    const size_t E = (size_t)t + 4 * MB_GRP;  // (the kernel reads up to 3 groups past a range's end)
+    const i64 N = T.N, nblk = M->nblk = (N + rb - 1) / rb;
+    const i64 most = (std::min<i64>(N, (i64)rb * T.L) + 3) / 4 + (i64)M->nr * MB_GRP + 2 * MB_GRP;
+    const int32_t *J = T.J.as<int32_t>();
+    const double *c = T.c64.as<double>();
+    const TbPlaces p = tb_places(nblk, most, 16 + 32 * rb, [&](int32_t *cnt) {
+        launch_blocks(k_mb_union<false>, nblk, N, (i64)rb * T.L, J, c, N, T.L, rb, M->nr, cnt, (const i64 *)nullptr,
+                      (i64)0, (int32_t *)nullptr, (int32_t *)nullptr, (double *)nullptr);
+    });
+    HIPOTF_REQUIRE(p.total < (1ll << 31) - 64, "matrix-core row-block table too large for 32-bit offsets");
+    DevBuf first;
+    if (!p.stride) first.upload(p.first);
     M->P.alloc((size_t)nblk * (M->nr + 1) * 4);
-    M->J.alloc(E * 16);
-    M->c64.alloc(E * 4 * M->rb * sizeof(double));
-    HIPOTF_CHECK(hipMemset((char *)M->J.p + (size_t)t * 16, 0, 4 * MB_GRP * 16));
-    HIPOTF_CHECK(hipMemset((char *)M->c64.p + (size_t)t * 32 * M->rb, 0, 4 * MB_GRP * 32 * (size_t)M->rb));
-    go(k_mb<true>);
-    HIPOTF_CHECK(hipDeviceSynchronize());
-    if (own) T.blocks[2].reset();
+    M->J.alloc((size_t)p.total * 16);
+    M->c64.alloc((size_t)p.total * 4 * rb * sizeof(double));
+    launch_blocks(k_mb_union<true>, nblk, N, (i64)rb * T.L, J, c, N, T.L, rb, M->nr, (int32_t *)nullptr,
+                  first.as<const i64>(), p.stride, M->P.as<int32_t>(), M->J.as<int32_t>(), M->c64.as<double>());
     T.mfma = std::move(M);
     return T.mfma.get();
 }
