@@ -79,12 +79,16 @@ DavidsonOut davidson(DevHam *H, int nroots, int mode, int block, double tol, dou
     HIPOTF_REQUIRE(maxspace >= 2 * k || maxspace == N, "maxspace must be >= 2 * block");
     DavidsonOut out;
 
-    // device memory of the whole solve, checked before anything is allocated: 2 * maxspace
+    // the tables of the solve's sigmas first (at 16 orbitals / 8 + 8 electrons hundreds of MB in FP32)
+    sigma_tables(H, 0, std::min(k, 8), mode == 0, st);
+    if (mode == 1) sigma_tables(H, 1, std::min(k, 8), false, st);
+
+    // device memory of the whole solve, checked before anything else is allocated: 2 * maxspace
     // subspace vectors (V, AV), the diagonal, k residuals (plain mode; the block mode forms its
     // residuals in free subspace slots), and the sigma work buffers (4 per basis, dim *
     // vectors per pass * word size; grown on first use).  The block mode passes as many of its
     // up to 8 vectors through one sigma as the memory left allows (nv_sigma).  The loop itself
-    // allocates nothing: restarts and the FP32 -> FP64 switch combine the subspace in place.
+    // allocates nothing (a few MB for reductions aside): restarts and the FP32 -> FP64 switch combine the subspace in place.
     int nv_sigma = 1;
     {
         const size_t vec = (size_t)N * sizeof(double);

@@ -280,6 +280,9 @@ constexpr int TUNING_FIELDS = 8;
 // lets FP32 take the fastest alpha-beta kernel whatever its order of additions
 void sigma(DevHam *H, int nv, const double *const *src, double *const *dst, int prec,
            hipStream_t st, int maxnv = 8, bool fixed = true);
+// builds the tables that sigmas of that precision and up to maxnv vectors a pass read, so that they
+// build none (their work buffers aside)
+void sigma_tables(DevHam *H, int prec, int maxnv, bool fixed, hipStream_t st);
 void diag_elements(DevHam *H, double *diags, hipStream_t st);  // accumulates
 // one FP64 sigma with the four work buffers carved from the library's static device scratch
 // array (no device allocation; every table must already exist); at most

@@ -670,6 +670,7 @@ static void launch_mbspmm_n(const T *X, T *Y, const MfmaBlockTable &M, i64 nrows
 // 23.2 / 22.8 us, 10 / 5 + 5 45 / 40 / 36 us, 12 / 6 + 6 207 / 216 / 240 us, 16 / 8 + 8 109 / 118 / 136 ms
 template <typename T>
 static void launch_mbspmm(const T *X, T *Y, const MfmaBlockTable &M, i64 nrows, i64 ncols, hipStream_t st) {
+    if (!X) return;  // (sigma_tables)
     auto waves = [&](int cols) { return (ncols + cols - 1) / cols * M.nblk; };
     const int cols = waves(128) >= 768 ? 128 : (waves(64) >= 384 ? 64 : 32);
     auto go = [&](auto rb) {
@@ -712,11 +713,13 @@ static void launch_rowspmm(const T *X, T *Y, SameSpinTable &tab, const T *C, i64
     if (rb == 4 || rb == 8 || rb == 16) {
         const int npass = rs_npass<T>(nrows, 256 * rs_cpl<T>(ncols));
         const RowBlockTable &rt = row_blocks(tab, rb, sizeof(T) == 4);
+        if (!X) return;
         if (rb == 4) launch_rbspmm<T, 4>(X, Y, rt, nrows, ncols, npass, st);
         else if (rb == 8) launch_rbspmm<T, 8>(X, Y, rt, nrows, ncols, npass, st);
         else launch_rbspmm<T, 16>(X, Y, rt, nrows, ncols, npass, st);
         return;
     }
+    if (!X) return;
     const i64 ntiles = (ncols + 63) / 64;
     const i64 bpt = (nrows + 3) / 4;
     const i64 ntiles_pad = (ntiles + 7) / 8 * 8;
@@ -900,6 +903,7 @@ static bool try_ab_src_r(DevHam *H, const T *xt, T *s1, int nvst, int v0, const 
         HIPOTF_REQUIRE(nblocks < (1ll << 31), "alpha-beta grid too large");
         const T *dw = diag_w_table<T>(H, st);
         auto go = [&](auto kern) {
+            if (!xt) return;
             HIPOTF_CHECK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                              (int)smem));
             for (int part = 0; part < parts; ++part) {
@@ -968,7 +972,8 @@ static const uint2 *ab_target_table(DevBasis *B, int n, int NN, int mo, int mc, 
 // launch, split by the top orbital; not in the deterministic mode (its LDS adds come from all
 // waves at once)
 template <typename T>
-static bool try_ab_mma(DevHam *H, const T *xt, T *s1, int nvst, int v0, const T *eri, hipStream_t st) {
+static bool try_ab_mma(DevHam *H, const T *xt, T *s1, int nvst, int v0, const T *eri, hipStream_t st,
+                       bool tables = false) {
     constexpr int prec = sizeof(T) == 4;
     if (deterministic(prec)) return false;
     DevBasis *B = H->basis;
@@ -993,6 +998,7 @@ static bool try_ab_mma(DevHam *H, const T *xt, T *s1, int nvst, int v0, const T 
         if (smem > lds || A.nsx + 1 > 4 * KS || rows > 16 * MO || n > 4 * MO || (MC && n - 1 > 16 * MC)) return false;
         const uint2 *tab = ab_target_table<T>(B, n, (int)nn, MO, MC, st);
         const T *dw = diag_w_table<T>(H, st);
+        if (!xt) return true;
         auto kern = k_ab_mma<T, MO, MC, KS, NWV, decltype(wpc)::value>;
         HIPOTF_CHECK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
         for (int cls = 0; cls < (MC ? 2 : 1); ++cls) {
@@ -1042,6 +1048,7 @@ static bool try_ab_cls(DevHam *H, const float *xt, float *s1, int nvst, int v0, 
     const i64 nblocks = (A.N + 7) / 8 * 8;
     HIPOTF_REQUIRE(nblocks < (1ll << 31), "alpha-beta grid too large");
     const float *dw = diag_w_table<float>(H, st);
+    if (!xt) return true;
     auto go = [&](auto kern, int ko, int vo, int kf) {
         HIPOTF_CHECK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
         hipLaunchKernelGGL(kern, dim3((unsigned)nblocks), dim3(AB_SRC_NJ), smem, st, xt, s1, nvst, v0,
@@ -1140,7 +1147,7 @@ static void launch_ab(DevHam *H, const T *xt, T *s1, int nv, const T *eri, hipSt
     int nvs = 1;
     if (nv >= 4 && fits(4)) nvs = 4;
     else if (nv >= 2 && fits(2)) nvs = 2;
-    while (v0 < nv) {
+    while (xt && v0 < nv) {
         const int m = std::min(nvs, nv - v0);
         if (m >= 4) { launch_ab_nvs<T, 4>(H, xt, s1, nv, v0, eri, st); v0 += 4; }
         else if (m >= 2) { launch_ab_nvs<T, 2>(H, xt, s1, nv, v0, eri, st); v0 += 2; }
@@ -1221,6 +1228,23 @@ static void sigma_t(DevHam *H, int nv, const double *const *src, double *const *
             case 7: sigma_group<T, 7>(H, sp, dp, st, fixed); break;
             default: sigma_group<T, 8>(H, sp, dp, st, fixed); break;
         }
+    }
+}
+
+// the launches of a sigma pass of nv vectors without vectors: each kernel's tables, no kernel
+template <typename T>
+static void sigma_tables_t(DevHam *H, int nv, bool fixed, hipStream_t st) {
+    const i64 NA = H->basis->pA->N, NB = H->basis->pB->N;
+    if (NA == 0 || NB == 0) return;
+    launch_rowspmm<T>(nullptr, nullptr, *H->ptA, nullptr, NA, NB * nv, fixed, st);
+    launch_rowspmm<T>(nullptr, nullptr, *H->ptB, nullptr, NB, NA * nv, fixed, st);
+    launch_ab<T>(H, nullptr, nullptr, nv, nullptr, st, fixed);
+}
+void sigma_tables(DevHam *H, int prec, int maxnv, bool fixed, hipStream_t st) {
+    HIPOTF_REQUIRE(H != nullptr && maxnv >= 1 && maxnv <= MAXNV, "sigma tables: bad arguments");
+    for (int nv = 1; nv <= maxnv; ++nv) {
+        if (prec == 0) sigma_tables_t<double>(H, nv, fixed, st);
+        else sigma_tables_t<float>(H, nv, fixed, st);
     }
 }
 

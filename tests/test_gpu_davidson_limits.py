@@ -49,3 +49,14 @@ def test_gram_schmidt_against_a_subspace_that_holds_the_vector(torch_cuda, N):
     got = L.load().mgs_orthogonalize_f64(N, 3, D._pp([ad, td, bd]), td.data_ptr())
     assert np.max(np.abs(host(td) - want)) < 1e-13
     assert abs(got - np.linalg.norm(want)) < 1e-13
+
+
+def test_tables_come_before_the_memory_check(torch_cuda):
+    """18 orbitals / 6 + 6 with 64 subspace vectors: more than the card holds, refused before anything is
+    computed.  The FP32 tables of the mixed solve (over 100 MB) are then there: their memory was not
+    counted as free."""
+    B, H, F = _dev(18, 6, 6)
+    before = torch_cuda.cuda.mem_get_info()[0]
+    with pytest.raises(L.HipOTFError, match="davidson: needs"):
+        D.solve(B, H, nroots=1, mixed=True, maxspace=64)
+    assert before - torch_cuda.cuda.mem_get_info()[0] > 100 << 20
