@@ -975,7 +975,7 @@ template <typename T>
 static bool try_ab_mma(DevHam *H, const T *xt, T *s1, int nvst, int v0, const T *eri, hipStream_t st,
                        bool tables = false) {
     constexpr int prec = sizeof(T) == 4;
-    if (deterministic(prec)) return false;
+    if (deterministic(prec) && !tables) return false;
     DevBasis *B = H->basis;
     const DevSpin &A = *B->pA, &Bs = *B->pB;
     const int n = H->n;
@@ -1153,6 +1153,11 @@ static void launch_ab(DevHam *H, const T *xt, T *s1, int nv, const T *eri, hipSt
         else if (m >= 2) { launch_ab_nvs<T, 2>(H, xt, s1, nv, v0, eri, st); v0 += 2; }
         else { launch_ab_nvs<T, 1>(H, xt, s1, nv, v0, eri, st); v0 += 1; }
     }
+    // hipotf_hvec_noalloc may follow under other choices: with the diagonal rows of the kernel that ran,
+    // the targets of the default one
+    if constexpr (sizeof(T) == 8)
+        if (!g_forbid_alloc && H->dw64.p && !B->abt64.p && B->host.dim <= NOALLOC_MAX_DIM)
+            try_ab_mma<T>(H, nullptr, nullptr, 1, 0, nullptr, st, true);
 }
 
 // work: NULL (the basis's own work buffers, grown as needed) or 4 consecutive 256-byte aligned

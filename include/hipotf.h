@@ -162,8 +162,9 @@ int hipotf_ab_timing(int enable, double *ms, int64_t *sections, int64_t *mma_lau
  * that forbid hipMalloc).  dst = H src in FP64 as hvec_cuda computes it, with the four sigma
  * work buffers in the library's static device scratch array (64 MiB per GPU, held until the
  * process ends), so at most 2,097,152 determinants (larger bases are refused).  The operator's
- * device tables must already exist for this basis (hipotf_prepare or one hvec_cuda call);
- * otherwise the call is refused rather than building them.  Calls on one GPU share the
+ * device tables must already exist for this basis: one hvec_cuda call after hipotf_prepare (which
+ * alone leaves the alpha-beta kernels' tables to the first call); otherwise the call is refused
+ * rather than building them.  Calls on one GPU share the
  * scratch array: calls that overlap on one GPU (several host threads or streams) race.
  * Returns 0 on success, 1 on error (message in hipotf_last_error()). */
 int hipotf_hvec_noalloc(void *basis, void *net, const double *src, double *dst);
