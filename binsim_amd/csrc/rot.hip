@@ -1240,12 +1240,12 @@ static void sweeps(DevPool *P, i64 n, const i64 *idxs, const double *thetas, con
         // pair segment of a run of them and split back before a row segment or the end
         double2 *z = nullptr;
         bool zipped = false;
-        if (il) {
-            P->tz.ensure((size_t)dim * sizeof(double2));
-            z = P->tz.as<double2>();
-        }
         auto zip = [&](bool on) {
             if (on == zipped) return;
+            if (on) {  // (a sweep on excitation levels alone never needs it)
+                P->tz.ensure((size_t)dim * sizeof(double2));
+                z = P->tz.as<double2>();
+            }
             if (on) hipLaunchKernelGGL(k_zip, dim3(grid_for(dim)), dim3(256), 0, st, psi, lam, z, dim);
             else hipLaunchKernelGGL(k_unzip, dim3(grid_for(dim)), dim3(256), 0, st, z, psi, lam, dim);
             HIPOTF_CHECK(hipGetLastError());

@@ -125,3 +125,20 @@ def test_window_pools_take_no_longer_than_whole_rows(torch_cuda, lo, hi):
     finally:
         A.set_config(0, {})
     assert took[0] < 3.0 * took[3]
+
+
+def test_no_interleaved_copy_on_levels_alone(torch_cuda):
+    """14 orbitals / 7 + 7: the adjoint sweep of a particle-hole pool has no pair segment, so the
+    interleaved (l, r) copy (16 bytes per determinant) is not allocated.  Its other buffers (gradient
+    partials of some 100 MB) are smaller than that copy."""
+    sos = ucc_spin_orbitals(14, 7, 7)
+    B, F = _functions(14, 7, 7, sos)
+    x = gpu_vec(torch_cuda, seeded_vector(B.dim, 1))
+    y, idx, th = torch_cuda.empty_like(x), np.arange(len(sos), dtype=np.int64), np.full(len(sos), 0.01)
+    F.hvec(x, y)
+    F.vqe_sweep(idx, th, x, y)
+    torch_cuda.cuda.synchronize()
+    before = torch_cuda.cuda.mem_get_info()[0]
+    F.vqe_energy_grad(idx, th, x, y)
+    torch_cuda.cuda.synchronize()
+    assert before - torch_cuda.cuda.mem_get_info()[0] < 16 * B.dim
