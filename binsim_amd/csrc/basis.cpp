@@ -160,6 +160,7 @@ DevBasis *make_dev_basis(const HostBasis &hb) {
             if ((a >> p) & 1) m ^= (1ull << p) - 1;
         M[i] = m;
     }
+    M.push_back(0);
     db->gaugeM.upload(M);
     return db.release();
 }

@@ -139,7 +139,8 @@ struct DevBasis {
     HostBasis host;           // own copy of the host description
     DevSpin A, B;             // B aliases A's tables when na == nb (shared pointers below)
     DevSpin *pA = nullptr, *pB = nullptr;
-    DevBuf gaugeM;            // u64[Na]: M(a) = XOR_{p in a} ((1<<p)-1)
+    DevBuf gaugeM;            // u64[Na]: M(a) = XOR_{p in a} ((1<<p)-1); then an int: the sigma under
+                              // way has a source element that is not finite
     i64 uid = 0;              // unique id (operators cache per-basis tables under it)
     // scratch shared by sigma calls on this basis
     DevBuf xt, xtT, s1, s2T;
@@ -172,6 +173,7 @@ struct RowBlockTable {
 // (k_mbspmm): each block's sources in nr source ranges, each range padded to whole groups of
 // MB_GRP batches of 4 sources (coefficient 0, a valid source), and two groups after the last
 constexpr int MB_RB = 8, MB_GRP = 4;
+constexpr i64 MB_RB16_FROM = 2048;  // strings
 struct MfmaBlockTable {
     int rb = MB_RB;           // strings per block: 8 or 16
     int nr = 1;               // source ranges: passes of the kernel

@@ -38,10 +38,11 @@ __device__ __forceinline__ float flip_sign(float v, u32 s) { return __uint_as_fl
 // ---------------------------------------------------------------------------------------
 // K1: gauge + dual layout (32x32 tiles through LDS)
 // ---------------------------------------------------------------------------------------
+// flag (if given): set to 1 by an element that is not finite (k_mbspmm)
 template <typename T, int NV>
 __global__ __launch_bounds__(256) void k_gauge_in(SrcPack src, T *__restrict__ xt, T *__restrict__ xtT,
                                                   const u64 *__restrict__ strsB,
-                                                  const u64 *__restrict__ M, i64 NA, i64 NB) {
+                                                  const u64 *__restrict__ M, i64 NA, i64 NB, int *flag) {
     __shared__ T tile[32][33];
     const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 32 x 8
     const i64 b0 = (i64)blockIdx.x * 32, a0 = (i64)blockIdx.y * 32;
@@ -52,6 +53,7 @@ __global__ __launch_bounds__(256) void k_gauge_in(SrcPack src, T *__restrict__ x
             if (a < NA && b < NB) {
                 double val = src.p[v][a * NB + b];
                 if (parity64(strsB[b] & M[a])) val = -val;
+                if (flag && !isfinite(val)) *flag = 1;
                 const T tv = (T)val;
                 xt[(a * NB + b) * NV + v] = tv;
                 tile[ty + 8 * i][tx] = tv;
@@ -221,6 +223,11 @@ __global__ __launch_bounds__(256) void k_rbspmm(const T *__restrict__ X, T *__re
 // gathered, but 49 ms with scalar coefficients and 76 ms on the matrix cores: too few loads in
 // flight beside the LDS buffers).  FP32, blocks of 4 vectors, 12 orbitals / 6 electrons: 173 (k_rbspmm)
 // -> 121 us per spin; 256 columns per wave the same.
+//
+// Infinities and NaN.  A product with a zero coefficient spreads them to rows of the block that are not
+// connected to their source; with 16 strings to a block that are more rows than any other form reaches,
+// so where the source vector holds any (flag, set by k_gauge_in) the blocks of 16 leave those products
+// out one by one (16 orbitals / 8 + 8: 0.52 s for such a sigma, 0.104 s without as before).
 // ---------------------------------------------------------------------------------------
 constexpr size_t MB_SLACK = 1024;  // bytes after the source vector that k_mbspmm may read
 template <typename T, int NP, int RB>
@@ -228,7 +235,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NP == 4 ? 3
 void k_mbspmm(const T *__restrict__ X, T *__restrict__ Y,
                                                 const int32_t *__restrict__ J, const int32_t *__restrict__ P,
                                                 const double *__restrict__ C, i64 nrows, i64 ncols, i64 nblk,
-                                                i64 nwork, i64 per_xcd, int nr, int r, int accumulate) {
+                                                i64 nwork, i64 per_xcd, int nr, int r, int accumulate,
+                                                const int *__restrict__ flag) {
     constexpr int W = 16 / sizeof(T);  // consecutive columns per lane and load
     typedef T VW __attribute__((ext_vector_type(16 / sizeof(T)), aligned(sizeof(T))));
     const int lane = threadIdx.x & 63, k = lane >> 4, j = lane & 15;
@@ -241,6 +249,31 @@ void k_mbspmm(const T *__restrict__ X, T *__restrict__ Y,
     const char *Xc = reinterpret_cast<const char *>(X + (col0 < ncols ? col0 : 0));
     int b = P[blk * (nr + 1) + r];
     const int e = P[blk * (nr + 1) + r + 1];
+    if constexpr (RB == 16) {
+        if (*flag) {
+            for (i64 col = tile * (16 * W * NP) + lane; col < ncols && col < (tile + 1) * (16 * W * NP); col += 64)
+                for (int h = 0; h < RB; h += 8) {
+                    double s[8];
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) {
+                        const i64 row = blk * RB + h + q;
+                        s[q] = accumulate && row < nrows ? (double)Y[row * ncols + col] : 0.0;
+                    }
+                    for (i64 at = (i64)b * 4; at < (i64)e * 4; ++at) {
+                        const double x = (double)X[(i64)J[at] * ncols + col];
+#pragma unroll
+                        for (int q = 0; q < 8; ++q) {
+                            const double c = C[at * RB + h + q];
+                            s[q] = c != 0.0 ? s[q] + c * x : s[q];
+                        }
+                    }
+#pragma unroll
+                    for (int q = 0; q < 8; ++q)
+                        if (blk * RB + h + q < nrows) Y[(blk * RB + h + q) * ncols + col] = (T)s[q];
+                }
+            return;
+        }
+    }
     typedef double V4 __attribute__((ext_vector_type(4)));
     typedef typename std::conditional<RB == 16, double, double2>::type CF;  // a lane's coefficients of a batch
     double acc[2][RB == 8 ? W * NP : 1];
@@ -554,9 +587,10 @@ template <typename T, int NV>
 __global__ __launch_bounds__(256) void k_finalize(const T *__restrict__ s1, const T *__restrict__ s2T,
                                                   const T *__restrict__ xt, double ecore, DstPack dst,
                                                   const u64 *__restrict__ strsB,
-                                                  const u64 *__restrict__ M, i64 NA, i64 NB) {
+                                                  const u64 *__restrict__ M, i64 NA, i64 NB, int *flag) {
     __shared__ T tile[32][33];
     const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    if (flag && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *flag = 0;  // (for the next sigma)
     const i64 b0 = (i64)blockIdx.x * 32, a0 = (i64)blockIdx.y * 32;
 #pragma unroll 1
     for (int v = 0; v < NV; ++v) {
@@ -653,7 +687,8 @@ static int rs_npass(i64 nrows, int tile_cols) {
 }
 
 template <typename T, int NP, int RB>
-static void launch_mbspmm_n(const T *X, T *Y, const MfmaBlockTable &M, i64 nrows, i64 ncols, hipStream_t st) {
+static void launch_mbspmm_n(const T *X, T *Y, const MfmaBlockTable &M, i64 nrows, i64 ncols, const int *flag,
+                            hipStream_t st) {
     constexpr int cols = 256 / sizeof(T) * NP;
     const i64 ntiles = (ncols + cols - 1) / cols, nwork = ntiles * M.nblk, per_xcd = (nwork + 7) / 8;
     const i64 nwg = (per_xcd + 3) / 4 * 8;
@@ -661,7 +696,7 @@ static void launch_mbspmm_n(const T *X, T *Y, const MfmaBlockTable &M, i64 nrows
     for (int r = 0; r < M.nr; ++r)
         hipLaunchKernelGGL((k_mbspmm<T, NP, RB>), dim3((unsigned)nwg), dim3(256), 0, st, X, Y, M.J.as<int32_t>(),
                            M.P.as<int32_t>(), M.c64.as<double>(), nrows, ncols, M.nblk, nwork, per_xcd, M.nr, r,
-                           r > 0 ? 1 : 0);
+                           r > 0 ? 1 : 0, flag);
     HIPOTF_CHECK(hipGetLastError());
 }
 
@@ -669,15 +704,16 @@ static void launch_mbspmm_n(const T *X, T *Y, const MfmaBlockTable &M, i64 nrows
 // the chip short of waves.  FP64 sigma with 128 / 64 / 32 columns: 8 orbitals / 4 + 4 electrons 24.9 /
 // 23.2 / 22.8 us, 10 / 5 + 5 45 / 40 / 36 us, 12 / 6 + 6 207 / 216 / 240 us, 16 / 8 + 8 109 / 118 / 136 ms
 template <typename T>
-static void launch_mbspmm(const T *X, T *Y, const MfmaBlockTable &M, i64 nrows, i64 ncols, hipStream_t st) {
+static void launch_mbspmm(const T *X, T *Y, const MfmaBlockTable &M, i64 nrows, i64 ncols, const int *flag,
+                          hipStream_t st) {
     if (!X) return;  // (sigma_tables)
     auto waves = [&](int cols) { return (ncols + cols - 1) / cols * M.nblk; };
     const int cols = waves(128) >= 768 ? 128 : (waves(64) >= 384 ? 64 : 32);
     auto go = [&](auto rb) {
         constexpr int RB = decltype(rb)::value, W = 16 / sizeof(T);
-        if (cols == 128) launch_mbspmm_n<T, 8 / W, RB>(X, Y, M, nrows, ncols, st);
-        else if (cols == 64 || W == 4) launch_mbspmm_n<T, 4 / W, RB>(X, Y, M, nrows, ncols, st);
-        else launch_mbspmm_n<T, 1, RB>(X, Y, M, nrows, ncols, st);
+        if (cols == 128) launch_mbspmm_n<T, 8 / W, RB>(X, Y, M, nrows, ncols, flag, st);
+        else if (cols == 64 || W == 4) launch_mbspmm_n<T, 4 / W, RB>(X, Y, M, nrows, ncols, flag, st);
+        else launch_mbspmm_n<T, 1, RB>(X, Y, M, nrows, ncols, flag, st);
     };
     if constexpr (sizeof(T) == 8) {
         if (M.rb == 16) return go(std::integral_constant<int, 16>{});
@@ -688,7 +724,7 @@ static void launch_mbspmm(const T *X, T *Y, const MfmaBlockTable &M, i64 nrows, 
 
 template <typename T>
 static void launch_rowspmm(const T *X, T *Y, SameSpinTable &tab, const T *C, i64 nrows,
-                           i64 ncols, bool fixed, hipStream_t st) {
+                           i64 ncols, bool fixed, const int *flag, hipStream_t st) {
     if (nrows == 0 || ncols == 0) return;
     HIPOTF_REQUIRE(nrows == tab.N, "internal: same-spin table does not match the row count");
     int rb = tuning(sizeof(T) == 4).rs_block;
@@ -698,7 +734,7 @@ static void launch_rowspmm(const T *X, T *Y, SameSpinTable &tab, const T *C, i64
         // the FP64 products take longer (mixed Davidson, blocks of 4: 40 iterations at 14 orbitals
         // 0.94 s on the matrix cores, 0.89 s on the VALU; 16 iterations at 16 orbitals 7.3 / 6.6 s)
         if (sizeof(T) == 8 || (!fixed && tab.N < 2048))
-            if (const MfmaBlockTable *M = mfma_blocks(tab)) return launch_mbspmm(X, Y, *M, nrows, ncols, st);
+            if (const MfmaBlockTable *M = mfma_blocks(tab)) return launch_mbspmm(X, Y, *M, nrows, ncols, flag, st);
         if constexpr (sizeof(T) == 4) {
             // FP32 otherwise: blocks of 4 strings, the same sums in the same order as blocks of 8 (FP32
             // sigma, 4 vectors: 12 orbitals 1.77 -> 1.67 ms, 14 orbitals 12.1 -> 11.5 ms).  Tables from
@@ -709,7 +745,7 @@ static void launch_rowspmm(const T *X, T *Y, SameSpinTable &tab, const T *C, i64
     // an allocation-free call with other passes than at its preparation: the matrix-core tables
     if constexpr (sizeof(T) == 8)
         if (rb == MB_RB && g_forbid_alloc && !tab.blocks[0][1] && tab.mfma)
-            return launch_mbspmm(X, Y, *tab.mfma, nrows, ncols, st);
+            return launch_mbspmm(X, Y, *tab.mfma, nrows, ncols, flag, st);
     if (rb == 4 || rb == 8 || rb == 16) {
         const int npass = rs_npass<T>(nrows, 256 * rs_cpl<T>(ncols));
         const RowBlockTable &rt = row_blocks(tab, rb, sizeof(T) == 4);
@@ -1186,14 +1222,17 @@ static void sigma_group(DevHam *H, const SrcPack &src, const DstPack &dst, hipSt
     }
     dim3 g2((unsigned)((NB + 31) / 32), (unsigned)((NA + 31) / 32));
     HIPOTF_REQUIRE(g2.y < 65536, "too many alpha strings for the tiled kernels");
+    // (only the blocks of 16 strings ask)
+    int *flag = sizeof(T) == 8 && std::max(NA, NB) >= MB_RB16_FROM ? reinterpret_cast<int *>(B->gaugeM.as<u64>() + NA)
+                                                                   : nullptr;
     hipLaunchKernelGGL((k_gauge_in<T, NV>), g2, dim3(256), 0, st, src, xt, xtT, Bs.strs.as<u64>(),
-                       B->gaugeM.as<u64>(), NA, NB);
+                       B->gaugeM.as<u64>(), NA, NB, flag);
     HIPOTF_CHECK(hipGetLastError());
     const bool f32 = sizeof(T) == 4;
     const T *CA = f32 ? (const T *)H->ptA->c32.p : (const T *)H->ptA->c64.p;
     const T *CB = f32 ? (const T *)H->ptB->c32.p : (const T *)H->ptB->c64.p;
-    launch_rowspmm<T>(xt, s1, *H->ptA, CA, NA, NB * NV, fixed, st);
-    launch_rowspmm<T>(xtT, s2T, *H->ptB, CB, NB, NA * NV, fixed, st);
+    launch_rowspmm<T>(xt, s1, *H->ptA, CA, NA, NB * NV, fixed, flag, st);
+    launch_rowspmm<T>(xtT, s2T, *H->ptB, CB, NB, NA * NV, fixed, flag, st);
     const T *eri = f32 ? (const T *)H->eri32.p : (const T *)H->eri64.p;
     AbTiming &tm = ab_timing();
     if (tm.on) HIPOTF_CHECK(hipEventRecord(tm.e0, st));
@@ -1207,7 +1246,7 @@ static void sigma_group(DevHam *H, const SrcPack &src, const DstPack &dst, hipSt
         ++tm.sections;
     }
     hipLaunchKernelGGL((k_finalize<T, NV>), g2, dim3(256), 0, st, s1, s2T, xt, H->ecore, dst,
-                       Bs.strs.as<u64>(), B->gaugeM.as<u64>(), NA, NB);
+                       Bs.strs.as<u64>(), B->gaugeM.as<u64>(), NA, NB, flag);
     HIPOTF_CHECK(hipGetLastError());
 }
 
@@ -1241,8 +1280,8 @@ template <typename T>
 static void sigma_tables_t(DevHam *H, int nv, bool fixed, hipStream_t st) {
     const i64 NA = H->basis->pA->N, NB = H->basis->pB->N;
     if (NA == 0 || NB == 0) return;
-    launch_rowspmm<T>(nullptr, nullptr, *H->ptA, nullptr, NA, NB * nv, fixed, st);
-    launch_rowspmm<T>(nullptr, nullptr, *H->ptB, nullptr, NB, NA * nv, fixed, st);
+    launch_rowspmm<T>(nullptr, nullptr, *H->ptA, nullptr, NA, NB * nv, fixed, nullptr, st);
+    launch_rowspmm<T>(nullptr, nullptr, *H->ptB, nullptr, NB, NA * nv, fixed, nullptr, st);
     launch_ab<T>(H, nullptr, nullptr, nv, nullptr, st, fixed);
 }
 void sigma_tables(DevHam *H, int prec, int maxnv, bool fixed, hipStream_t st) {

@@ -460,7 +460,7 @@ const MfmaBlockTable *mfma_blocks(SameSpinTable &T) {
     // the products.  FP64 sigma, blocks of 8 / 16: 16 orbitals / 8 + 8 electrons 110.9 / 104.5 ms, 18 / 5
     // + 5 52.7 / 50.2 ms, 14 / 7 + 7 (3,432 strings) 4.02 / 3.87 ms; but 13 / 5 + 7 (1,287 and 1,716)
     // 0.66 / 0.71 ms, 10 / 5 + 5 36 / 40 us: there half the waves, and the slices come from L2 anyway
-    const int rb = M->rb = T.N >= 2048 ? 16 : 8;
+    const int rb = M->rb = T.N >= MB_RB16_FROM ? 16 : 8;
     // as many source ranges as keep the gathered slice of 128 columns about within an XCD's 4 MB L2
     // (FP64 sigma, 16 orbitals / 8 + 8 electrons, slice 13.2 MB: 106.4 / 104.5 / 109.3 ms with 2 / 4 /
     // 8 ranges; 18 orbitals / 5 + 5, 8.8 MB: 54.4 / 50.2 / 50.7 ms with 1 / 2 / 4)
