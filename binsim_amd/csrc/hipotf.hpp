@@ -279,7 +279,7 @@ constexpr int TUNING_FIELDS = 8;
 
 // sigma: dst_v = H src_v for nv vectors; prec 0 = float64 work, 1 = float32 work; at most
 // maxnv (1..8) vectors share one pass (its work buffers hold dim * maxnv words each); fixed = false
-// lets FP32 take the fastest alpha-beta kernel whatever its order of additions
+// lets FP32 below 14 orbitals take the matrix-core kernels (another order of additions)
 void sigma(DevHam *H, int nv, const double *const *src, double *const *dst, int prec,
            hipStream_t st, int maxnv = 8, bool fixed = true);
 // builds the tables that sigmas of that precision and up to maxnv vectors a pass read, so that they

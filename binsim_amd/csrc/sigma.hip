@@ -729,7 +729,7 @@ static void launch_rowspmm(const T *X, T *Y, SameSpinTable &tab, const T *C, i64
     HIPOTF_REQUIRE(nrows == tab.N, "internal: same-spin table does not match the row count");
     int rb = tuning(sizeof(T) == 4).rs_block;
     if (rb == MB_RB && tuning(sizeof(T) == 4).rs_passes == 0) {  // the defaults
-        // FP32 without a fixed rounding (the Davidson driver's): the matrix cores below 2,048 strings
+        // FP32 in the Davidson driver (fixed = false): the matrix cores below 2,048 strings
         // (4 vectors, 12 orbitals: 173 -> 121 us per spin), blocks of 4 on the VALU from there, where
         // the FP64 products take longer (mixed Davidson, blocks of 4: 40 iterations at 14 orbitals
         // 0.94 s on the matrix cores, 0.89 s on the VALU; 16 iterations at 16 orbitals 7.3 / 6.6 s)
@@ -795,17 +795,19 @@ static void launch_ab_ept(DevHam *H, const T *xt, T *s1, int nvst, int v0, const
 template <typename T, int NVS>
 constexpr int ab_eptmax() { return (sizeof(T) == 8 && NVS >= 4) ? 4 : 8; }
 
-// alpha-beta kernel family (SigmaTuning::ab_kernel): 0 takes the first of matrix-core (FP64 up
-// to 18 orbitals; FP32 of a fixed rounding 14 to 16), class-split (FP32 vector pairs, ab_cls.hpp), source-lane, register, chunked that
-// applies; 1..3 start the search at source-lane, register, chunked; 4 is 1 with FP32 vector
-// pairs on the class-split kernel; 5 puts the matrix-core kernel (ab_mma.hpp, one vector per
-// launch) first.  The matrix-core kernel's FP64 range is all it can hold: it is the fastest at
-// every size measured (whole FP64 sigma against the source-lane kernel beside the same row SpMM: 12
-// orbitals 6 + 6 0.22 / 0.51 ms, 14 / 7 + 7 4.1 / 9.8 ms, 16 / 8 + 8 109 / 198 ms).
-// FP32 calls that promise the caller a fixed rounding (fixed = true: hipotf_hvec_block, whose FP32
-// results below 14 orbitals are those of the class-split and source-lane kernels) keep them there;
-// the Davidson driver's FP32 phase takes the matrix cores at every size (12 orbitals, 4 vectors:
-// 1.36 -> 0.37 ms)
+// alpha-beta kernel family (SigmaTuning::ab_kernel): 0 takes the first of matrix-core (FP64 up to 18
+// orbitals, FP32 14 to 16), class-split (FP32 vector pairs, ab_cls.hpp), source-lane, register,
+// chunked that applies; 1..3 start the search at source-lane, register, chunked; 4 is 1 with FP32
+// vector pairs on the class-split kernel; 5 puts the matrix-core kernel (ab_mma.hpp, one vector per
+// launch) first.  The matrix-core kernel is the fastest in FP64 at every size measured that its forms
+// hold (whole FP64 sigma against the source-lane kernel beside the same row SpMM: 12
+// orbitals 6 + 6 0.22 / 0.51 ms, 14 / 7 + 7 4.1 / 9.8 ms, 16 / 8 + 8 109 / 198 ms); they hold 17 k-steps
+// at 17 and 18 orbitals, 67 single excitations (not 17 / 7 + 5 or 18 / 6 + 4, which run on the kernels
+// after it).
+// FP32: hipotf_hvec_block (fixed = true) keeps the kernel of its size below 14 orbitals, whose sums run
+// in another order and, for the rows, in FP32; nothing but the 2e-5 of FP64 is promised there.  The
+// Davidson driver's FP32 phase takes the matrix cores at every size (12 orbitals, 4 vectors: 1.36 ->
+// 0.37 ms)
 static bool ab_mma_first(int pref, int prec, int n, bool fixed) {
     return pref == 5 || (pref == 0 && (prec == 0 || !fixed || (n >= 14 && n <= 16)));
 }
