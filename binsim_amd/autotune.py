@@ -21,7 +21,7 @@ Tuned per precision (FP64 sigma of one vector; FP32 block sigma of ``k`` vectors
 * ``ab_nvs``: vectors per source-lane launch in FP32 (1 or 2);
 * ``rs_block``: destination alpha (beta) strings per workgroup of the same-spin row SpMM that
   share each gathered source row (4, 8, 16; 0 = one destination row per wave; 8 with
-  ``rs_passes`` 0, the library's default, runs on the matrix cores in FP64 and in blocks of 4 in
+  ``rs_passes`` 0, the library's default, runs on the matrix cores in FP64 and in blocks of 4 or 8 in
   FP32);
 * ``rs_passes``: the same-spin row SpMM gathers its sources in 1, 2, 4 or 8 alpha-string
   ranges (source alpha block of N/passes strings per launch; the library's default, 0, takes

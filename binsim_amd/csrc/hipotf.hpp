@@ -254,7 +254,7 @@ struct SigmaTuning {
     int deterministic = 0;  // 1: alpha-beta scatter wave by wave (bitwise reproducible)
     int rs_block = 8;       // row SpMM: destination rows sharing each gathered source row
                             // (4, 8, 16), or 0 for one row per wave; 8 with rs_passes 0, the
-                            // defaults, is the matrix-core form in FP64 and blocks of 4 in FP32
+                            // defaults, is the matrix-core form in FP64, blocks of 4 or 8 in FP32
     int sweep_mode = 4;     // VQE rotation sweeps (FP64 table): 0 fused, on excitation levels in
                             // LDS where the pool allows (rot_levels.hpp), else with as many
                             // rows (and the leading part of one more) in LDS as fit, the

@@ -737,9 +737,12 @@ static void launch_rowspmm(const T *X, T *Y, SameSpinTable &tab, const T *C, i64
             if (const MfmaBlockTable *M = mfma_blocks(tab)) return launch_mbspmm(X, Y, *M, nrows, ncols, flag, st);
         if constexpr (sizeof(T) == 4) {
             // FP32 otherwise: blocks of 4 strings, the same sums in the same order as blocks of 8 (FP32
-            // sigma, 4 vectors: 12 orbitals 1.77 -> 1.67 ms, 14 orbitals 12.1 -> 11.5 ms).  Tables from
-            // the host have the blocks of 8 in both precisions, and another set costs seconds
-            if (tab.dev_built) rb = 4;
+            // sigma, 4 vectors: 12 orbitals 1.77 -> 1.67 ms, 14 orbitals 12.1 -> 11.5 ms; one vector, 18
+            // orbitals / 6 + 6, 18,564 strings, 612 -> 609 ms, but 18 / 7 + 7, 31,824 strings, 1.80 -> 1.82 s:
+            // the gathers, 1.4 times as many, miss the L2 there; 18 / 2 + 7, few columns, 14.3 -> 13.2 ms,
+            // 8 vectors 74.7 -> 75.5).  Tables from the host have the blocks of 8 in both precisions, and
+            // another set costs seconds
+            if (tab.dev_built && (tab.N < 24576 || ncols < 1024)) rb = 4;
         }
     }
     // an allocation-free call with other passes than at its preparation: the matrix-core tables

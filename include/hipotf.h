@@ -138,7 +138,7 @@ int hipotf_prepare(void *basis, void *net);
  * row-SpMM source-range passes 1|2|4|8 (0: as many as keep a column tile's gathered slice
  * within an XCD's L2), deterministic 0|1, same-spin destination rows per
  * gathered source row 4|8|16 (0: one row per wave; 8 with 0 passes, the defaults: FP64 on the
- * matrix cores, FP32 in blocks of 4), VQE rotation sweeps 0 fused (runs of particle-hole
+ * matrix cores, FP32 in blocks of 4 or 8), VQE rotation sweeps 0 fused (runs of particle-hole
  * generators on excitation levels in LDS; else as many rows in LDS as fit, the others in global memory) | 1 fused with rows in global memory | 2 one
  * launch per generator | 3 fused with at most one row and half of the next in LDS, +4 (4..7)
  * the same with the adjoint sweep's alpha-pair segments on interleaved (l, r) rows (default 4;
