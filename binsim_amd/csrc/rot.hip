@@ -994,7 +994,7 @@ static std::vector<Segment> plan_sweep(DevPool *P, const i64 *idxs, i64 n, int n
             if (!pair && !grad && t.count < (back ? (nel <= lv_cap(true) ? 1 : 8) : (k == 1 ? 8 : 16))) continue;
             LevelPlan *lp = level_plan(P, spin, pair, k);
             const bool fits = lp && !(back && (lp->maxslot > lv_cap(true) || lp->maxlen > 2048)) &&
-                              longest(*lp) >= 16 && units * lp->nbins < 1ll << 22;  // (less than 2^32 threads)
+                              longest(*lp) >= 16 && units * lp->nbins <= (1ll << 22) - 8;  // (less than 2^32 threads)
             if (fits) {
                 t.kind = pair ? SEG_LV_PAIR : (spin == 0 ? SEG_LV_ROW_B : SEG_LV_ROW_A);
                 t.lv = lp;

@@ -390,6 +390,7 @@ static void row_blocks_t(SameSpinTable &S, RowBlockTable &R, int rb) {
     R.P.alloc((size_t)nblk * (SS_RANGES + 1) * sizeof(int32_t));
     launch_blocks(k_rb_union<true, T>, nblk, N, (i64)rb * S.L, J, c, N, S.L, rb, (int32_t *)nullptr,
                   off.as<const i64>(), p.stride, R.J.as<int32_t>(), R.c.as<T>(), R.P.as<int32_t>());
+    if (!p.stride) HIPOTF_CHECK(hipDeviceSynchronize());  // (off is freed here)
 }
 void row_blocks_dev(SameSpinTable &S, RowBlockTable &R, int rb, int prec) {
     if (prec == 0) row_blocks_t<double>(S, R, rb);
@@ -481,6 +482,7 @@ const MfmaBlockTable *mfma_blocks(SameSpinTable &T) {
     M->c64.alloc((size_t)p.total * 4 * rb * sizeof(double));
     launch_blocks(k_mb_union<true>, nblk, N, (i64)rb * T.L, J, c, N, T.L, rb, M->nr, (int32_t *)nullptr,
                   first.as<const i64>(), p.stride, M->P.as<int32_t>(), M->J.as<int32_t>(), M->c64.as<double>());
+    if (!p.stride) HIPOTF_CHECK(hipDeviceSynchronize());  // (first is freed here)
     T.mfma = std::move(M);
     return T.mfma.get();
 }
