@@ -38,8 +38,8 @@ __device__ __forceinline__ float flip_sign(float v, u32 s) { return __uint_as_fl
 // ---------------------------------------------------------------------------------------
 // K1: gauge + dual layout (32x32 tiles through LDS)
 // ---------------------------------------------------------------------------------------
-// flag (if given): set to 1 by an element that is not finite (k_mbspmm)
-template <typename T, int NV>
+// FLAG: *flag is set to 1 by an element that is not finite (k_mbspmm)
+template <typename T, int NV, bool FLAG>
 __global__ __launch_bounds__(256) void k_gauge_in(SrcPack src, T *__restrict__ xt, T *__restrict__ xtT,
                                                   const u64 *__restrict__ strsB,
                                                   const u64 *__restrict__ M, i64 NA, i64 NB, int *flag) {
@@ -53,7 +53,7 @@ __global__ __launch_bounds__(256) void k_gauge_in(SrcPack src, T *__restrict__ x
             if (a < NA && b < NB) {
                 double val = src.p[v][a * NB + b];
                 if (parity64(strsB[b] & M[a])) val = -val;
-                if (flag && !isfinite(val)) *flag = 1;
+                if (FLAG && !isfinite(val)) *flag = 1;
                 const T tv = (T)val;
                 xt[(a * NB + b) * NV + v] = tv;
                 tile[ty + 8 * i][tx] = tv;
@@ -583,14 +583,14 @@ __global__ __launch_bounds__(1024) void k_ab_reg(const T *__restrict__ xt, T *__
 // ---------------------------------------------------------------------------------------
 // K5: sigma = E (s1 + s2T^T + E_core x~), FP64 output vectors
 // ---------------------------------------------------------------------------------------
-template <typename T, int NV>
+template <typename T, int NV, bool FLAG>
 __global__ __launch_bounds__(256) void k_finalize(const T *__restrict__ s1, const T *__restrict__ s2T,
                                                   const T *__restrict__ xt, double ecore, DstPack dst,
                                                   const u64 *__restrict__ strsB,
                                                   const u64 *__restrict__ M, i64 NA, i64 NB, int *flag) {
     __shared__ T tile[32][33];
     const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-    if (flag && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *flag = 0;  // (for the next sigma)
+    if (FLAG && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *flag = 0;  // (for the next sigma)
     const i64 b0 = (i64)blockIdx.x * 32, a0 = (i64)blockIdx.y * 32;
 #pragma unroll 1
     for (int v = 0; v < NV; ++v) {
@@ -1230,8 +1230,17 @@ static void sigma_group(DevHam *H, const SrcPack &src, const DstPack &dst, hipSt
     // (only the blocks of 16 strings ask)
     int *flag = sizeof(T) == 8 && std::max(NA, NB) >= MB_RB16_FROM ? reinterpret_cast<int *>(B->gaugeM.as<u64>() + NA)
                                                                    : nullptr;
-    hipLaunchKernelGGL((k_gauge_in<T, NV>), g2, dim3(256), 0, st, src, xt, xtT, Bs.strs.as<u64>(),
-                       B->gaugeM.as<u64>(), NA, NB, flag);
+    auto gauge = [&](auto kern) {
+        hipLaunchKernelGGL(kern, g2, dim3(256), 0, st, src, xt, xtT, Bs.strs.as<u64>(), B->gaugeM.as<u64>(), NA, NB,
+                           flag);
+    };
+    auto finalize = [&](auto kern) {
+        hipLaunchKernelGGL(kern, g2, dim3(256), 0, st, s1, s2T, xt, H->ecore, dst, Bs.strs.as<u64>(),
+                           B->gaugeM.as<u64>(), NA, NB, flag);
+    };
+    constexpr bool F64 = sizeof(T) == 8;
+    if (flag) gauge(k_gauge_in<T, NV, F64>);
+    else gauge(k_gauge_in<T, NV, false>);
     HIPOTF_CHECK(hipGetLastError());
     const bool f32 = sizeof(T) == 4;
     const T *CA = f32 ? (const T *)H->ptA->c32.p : (const T *)H->ptA->c64.p;
@@ -1250,8 +1259,8 @@ static void sigma_group(DevHam *H, const SrcPack &src, const DstPack &dst, hipSt
         tm.ms += ms;
         ++tm.sections;
     }
-    hipLaunchKernelGGL((k_finalize<T, NV>), g2, dim3(256), 0, st, s1, s2T, xt, H->ecore, dst,
-                       Bs.strs.as<u64>(), B->gaugeM.as<u64>(), NA, NB, flag);
+    if (flag) finalize(k_finalize<T, NV, F64>);
+    else finalize(k_finalize<T, NV, false>);
     HIPOTF_CHECK(hipGetLastError());
 }
 
